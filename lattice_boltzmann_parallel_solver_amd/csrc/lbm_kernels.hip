@@ -1777,6 +1777,52 @@ __global__ __launch_bounds__(kSweepThreads, K == 3 ? 5 : 4) void k_sweepk_batch(
 
 __global__ void k_add_step(int64_t *step, int64_t k) { *step += k; }
 
+// AoS records of nine values are 72 (36) bytes apart, so a wavefront's store of
+// one direction touches 36 lines and writes a ninth of each: equilibria and
+// streamed populations left at 3.0-3.5 TB/s that way (4200x1800 FP64).  Each
+// wave therefore turns its records round in LDS (stride 9: no bank conflicts)
+// and writes them out as one contiguous run, 16 bytes a lane where the run is
+// 16-byte aligned (at 4200x1800 FP64 the equilibrium went from 205 to 110 us,
+// 6.6 TB/s; streaming from 361 to 263; k_finalize from 285 to 227, and at
+// 8192x2048 FP32 from 583 to 387).  Loads of records stay per direction: the
+// lines a wave's first load brings in serve the other eight from L1 (5.1 TB/s;
+// staged the same way: velocity 143 -> 131 us in FP64 but 6.3 -> 6.8 in FP32
+// at 1021x773, density 118 -> 118 and 6.5 -> 7.5).
+constexpr int kRecLds = 64 * 9;  // values of one wave's records
+
+// The records of `cnt` (<= 64) consecutive nodes, lane l's v for node l, to
+// out[0 .. 9 cnt).  `lds`: kRecLds values of this wave.  Every lane calls it.
+template <class T>
+__device__ __forceinline__ void store_records(T *out, uint32_t cnt, const T v[9], T *lds) {
+    const uint32_t lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < 9; i++) lds[lane * 9 + i] = v[i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t n = cnt * 9;
+    constexpr uint32_t kVec = 16 / sizeof(T);
+    if ((reinterpret_cast<uintptr_t>(out) & 15) == 0) {
+        using V4 = uint32_t __attribute__((ext_vector_type(4)));
+        const uint32_t nv = n / kVec;
+#pragma unroll
+        for (uint32_t k = 0; k < (kRecLds / kVec + 63) / 64; k++) {
+            const uint32_t j = k * 64 + lane;
+            if (j < nv) reinterpret_cast<V4 *>(out)[j] = reinterpret_cast<const V4 *>(lds)[j];
+        }
+        const uint32_t j = nv * kVec + lane;
+        if (j < n) out[j] = lds[j];
+    } else {
+#pragma unroll
+        for (uint32_t k = 0; k < 9; k++) {
+            const uint32_t j = k * 64 + lane;
+            if (j < n) out[j] = lds[j];
+        }
+    }
+    // the next call's writes come after these reads
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // ---------------------------------------------------------------------------
 // first collision (from the AoS FP64 step input)
 // ---------------------------------------------------------------------------
@@ -1848,21 +1894,24 @@ __global__ __launch_bounds__(kBlock) void k_finalize(const S *__restrict__ src,
                                                      const typename Io<S>::C *__restrict__ side_prev, Geom g,
                                                      BcView bc, double *__restrict__ fo, double *__restrict__ ro,
                                                      double *__restrict__ uo, double *__restrict__ partials) {
+    __shared__ __align__(16) double rec[kBlock / 64][kRecLds];
     const uint32_t n = blockIdx.x * kBlock + threadIdx.x;
     double a0 = 0, a1 = 0, a2 = 0;
-    if (n < g.N) {
+    if ((n & ~63u) < g.N) {
         double f[9], rho, jx, jy, ux, uy;
-        finalize_node<S>(src, side_prev, g, bc, n, f, rho, jx, jy, ux, uy);
+        finalize_node<S>(src, side_prev, g, bc, min(n, g.N - 1), f, rho, jx, jy, ux, uy);
         if (fo)
-            for (int i = 0; i < 9; i++) fo[(size_t)n * 9 + i] = f[i];
-        if (ro) ro[n] = rho;
-        if (uo) {
-            uo[2 * (size_t)n] = ux;
-            uo[2 * (size_t)n + 1] = uy;
+            store_records(fo + (size_t)(n & ~63u) * 9, min(64u, g.N - (n & ~63u)), f, rec[threadIdx.x >> 6]);
+        if (n < g.N) {
+            if (ro) ro[n] = rho;
+            if (uo) {
+                uo[2 * (size_t)n] = ux;
+                uo[2 * (size_t)n + 1] = uy;
+            }
+            a0 = rho;
+            a1 = jx;
+            a2 = jy;
         }
-        a0 = rho;
-        a1 = jx;
-        a2 = jy;
     }
     if (partials) block_sum3(a0, a1, a2, partials + 3 * (size_t)blockIdx.x);
 }
@@ -1940,30 +1989,45 @@ __device__ __forceinline__ void feq_t(T rho, T ux, T uy, T e[9]) {
         e[i] = ((T)kWd[i] * rho) * (((T(1) + T(3) * cu[i]) + T(4.5) * (cu[i] * cu[i])) - T(1.5) * usq);
 }
 
+// Blocks in XCD order: the three source rows of neighbouring blocks' nodes are
+// then read through one L2 instead of three.
 template <class T>
-__global__ void k_stream_aos(const T *__restrict__ in, T *__restrict__ out, int nx, int ny) {
-    const int64_t n = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (n >= (int64_t)nx * ny) return;
-    const int x = (int)(n / ny), y = (int)(n - (int64_t)x * ny);
+__global__ __launch_bounds__(kBlock) void k_stream_aos(const T *__restrict__ in, T *__restrict__ out, int nx, int ny) {
+    __shared__ __align__(16) T rec[kBlock / 64][kRecLds];
+    const int64_t N = (int64_t)nx * ny;
+    const int64_t n0 = (int64_t)xcd_block(blockIdx.x, gridDim.x) * kBlock;
+    const int64_t w0 = n0 + (threadIdx.x & ~63u);  // first node of the wave
+    if (w0 >= N) return;
+    const uint32_t cnt = (uint32_t)min((int64_t)64, N - w0);
+    const int64_t xb = n0 / ny;  // uniform
+    const uint32_t off = (uint32_t)(n0 - xb * ny) + min(threadIdx.x, (uint32_t)(N - 1 - n0));
+    const uint32_t dx = off / (uint32_t)ny;
+    const int x = (int)xb + (int)dx, y = (int)(off - dx * (uint32_t)ny);
+    const int xm = x == 0 ? nx - 1 : x - 1, xp = x + 1 == nx ? 0 : x + 1;
+    const int ym = y == 0 ? ny - 1 : y - 1, yp = y + 1 == ny ? 0 : y + 1;
+    T v[9];
 #pragma unroll
     for (int i = 0; i < 9; i++) {
-        const int sx = (x - kCX[i] + nx) % nx, sy = (y - kCY[i] + ny) % ny;
-        out[n * 9 + i] = in[((int64_t)sx * ny + sy) * 9 + i];
+        const int sx = kCX[i] == 1 ? xm : (kCX[i] == -1 ? xp : x), sy = kCY[i] == 1 ? ym : (kCY[i] == -1 ? yp : y);
+        v[i] = in[((int64_t)sx * ny + sy) * 9 + i];
     }
+    store_records(out + w0 * 9, cnt, v, rec[threadIdx.x >> 6]);
 }
 
 template <class T>
-__global__ void k_equilibrium_aos(const T *__restrict__ rho, const T *__restrict__ u, T *__restrict__ feq,
-                                  int64_t n) {
-    const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (c >= n) return;
+__global__ __launch_bounds__(kBlock) void k_equilibrium_aos(const T *__restrict__ rho, const T *__restrict__ u,
+                                                            T *__restrict__ feq, int64_t n) {
+    __shared__ __align__(16) T rec[kBlock / 64][kRecLds];
+    const int64_t w0 = (int64_t)blockIdx.x * kBlock + (threadIdx.x & ~63u);
+    if (w0 >= n) return;
+    const int64_t c = min(w0 + (threadIdx.x & 63), n - 1);
     T e[9];
     feq_t<T>(rho[c], u[2 * c], u[2 * c + 1], e);
-    for (int i = 0; i < 9; i++) feq[c * 9 + i] = e[i];
+    store_records(feq + w0 * 9, (uint32_t)min((int64_t)64, n - w0), e, rec[threadIdx.x >> 6]);
 }
 
 template <class T>
-__global__ void k_density_aos(const T *__restrict__ f, T *__restrict__ rho, int64_t n) {
+__global__ __launch_bounds__(kBlock) void k_density_aos(const T *__restrict__ f, T *__restrict__ rho, int64_t n) {
 #pragma clang fp contract(off)
     const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (c >= n) return;
@@ -1972,7 +2036,8 @@ __global__ void k_density_aos(const T *__restrict__ f, T *__restrict__ rho, int6
 }
 
 template <class T>
-__global__ void k_velocity_aos(const T *__restrict__ rho, const T *__restrict__ f, T *__restrict__ u, int64_t n) {
+__global__ __launch_bounds__(kBlock) void k_velocity_aos(const T *__restrict__ rho, const T *__restrict__ f,
+                                                         T *__restrict__ u, int64_t n) {
 #pragma clang fp contract(off)
     const int64_t c = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (c >= n) return;
