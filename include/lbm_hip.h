@@ -293,6 +293,16 @@ int lbm_velocity(const void *rho, const void *f, void *u, int64_t ncells, int dt
 /* BGK collision f + (equilibrium(rho, u) - f)*omega, lattice_boltzmann_method.py:213-215. */
 int lbm_collide(const void *f, const void *rho, const void *u, double omega, void *f_out,
                 int64_t ncells, int dtype, void *stream);
+/* lattice_boltzmann_step(), lattice_boltzmann_method.py:191-228, in one pass:
+ * collision of f with the given rho and u, the program's pressure fix,
+ * streaming, its boundary rules, and the new moments.  FP64, nx*ny nodes;
+ * prog NULL = fully periodic.  The outputs overlap no input. */
+int lbm_step(const lbm_bc_prog *prog, const double *f, const double *rho, const double *u, double omega,
+             int nx, int ny, double *f_out, double *rho_out, double *u_out, void *stream);
+/* The same on host arrays, through `work` (device memory, 24*nx*ny doubles).
+ * Synchronous. */
+int lbm_step_host(const lbm_bc_prog *prog, const double *f, const double *rho, const double *u, double omega,
+                  int nx, int ny, double *f_out, double *rho_out, double *u_out, double *work, void *stream);
 /* Post-streaming boundary rules of a program applied in place to f_post
  * (the closures of boundary_conditions.py:93-111, 138-165, 192-212, 239-252,
  * 267-281).  f_prev is read only if the program has an outlet. FP64 only. */

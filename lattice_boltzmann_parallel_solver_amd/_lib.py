@@ -108,6 +108,8 @@ _SIGNATURES = {
     "lbm_density": (_I, [_P, _P, _I64, _I, _P]),
     "lbm_velocity": (_I, [_P, _P, _P, _I64, _I, _P]),
     "lbm_collide": (_I, [_P, _P, _P, _D, _P, _I64, _I, _P]),
+    "lbm_step": (_I, [_P, _P, _P, _P, _D, _I, _I, _P, _P, _P, _P]),
+    "lbm_step_host": (_I, [_P, _P, _P, _P, _D, _I, _I, _P, _P, _P, _P, _P]),
     "lbm_bc_apply": (_I, [_P, _P, _P, _P, _P]),
     "lbm_bc_pressure": (_I, [_P, _P, _P, _P, _P]),
     "lbm_moments_sum_noalloc": (_I, [_P, _I64, _P, _P]),

@@ -1876,6 +1876,8 @@ int lbm_collide(const void *f, const void *rho, const void *u, double omega, voi
 }
 
 static int prog_on_device(const lbm_bc_prog *prog, BcView &view, const char *fn) {
+    static std::mutex upload;  // threads that meet on one program upload it once
+    std::lock_guard<std::mutex> hold(upload);
     int dev = 0;
     LBM_HIP_CHECK(hipGetDevice(&dev), fn);
     auto *p = const_cast<lbm_bc_prog *>(prog);
@@ -1909,6 +1911,56 @@ static int prog_on_device(const lbm_bc_prog *prog, BcView &view, const char *fn)
     view.d2 = p->d2;
     view.flags = p->flags;
     return LBM_OK;
+}
+
+int lbm_step(const lbm_bc_prog *prog, const double *f, const double *rho, const double *u, double omega, int nx, int ny,
+             double *f_out, double *rho_out, double *u_out, void *stream) {
+    if (nx < 1 || ny < 1 || (int64_t)nx * ny > 0x7fffffffLL) {
+        set_error("lbm_step: lattice must satisfy 1 <= nx*ny < 2^31");
+        return LBM_ERR_ARG;
+    }
+    if (!(omega > 0.0 && omega < 2.0)) {
+        set_error("lbm_step: omega must satisfy 0 < omega < 2");
+        return LBM_ERR_ARG;
+    }
+    if (!f || !rho || !u || !f_out || !rho_out || !u_out || f == f_out || rho == rho_out || u == u_out) {
+        set_error("lbm_step: need f, rho, u and distinct non-NULL outputs");
+        return LBM_ERR_ARG;
+    }
+    if (prog && (prog->nx != nx || prog->ny != ny)) {
+        set_error("lbm_step: program compiled for " + std::to_string(prog->nx) + "x" + std::to_string(prog->ny) +
+                  ", lattice is " + std::to_string(nx) + "x" + std::to_string(ny));
+        return LBM_ERR_ARG;
+    }
+    BcView view;
+    if (prog)
+        if (int rc = prog_on_device(prog, view, "lbm_step")) return rc;
+    LBM_HIP_CHECK(launch_step_aos((uint32_t)nx, (uint32_t)ny, view, f, rho, u, omega, f_out, rho_out, u_out,
+                                  static_cast<hipStream_t>(stream)),
+                  "lbm_step");
+    return LBM_OK;
+}
+
+int lbm_step_host(const lbm_bc_prog *prog, const double *f, const double *rho, const double *u, double omega, int nx,
+                  int ny, double *f_out, double *rho_out, double *u_out, double *work, void *stream) {
+    if (nx < 1 || ny < 1 || !f || !rho || !u || !f_out || !rho_out || !u_out || !work) {
+        set_error("lbm_step_host: need nx, ny >= 1, host arrays and the work buffer");
+        return LBM_ERR_ARG;
+    }
+    const size_t N = (size_t)nx * ny;
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    double *in = work, *out = work + 12 * N;
+    LBM_HIP_CHECK(hipMemcpyAsync(in, f, 9 * N * sizeof(double), hipMemcpyHostToDevice, s), "lbm_step_host");
+    LBM_HIP_CHECK(hipMemcpyAsync(in + 9 * N, rho, N * sizeof(double), hipMemcpyHostToDevice, s), "lbm_step_host");
+    LBM_HIP_CHECK(hipMemcpyAsync(in + 10 * N, u, 2 * N * sizeof(double), hipMemcpyHostToDevice, s), "lbm_step_host");
+    const int rc = lbm_step(prog, in, in + 9 * N, in + 10 * N, omega, nx, ny, out, out + 9 * N, out + 10 * N, stream);
+    if (rc == LBM_OK) {
+        LBM_HIP_CHECK(hipMemcpyAsync(f_out, out, 9 * N * sizeof(double), hipMemcpyDeviceToHost, s), "lbm_step_host");
+        LBM_HIP_CHECK(hipMemcpyAsync(rho_out, out + 9 * N, N * sizeof(double), hipMemcpyDeviceToHost, s), "lbm_step_host");
+        LBM_HIP_CHECK(hipMemcpyAsync(u_out, out + 10 * N, 2 * N * sizeof(double), hipMemcpyDeviceToHost, s), "lbm_step_host");
+    }
+    LBM_HIP_CHECK(hipStreamSynchronize(s), "lbm_step_host");
+    return rc;
 }
 
 int lbm_bc_apply(const lbm_bc_prog *prog, const double *f_pre, double *f_post, const double *f_prev, void *stream) {

@@ -1790,13 +1790,16 @@ __global__ void k_add_step(int64_t *step, int64_t k) { *step += k; }
 // at 1021x773, density 118 -> 118 and 6.5 -> 7.5).
 constexpr int kRecLds = 64 * 9;  // values of one wave's records
 
-// The records of `cnt` (<= 64) consecutive nodes, lane l's v for node l, to
-// out[0 .. 9 cnt).  `lds`: kRecLds values of this wave.  Every lane calls it.
+// The records of `cnt` (<= 64 - first) consecutive nodes, lane first + l's v
+// for node l, to out[0 .. 9 cnt).  `lds`: kRecLds values of this wave.  Every
+// lane calls it.
 template <class T>
-__device__ __forceinline__ void store_records(T *out, uint32_t cnt, const T v[9], T *lds) {
+__device__ __forceinline__ void store_records(T *out, uint32_t cnt, const T v[9], T *lds, uint32_t first = 0) {
     const uint32_t lane = threadIdx.x & 63;
+    if (lane >= first) {
 #pragma unroll
-    for (int i = 0; i < 9; i++) lds[lane * 9 + i] = v[i];
+        for (int i = 0; i < 9; i++) lds[(lane - first) * 9 + i] = v[i];
+    }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
     const uint32_t n = cnt * 9;
@@ -2012,6 +2015,235 @@ __global__ __launch_bounds__(kBlock) void k_stream_aos(const T *__restrict__ in,
         v[i] = in[((int64_t)sx * ny + sy) * 9 + i];
     }
     store_records(out + w0 * 9, cnt, v, rec[threadIdx.x >> 6]);
+}
+
+// ---------------------------------------------------------------------------
+// one whole step on AoS FP64 arrays: (f, rho, u) -> (f, rho, u)
+//
+// Collision with the given moments, pressure fix, streaming, boundary classes
+// and new moments in one pass: 96 bytes in and 96 out a node, where loading a
+// context, stepping it and reading it back moved 528 (three copies, a
+// collision into planes, a read-out).  A block sweeps `rows` output rows of a
+// strip of W columns upwards, one lane per column plus a halo column on each
+// side, the next row's records loaded while the current one is collided; the
+// six y-moving populations change lanes through LDS (two buffers, so one
+// barrier a row), the row history (cx = +1 of the last two rows, cx = 0 of the
+// last) stays in registers, with the last row's own populations for the
+// reflections.  Arithmetic and order are k_collide_first's and k_finalize's.
+// Four rows a block (4200x1800 at 1, 2, 4, 8, 16, 33 rows: 387, 310, 307, 315,
+// 331, 321 us: the halo rows come from L2, and short ranges keep the rows that
+// run at once close in memory), fewer where the lattice has not 768 row ranges
+// (three resident blocks a CU) of them: there the launch is latency.
+// 4200x1800: 800 -> 307 us a step (4.7 TB/s of the 192 bytes a node), 20x30:
+// 58 -> 18 us a call.
+// ---------------------------------------------------------------------------
+struct StepAosParams {
+    const double *f, *rho, *u;
+    double *fo, *ro, *uo;
+    uint32_t lx, ly;
+    BcView bc;
+    double omega;
+    uint32_t rows;    // output rows per block
+    uint32_t strips;  // column strips of W output columns
+    uint32_t W;       // at most kBlock - 2
+};
+
+// Stores through a buffer descriptor: lanes whose offset lies past its end
+// store nothing, without a branch (a branch would leave the compiler unable to
+// count the stores in flight, and every wait for a load would drain them).
+using BufRsrc = __amdgpu_buffer_rsrc_t;
+__device__ __forceinline__ BufRsrc run_rsrc(void *base, uint32_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(base);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(((uint64_t)hi << 32) | lo), 0,
+                                             __builtin_amdgcn_readfirstlane(bytes), 0x00027000);
+}
+__device__ __forceinline__ void buf_store(BufRsrc r, uint32_t off, double v) {
+    using V2 = uint32_t __attribute__((ext_vector_type(2)));
+    const V2 d = {(uint32_t)__double2loint(v), (uint32_t)__double2hiint(v)};
+    __builtin_amdgcn_raw_buffer_store_b64(d, r, off, 0, 0);
+}
+
+constexpr uint32_t kStepClasses = 64;  // classes kept in LDS (all composites have fewer)
+
+// kLdsClasses: the program's classes fit the LDS table; else they are read
+// from memory where a node has one.
+template <bool kLdsClasses>
+__global__ __launch_bounds__(kBlock, 3) void k_step_aos(StepAosParams p) {
+#pragma clang fp contract(off)
+    constexpr uint32_t kCols = kBlock + 1;  // a spare column for lanes past the strip
+    __shared__ double ex[2][6][kCols];
+    __shared__ __align__(16) double rec[kBlock / 64][kRecLds];
+    __shared__ ClassEntry cls[kLdsClasses ? kStepClasses : 1];
+    const uint32_t tid = threadIdx.x, lx = p.lx, ly = p.ly;
+    const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+    const uint32_t rb = blk / p.strips, strip = blk - rb * p.strips;
+    const uint32_t xa = rb * p.rows, R = min(p.rows, lx - xa);
+    const uint32_t y0 = strip * p.W, W = min(p.W, ly - y0);
+    const uint32_t l = min(tid, W + 1);                // local column: global y0 - 1 + l
+    const uint32_t col = tid <= W + 1 ? tid : kBlock;  // LDS column written
+    uint32_t y = y0 + l + ly - 1;                      // in [ly - 1, 2 ly]
+    y = y >= ly ? (y - ly >= ly ? y - 2 * ly : y - ly) : y;
+    const uint32_t lm = l == 0 ? 0 : l - 1, lp = min(l + 1, W + 1);
+    // this wave's output lanes first .. first + cnt - 1 and their first column
+    const uint32_t lane = tid & 63, wave0 = __builtin_amdgcn_readfirstlane(tid & ~63u);
+    const uint32_t first = wave0 == 0 ? 1 : 0;
+    const uint32_t cnt = wave0 + first > W ? 0 : min(wave0 + 63, W) - (wave0 + first) + 1;
+    const uint32_t yout = y0 + wave0 + first - 1;
+    double *wrec = rec[tid >> 6];
+    const bool pressure = (p.bc.flags & kProgPressure) != 0;
+    // with no program, a load of the same kind whose value is masked out
+    const uint16_t *codes = p.bc.codes ? p.bc.codes : reinterpret_cast<const uint16_t *>(p.f);
+    const uint32_t code_mask = p.bc.codes ? 0xffffu : 0u;
+    if (kLdsClasses && p.bc.codes) {
+        const uint32_t words = p.bc.nclasses * (uint32_t)(sizeof(ClassEntry) / 4);
+        for (uint32_t i = tid; i < words; i += blockDim.x)
+            reinterpret_cast<uint32_t *>(cls)[i] = reinterpret_cast<const uint32_t *>(p.bc.classes)[i];
+    }
+    struct Rec {
+        double f[9], rho, ux, uy;
+        uint32_t code;
+    };
+    auto row_at = [&](uint32_t it) {  // row xa - 1 + it, periodic
+        const uint32_t r = xa + it + lx - 1;
+        return r >= lx ? (r - lx >= lx ? r - 2 * lx : r - lx) : r;
+    };
+    auto load = [&](uint32_t x) {
+        Rec a;
+        const size_t n = (size_t)x * ly + y;
+#pragma unroll
+        for (int i = 0; i < 9; i++) a.f[i] = p.f[n * 9 + i];
+        a.rho = p.rho[n];
+        a.ux = p.u[2 * n];
+        a.uy = p.u[2 * n + 1];
+        a.code = codes[n] & code_mask;
+        return a;
+    };
+    auto collide = [&](const Rec &a, double e[9], double s[9]) {
+        feq_f64(a.rho, a.ux, a.uy, e);
+#pragma unroll
+        for (int i = 0; i < 9; i++) s[i] = a.f[i] + (e[i] - a.f[i]) * p.omega;
+    };
+    Rec nx = load(row_at(0));
+    double A[3] = {0, 0, 0}, B[3] = {0, 0, 0}, Cc[3] = {0, 0, 0}, D = 0;
+    uint32_t code = 0;
+    auto body = [&](uint32_t it, auto out_tag) {
+        constexpr bool kOut = decltype(out_tag)::value;
+        const Rec a = nx;
+        const uint32_t x = row_at(it);
+        nx = load(row_at(min(it + 1, R + 1)));
+        double s[9];
+        {
+            double e[9];
+            collide(a, e, s);
+        }
+        if (pressure && (x == 0 || x == lx - 1)) {
+            // columns 0 and lx - 1 take E(rho_in, u) + (s - e) of row lx - 2 in
+            // directions d1, and E(rho_out, u) + (s - e) of row 1 in d2
+            auto fix = [&](uint32_t from, double rho, uint32_t dirs) {
+                const Rec b = load(from);
+                double eb[9], sb[9], ef[9];
+                collide(b, eb, sb);
+                feq_f64(rho, b.ux, b.uy, ef);
+#pragma unroll
+                for (int i = 0; i < 9; i++)
+                    if ((dirs >> i) & 1u) s[i] = ef[i] + (sb[i] - eb[i]);
+            };
+            if (x == 0) fix(lx - 2, p.bc.rho_in, p.bc.d1);
+            if (x == lx - 1) fix(1 % lx, p.bc.rho_out, p.bc.d2);
+        }
+        double(*exb)[kCols] = ex[it & 1];
+        const double(*exp_)[kCols] = ex[(it + 1) & 1];
+#pragma unroll
+        for (int j = 0; j < 6; j++) exb[j][col] = s[kYM[j]];
+        __syncthreads();
+        double Y[9];
+        Y[0] = s[0];
+        Y[1] = s[1];
+        Y[3] = s[3];
+        Y[2] = exb[0][lm];
+        Y[5] = exb[1][lm];
+        Y[6] = exb[2][lm];
+        Y[4] = exb[3][lp];
+        Y[7] = exb[4][lp];
+        Y[8] = exb[5][lp];
+        if constexpr (kOut) {
+            const uint32_t r = row_at(it - 1);
+            double v[9] = {B[0], A[0], B[1], Y[3], B[2], A[1], Y[6], Y[7], A[2]};
+            double out3[3] = {0, 0, 0};
+            if ((p.bc.flags & kProgOutlet) && r == lx - 1) {
+                // the outlet's step input; consumed here (the empty asm), so
+                // that other rows never wait on these loads
+#pragma unroll
+                for (int q = 0; q < 3; q++) {
+                    out3[q] = p.f[((size_t)(lx - 2) * ly + y) * 9 + (q == 0 ? 3 : 5 + q)];
+                    asm volatile("" : "+v"(out3[q]));
+                }
+            }
+            if (code) {
+                // reflections read the node's own collided populations: 0, 1 and
+                // 3 from registers, the others where this lane published them
+                // one row ago
+                uint32_t w;
+                if constexpr (kLdsClasses) w = cls[code].src;
+                else w = p.bc.classes[code].src;
+#pragma unroll
+                for (int d = 0; d < 9; d++) {
+                    const uint32_t kind = (w >> (2 * d)) & 3u;
+                    double k;
+                    if constexpr (kLdsClasses) k = cls[code].k[d];
+                    else k = p.bc.classes[code].k[d];
+                    const int o = kOpp[d];
+                    const double refl = o == 0 ? B[0] : o == 1 ? Cc[0] : o == 3 ? D : exp_[kYSlot[o]][l];
+                    if (kind == kSrcReflect) v[d] = refl - k;
+                    else if (kind == kSrcConst) v[d] = k;
+                    else if (kind == kSrcOutlet) v[d] = out3[outlet_slot(d)];
+                    asm volatile("" : "+v"(v[d]));
+                }
+            }
+            double rho, jx, jy, ux, uy;
+            moments_f64(v, rho, jx, jy);
+            velocity_f64(rho, jx, jy, ux, uy);
+            // records turned round in LDS, as in store_records
+            if (lane >= first) {
+#pragma unroll
+                for (int i = 0; i < 9; i++) wrec[(lane - first) * 9 + i] = v[i];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const size_t n = (size_t)r * ly + yout;
+            const BufRsrc rf = run_rsrc(p.fo + n * 9, cnt * 72);
+#pragma unroll
+            for (uint32_t k = 0; k < 9; k++) buf_store(rf, (k * 64 + lane) * 8, wrec[k * 64 + lane]);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const uint32_t j = lane - first;  // lanes before the first wrap past the end
+            buf_store(run_rsrc(p.ro + n, cnt * 8), min(j, 0x1000u) * 8, rho);
+            const BufRsrc ru = run_rsrc(p.uo + 2 * n, cnt * 16);
+            buf_store(ru, min(j, 0x1000u) * 16, ux);
+            buf_store(ru, min(j, 0x1000u) * 16 + 8, uy);
+        }
+#pragma unroll
+        for (int j = 0; j < 3; j++) A[j] = Cc[j];
+        B[0] = Y[0];
+        B[1] = Y[2];
+        B[2] = Y[4];
+        Cc[0] = Y[1];
+        Cc[1] = Y[5];
+        Cc[2] = Y[8];
+        D = Y[3];
+        code = a.code;
+    };
+    body(0, Flag<false>{});
+    body(1, Flag<false>{});
+    // as many stores on this path as on the loop's back edge (all past the end
+    // of an empty run, so none writes), or the loop's first wait for loads,
+    // counted for the path with fewer stores, would drain the loop's own
+    const BufRsrc none = run_rsrc(p.fo, 0);
+#pragma unroll
+    for (uint32_t k = 0; k < 12; k++) buf_store(none, lane * 8, 0.0);
+    for (uint32_t it = 2; it < R + 2; it++) body(it, Flag<true>{});
 }
 
 template <class T>
@@ -2891,6 +3123,34 @@ hipError_t launch_equilibrium_aos(const void *rho, const void *u, void *feq, int
         hipLaunchKernelGGL(k_equilibrium_aos<float>, dim3(grid_for(n)), dim3(kBlock), 0, s,
                            static_cast<const float *>(rho), static_cast<const float *>(u), static_cast<float *>(feq),
                            n);
+    return hipGetLastError();
+}
+
+hipError_t launch_step_aos(uint32_t lx, uint32_t ly, const BcView &bc, const double *f, const double *rho,
+                           const double *u, double omega, double *fo, double *ro, double *uo, hipStream_t s) {
+    constexpr uint32_t kMaxW = kBlock - 2;
+    StepAosParams p;
+    p.f = f;
+    p.rho = rho;
+    p.u = u;
+    p.fo = fo;
+    p.ro = ro;
+    p.uo = uo;
+    p.lx = lx;
+    p.ly = ly;
+    p.bc = bc;
+    p.omega = omega;
+    p.strips = (ly + kMaxW - 1) / kMaxW;
+    p.W = (ly + p.strips - 1) / p.strips;
+    p.strips = (ly + p.W - 1) / p.W;  // every strip holds a column
+    const uint64_t slots = 3 * 256;
+    p.rows = (uint32_t)std::min<uint64_t>(4, std::max<uint64_t>(1, ((uint64_t)lx * p.strips + slots - 1) / slots));
+    const uint64_t grid = (uint64_t)((lx + p.rows - 1) / p.rows) * p.strips;
+    const unsigned threads = (p.W + 2 + 63) / 64 * 64;
+    if (bc.nclasses <= kStepClasses)
+        hipLaunchKernelGGL(k_step_aos<true>, dim3((unsigned)grid), dim3(threads), 0, s, p);
+    else
+        hipLaunchKernelGGL(k_step_aos<false>, dim3((unsigned)grid), dim3(threads), 0, s, p);
     return hipGetLastError();
 }
 

@@ -157,6 +157,10 @@ int partial_rows_needed(const Geom &g, const LaunchCfg &cfg);
 hipError_t launch_stream_aos(const void *in, void *out, int nx, int ny, int dtype, hipStream_t s);
 hipError_t launch_equilibrium_aos(const void *rho, const void *u, void *feq, int64_t n, int dtype,
                                   hipStream_t s);
+// One whole step on AoS FP64 arrays: (f, rho, u) -> (fo, ro, uo), none of the
+// outputs overlapping an input.  bc: device tables (default: fully periodic).
+hipError_t launch_step_aos(uint32_t lx, uint32_t ly, const BcView &bc, const double *f, const double *rho,
+                           const double *u, double omega, double *fo, double *ro, double *uo, hipStream_t s);
 hipError_t launch_density_aos(const void *f, void *rho, int64_t n, int dtype, hipStream_t s);
 hipError_t launch_velocity_aos(const void *rho, const void *f, void *u, int64_t n, int dtype,
                                hipStream_t s);

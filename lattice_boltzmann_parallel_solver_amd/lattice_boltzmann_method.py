@@ -5,14 +5,12 @@ runs as a HIP kernel (liblbm_hip.so).  numpy inputs return numpy outputs
 (copied through the device), float64/float32 torch device tensors return
 device tensors.  ``lattice_boltzmann_step`` runs the whole step (collision
 with the given density/velocity, streaming, boundary, moments) on the GPU
-through a cached device context; the boundary must be one of this package's
-boundary objects (they compile to a device program), not an arbitrary
-Python callable.
+in one kernel; the boundary must be one of this package's boundary objects
+(they compile to a device program), not an arbitrary Python callable.
 """
 
 from __future__ import annotations
 
-from collections import OrderedDict
 from typing import Callable, Tuple
 
 import numpy as np
@@ -99,26 +97,6 @@ def equilibrium_distr_func(density_func, velocity_field):
     return back(out, kind)
 
 
-# cached device contexts for lattice_boltzmann_step, keyed by shape and boundary program
-_STEP_CONTEXTS: "OrderedDict[tuple, object]" = OrderedDict()
-_MAX_CONTEXTS = 4
-
-
-def _step_context(lx: int, ly: int, boundary):
-    from .solver import Lattice
-
-    prog = None if boundary is None else boundary.program(lx, ly)
-    key = (lx, ly, id(prog))
-    ctx = _STEP_CONTEXTS.get(key)
-    if ctx is None or ctx._program is not prog:
-        ctx = Lattice(lx, ly, boundary=prog, storage="f64")
-        _STEP_CONTEXTS[key] = ctx
-        while len(_STEP_CONTEXTS) > _MAX_CONTEXTS:
-            _STEP_CONTEXTS.popitem(last=False)[1].close()
-    _STEP_CONTEXTS.move_to_end(key)
-    return ctx
-
-
 def lattice_boltzmann_step(f, density, velocity, omega: float,
                            boundary: Callable = None,
                            parallel_communication: Callable = None) -> Tuple:
@@ -140,21 +118,23 @@ def lattice_boltzmann_step(f, density, velocity, omega: float,
                         "(boundary_utils.compose(...) builds one from primitives); arbitrary Python "
                         "callables cannot run inside the fused GPU step")
     lx, ly = int(f.shape[0]), int(f.shape[1])
-    ctx = _step_context(lx, ly, boundary)
-    torch_in = False
-    try:
-        import torch
-
-        torch_in = isinstance(f, torch.Tensor)
-    except ImportError:  # pragma: no cover
-        pass
-    ctx.set_state(f, density, velocity)
-    ctx.run(omega, 1)
-    if torch_in:
-        torch = torch_cuda()
-        fo = torch.empty((lx, ly, 9), dtype=torch.float64, device="cuda")
-        ro = torch.empty((lx, ly), dtype=torch.float64, device="cuda")
-        uo = torch.empty((lx, ly, 2), dtype=torch.float64, device="cuda")
-        ctx.state_into(fo, ro, uo)
-        return fo, ro, uo
-    return ctx.state()
+    assert tuple(f.shape) == (lx, ly, 9), f"f must have shape {(lx, ly, 9)}"
+    assert tuple(velocity.shape) == (lx, ly, 2), f"velocity must have shape {(lx, ly, 2)}"
+    prog = None if boundary is None else boundary.program(lx, ly)
+    handle = None if prog is None else prog.handle
+    torch = torch_cuda()
+    if isinstance(f, torch.Tensor):
+        ins = [t.detach() for t in (f, density, velocity)]
+        if any(t.device.type != "cuda" for t in ins):
+            raise ValueError("torch inputs must be device tensors")
+        ins = [t.to("cuda", torch.float64).contiguous() for t in ins]
+        outs = tuple(torch.empty_like(t) for t in ins)
+        check(_lib.load().lbm_step(handle, *(t.data_ptr() for t in ins), float(omega), lx, ly,
+                                   *(t.data_ptr() for t in outs), stream()))
+        return outs
+    ins = [np.ascontiguousarray(a, dtype=np.float64) for a in (f, density, velocity)]
+    outs = tuple(np.empty(a.shape) for a in ins)
+    work = torch.empty(24 * lx * ly, dtype=torch.float64, device="cuda")
+    check(_lib.load().lbm_step_host(handle, *(a.ctypes.data for a in ins), float(omega), lx, ly,
+                                    *(a.ctypes.data for a in outs), work.data_ptr(), stream()))
+    return outs
