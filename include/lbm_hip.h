@@ -161,15 +161,20 @@ int lbm_set_launch(lbm_ctx *ctx, int cells_per_thread, int xcd_remap, int nt_sto
 /* Temporal blocking of lbm_run: steps_per_launch = 2 advances two steps per
  * kernel launch (a row sweep that keeps the intermediate state on chip and
  * reads and writes the populations once per two steps; results are identical
- * to single steps), 1 = one step per launch (default).  rows_per_block: rows
- * each block of the two-step kernel sweeps (0 = automatic).  Rows wider than
- * one block (ny > 2048 FP32/FP16, > 1024 FP64) run as column tiles with a
- * halo column each side.  Two steps need no pressure fix in the boundary
- * program, nx >= 3 and at most 128 boundary classes; otherwise LBM_ERR_ARG.
+ * to single steps), 1 = one step per launch.  rows_per_block: rows each block
+ * of the two-step kernel sweeps (0 = automatic).  Rows wider than one block
+ * (ny > 2048 FP32/FP16, > 1024 FP64) run as column tiles with a halo column
+ * each side.  Two steps need no pressure fix in the boundary program, nx >= 3
+ * and at most 128 boundary classes; otherwise LBM_ERR_ARG.
  * steps_per_launch = 3 or 4: that many steps per launch (FP32/FP16, ny <=
  * 1024, the LDS of K - 1 intermediate stages within 160 KiB: ny <= 1024 for
  * 3, about 700 for 4); a run's remainder goes two steps and one step at a
- * time.  No counterpart in the reference (a launch setting of this library). */
+ * time.  With 2 or more and rows_per_block = 0, small lattices (2^18 nodes in
+ * FP64, 3 * 2^16 else) advance up to eight steps per launch on tiles held on
+ * chip.  A context that this and lbm_set_launch were never called on takes the
+ * number of steps that measured fastest for it.  Results are identical in
+ * every setting.  No counterpart in the reference (a launch setting of this
+ * library). */
 int lbm_set_temporal(lbm_ctx *ctx, int steps_per_launch, int rows_per_block);
 /* Column tiles of the two-step kernel: blocks of at most `threads` threads (a
  * multiple of 64 up to 1024; 0 = whole rows up to 1024 threads, the default),

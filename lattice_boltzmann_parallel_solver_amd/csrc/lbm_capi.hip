@@ -125,9 +125,19 @@ struct lbm_ctx {
     double *partials = nullptr;
     double *sums = nullptr;
     LaunchCfg cfg;
+    // tiling of the tile kernel, worked out by the first run that may take it
+    TileShape tile;
+    bool tile_ready = false;
 };
 
 namespace {
+
+// Whether three steps per launch beat two for FP32 rows of `waves`
+// wavefronts (measured on 8192-row channels: blocks of 7-8 and of 11 or more
+// waves gain 10-36 %; 9-10 lose or tie, 6 and fewer lose or tie).
+bool three_steps_pay(int storage, unsigned waves) {
+    return storage == LBM_STORE_F32 && (waves == 7 || waves == 8 || waves >= 11);
+}
 
 // Two-step runs of at least this many launches take the range-interleaved row
 // order (moving the state there and back costs about two launches).
@@ -290,6 +300,7 @@ int lbm_set_launch(lbm_ctx *c, int v, int xcd, int nt) {
     c->cfg.cells_per_thread = v;
     c->cfg.xcd_remap = xcd ? 1 : 0;
     c->cfg.nt_stores = nt ? 1 : 0;
+    c->cfg.shape_given = true;
     return LBM_OK;
 }
 
@@ -377,6 +388,7 @@ int lbm_set_bc(lbm_ctx *c, const lbm_bc_prog *prog) {
     LBM_HIP_CHECK(hipStreamSynchronize(c->stream), "lbm_set_bc");
     (void)hipFree(c->bc.mem);
     c->bc = BcUpload{};
+    c->tile_ready = false;
     if (prog) LBM_HIP_CHECK(upload_bc(*prog, c->bc), "lbm_set_bc: upload");
     return LBM_OK;
 }
@@ -420,6 +432,24 @@ int lbm_set_state_equilibrium(lbm_ctx *c, const double *rho, const double *u, in
     return LBM_OK;
 }
 
+// Steps per launch of a run: the caller's, or for a context that was given no
+// launch setting at all (0) what measured fastest.  Two wherever the row sweep
+// applies and one row a block fills the GPU (64x4000 FP32 has not the rows: 5.9
+// us a step with one, 9.7 with two; 1200x514 FP64 16.1 and 15.2, 8192x2048 FP32
+// 202 and 113); three for long FP32 lattices of the widths where they pay
+// (8192x1024: 131 GLUPS with two, 177 with three; 2000x1024: 15.9 us and 16.0).
+// 0 stays 0 where only tiles and single steps apply.
+static int run_steps_per_launch(const lbm_ctx *c) {
+    if (c->cfg.steps_per_launch > 0) return c->cfg.steps_per_launch;
+    if (c->cfg.shape_given) return 1;
+    const SweepShape sh = sweep_shape(c->storage, c->g.ly);
+    if (!sweep_supported(c->storage, c->g, c->bc.view) || (uint64_t)c->g.lx * sh.ntiles < 256) return 0;
+    if (c->g.lx >= 4096 && three_steps_pay(c->storage, (c->g.ly + 63) / 64) &&
+        sweepk_supported(c->storage, c->g, c->bc.view, 3))
+        return 3;
+    return 2;
+}
+
 int lbm_run(lbm_ctx *c, double omega, int64_t nsteps) {
     int rc = check_ctx(c, "lbm_run");
     if (rc) return rc;
@@ -446,7 +476,25 @@ int lbm_run(lbm_ctx *c, double omega, int64_t nsteps) {
         left--;
     }
     const bool probing = c->probe.cell >= 0;
-    const int K = c->cfg.steps_per_launch;
+    const int K = run_steps_per_launch(c);
+    // Small lattices: several steps per launch on tiles.  A step alone, one
+    // step per launch and row counts or column tiles that the caller chose keep
+    // their kernels.
+    const bool tiles = K != 1 && !c->cfg.shape_given && c->cfg.sweep_rows == 0 && c->cfg.sweep_tile == 0;
+    if (tiles && !c->tile_ready) {
+        c->tile = tile_shape(c->storage, c->g, c->bc.view);
+        c->tile_ready = true;
+    }
+    while (tiles && left > 1 && c->tile.K > 0) {
+        TileShape sh = c->tile;
+        sh.K = (int)std::min<int64_t>(sh.K, left);
+        const int64_t slot = probing ? c->steps - c->probe_base - 1 : -1;
+        LBM_HIP_CHECK(launch_tile(c->storage, sh, c->g, c->st, c->cur, c->bc.view, omega, c->probe, slot, c->stream),
+                      "tile kernel");
+        c->cur ^= 1;
+        c->steps += sh.K;
+        left -= sh.K;
+    }
     if (K >= 3 && sweepk_supported(c->storage, c->g, c->bc.view, K)) {
         for (; left >= K; left -= K) {
             // materialises f_{steps} .. f_{steps+K-1}
@@ -905,13 +953,6 @@ void release_batch(lbm_batch *b) {
     if (b->fork) (void)hipEventDestroy(b->fork);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     if (b->h_stage) (void)hipHostFree(b->h_stage);
-}
-
-// Whether three steps per launch beat two for FP32 rows of `waves`
-// wavefronts (measured on 8192-row channels: blocks of 7-8 and of 11 or more
-// waves gain 10-36 %; 9-10 lose or tie, 6 and fewer lose or tie).
-bool three_steps_pay(int storage, unsigned waves) {
-    return storage == LBM_STORE_F32 && (waves == 7 || waves == 8 || waves >= 11);
 }
 
 // Side streams of a batch, and the batch size (nodes) from which a batch

@@ -1775,6 +1775,179 @@ __global__ __launch_bounds__(kSweepThreads, K == 3 ? 5 : 4) void k_sweepk_batch(
     sweepk_block<S, K, false>(p, (blk - j.block0) * j.rows, smem);
 }
 
+// ---------------------------------------------------------------------------
+// K steps per launch on tiles held in registers and LDS, for small lattices
+//
+// A lattice of some hundred thousand nodes is bound by launches and latency:
+// one step per launch takes 5 us at 300x300 FP64 whatever the arithmetic, and
+// the row sweep's blocks walk their rows one after another.  Here a block holds
+// a tile of the output plus the halo that K steps reach, one node per thread:
+// the first step pulls from the state buffer, each later one from the collided
+// populations that the block's threads publish in LDS (two buffers, one barrier
+// a step), the last stores the tile.  Nodes of the halo are computed by several
+// blocks, which costs arithmetic that the idle GPU has; results are the same
+// for every tiling, since every node goes through the single step's arithmetic.
+// A node s - 1 nodes inside the region is right after step s.  With the
+// pressure fix, rows 0 and lx - 1 take values from the rows two beyond the
+// periodic seam, so the halo is two rows deeper (the producers write them into
+// the consumers' LDS slots, as store_node does in memory); lattices so short that
+// K steps reach across the seam twice take fewer steps.
+// ---------------------------------------------------------------------------
+template <class S>
+struct TileParams {
+    const S *src;
+    S *dst;
+    const typename Io<S>::C *side_prev;
+    typename Io<S>::C *side_next;
+    Geom g;
+    BcView bc;
+    double omega;
+    int64_t probe_cell;  // -1: no probe
+    double *probe_ring;  // sample of step s (1-based) in slot probe_slot + s - 1
+    int64_t probe_cap, probe_slot;
+    uint32_t K;               // steps
+    uint32_t tx, ty;          // output nodes of a tile
+    uint32_t hx, hy;          // halo on each side
+    uint32_t offx, offy;      // multiples of lx, ly at least hx, hy, less hx, hy
+    uint32_t tiles_y;         // tiles along y
+    uint32_t copies;          // times a row can appear in a tile's region
+};
+
+template <class S>
+struct TileLds {
+    size_t side, cls, total;  // ex at 0: two buffers of eight planes of `nodes` values
+    __host__ __device__ TileLds(uint32_t nodes, uint32_t ry, uint32_t copies, uint32_t nclasses) {
+        side = align16(16 * (size_t)nodes * sizeof(S));
+        cls = align16(side + 2 * (size_t)copies * 3 * ry * sizeof(typename Io<S>::C));
+        total = cls + (size_t)nclasses * sizeof(ClassEntry);
+    }
+};
+
+constexpr int tile_threads(size_t elem, bool pressure) { return elem == 8 ? (pressure ? 512 : 768) : (pressure ? 768 : 1024); }
+
+template <class S, bool kPressure>
+__global__ __launch_bounds__(tile_threads(sizeof(S), kPressure)) void k_tile(TileParams<S> p) {
+    using C = typename Io<S>::C;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const Geom &g = p.g;
+    const uint32_t lx = g.lx, ly = g.ly;
+    const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+    const uint32_t bx = blk / p.tiles_y, by = blk - bx * p.tiles_y;
+    const uint32_t x0 = bx * p.tx, y0 = by * p.ty;
+    const uint32_t rx = p.tx + 2 * p.hx, ry = p.ty + 2 * p.hy, nodes = rx * ry;  // the region
+    const bool active = threadIdx.x < nodes;
+    const uint32_t t = min(threadIdx.x, nodes - 1);
+    const uint32_t i = t / ry, j = t - i * ry;
+    const uint32_t ux = x0 + i + p.offx;
+    const uint32_t x = ux % lx, y = (y0 + j + p.offy) % ly;
+    const uint32_t copy = ux / lx - (x0 + p.offx) / lx;
+    const bool owned = active && i >= p.hx && j >= p.hy && i - p.hx < min(p.tx, lx - x0) && j - p.hy < min(p.ty, ly - y0);
+    const bool has_bc = p.bc.codes != nullptr;
+    const TileLds<S> L(nodes, ry, p.copies, has_bc ? p.bc.nclasses : 0);
+    S *ex = reinterpret_cast<S *>(smem);
+    C *side = reinterpret_cast<C *>(smem + L.side);
+    ClassEntry *cls = reinterpret_cast<ClassEntry *>(smem + L.cls);
+    const uint32_t n = x * ly + y;
+    const uint32_t code = has_bc ? p.bc.codes[n] : 0;
+    if (has_bc) {
+        const uint32_t words = p.bc.nclasses * (uint32_t)(sizeof(ClassEntry) / 4);
+        for (uint32_t k = threadIdx.x; k < words; k += blockDim.x)
+            reinterpret_cast<uint32_t *>(cls)[k] = reinterpret_cast<const uint32_t *>(p.bc.classes)[k];
+    }
+    C v[9];
+    pull<S>(p.src, g, x, y, v);
+    uint32_t flags = 0;
+    if (code) flags = apply_class<S>(p.bc, p.src, p.side_prev, g, n, x, y, v);
+    // LDS slots the pulls read: the upstream node's, or, where the node's class
+    // reflects, the node's own opposite one (nodes on the region's rim read some
+    // slot of it; what they compute is not used).  What is left of the class
+    // for the loop is constants, outlet copies and reflections off a moving wall.
+    const uint32_t w = code ? p.bc.classes[code].src : 0u;
+    uint32_t from[9];
+    bool rest = false;
+#pragma unroll
+    for (int d = 1; d < 9; d++) {
+        const uint32_t kind = (w >> (2 * d)) & 3u;
+        const int q = min(max((int)t - kCX[d] * (int)ry - kCY[d], 0), (int)nodes - 1);
+        from[d] = kind == kSrcReflect ? (kOpp[d] - 1) * nodes + t : (d - 1) * nodes + (uint32_t)q;
+        rest |= kind == kSrcReflect ? p.bc.classes[code].k[d] != 0.0 : kind != kSrcStream;
+    }
+    rest |= (w & 3u) != kSrcStream;
+    for (uint32_t s = 1;; s++) {
+        NodeOut<S> o;
+        collide_node<S>(v, p.omega, o);
+        if (p.probe_cell >= 0 && owned && (int64_t)n == p.probe_cell) {
+            const int64_t slot = p.probe_slot + (int64_t)s - 1;
+            if (slot >= 0) {
+                double *pr = p.probe_ring + 3 * (slot % p.probe_cap);
+                pr[0] = o.rho;
+                pr[1] = (double)o.ux;
+                pr[2] = (double)o.uy;
+            }
+        }
+        if (s == p.K) {
+            if (!owned) return;
+            if constexpr (kPressure) {
+                store_node<S>(p.dst, p.side_next, g, p.bc, x, y, flags, v, o, false);
+            } else {
+#pragma unroll
+                for (int d = 0; d < 9; d++) Io<S>::st(p.dst + pop(g, x, d, y), o.s[d], false);
+                if (flags & kFlagOutletSide) {
+                    p.side_next[(size_t)y * 3 + 0] = v[3];
+                    p.side_next[(size_t)y * 3 + 1] = v[6];
+                    p.side_next[(size_t)y * 3 + 2] = v[7];
+                }
+            }
+            return;
+        }
+        S *e = ex + (size_t)(s & 1) * 8 * nodes;
+        C *sd = side + ((size_t)(s & 1) * p.copies + copy) * 3 * ry;
+        if (active) {
+            const uint32_t skip = kPressure ? flags >> kSkipShift : 0;
+#pragma unroll
+            for (int d = 1; d < 9; d++)
+                if (!((skip >> d) & 1u)) lds_put<S>(e + (d - 1) * nodes + t, o.s[d]);
+            if (flags & kFlagOutletSide) {
+                sd[j] = v[3];
+                sd[ry + j] = v[6];
+                sd[2 * ry + j] = v[7];
+            }
+            if (kPressure && (flags & (kFlagPressureIn | kFlagPressureOut))) {
+#pragma clang fp contract(off)
+                C eq[9];
+                if ((flags & kFlagPressureIn) && i + 2 < rx) {
+                    feq_rep<S>(p.bc.rho_in, o, eq);
+#pragma unroll
+                    for (int d = 1; d < 9; d++)
+                        if ((p.bc.d1 >> d) & 1u) lds_put<S>(e + (d - 1) * nodes + t + 2 * ry, eq[d] + (o.s[d] - o.e[d]));
+                }
+                if ((flags & kFlagPressureOut) && i >= 2) {
+                    feq_rep<S>(p.bc.rho_out, o, eq);
+#pragma unroll
+                    for (int d = 1; d < 9; d++)
+                        if ((p.bc.d2 >> d) & 1u) lds_put<S>(e + (d - 1) * nodes + t - 2 * ry, eq[d] + (o.s[d] - o.e[d]));
+                }
+            }
+        }
+        __syncthreads();
+        v[0] = round_to_storage<S>(o.s[0]);
+#pragma unroll
+        for (int d = 1; d < 9; d++) v[d] = lds_get<S>(e + from[d]);
+        if (rest) {
+#pragma unroll
+            for (int d = 0; d < 9; d++) {
+                const uint32_t kind = (w >> (2 * d)) & 3u;
+                const double k = cls[code].k[d];
+                C c = v[d] - (C)k;  // reflect: v holds the node's own opposite population
+                if constexpr (Io<S>::kDev) c = kind == kSrcConst ? (C)(k - kWd[d]) : c;
+                else c = kind == kSrcConst ? k : c;
+                if (d == 3 || d == 6 || d == 7) c = kind == kSrcOutlet ? sd[outlet_slot(d) * ry + j] : c;
+                v[d] = kind == kSrcStream ? v[d] : c;
+            }
+        }
+    }
+}
+
 __global__ void k_add_step(int64_t *step, int64_t k) { *step += k; }
 
 // AoS records of nine values are 72 (36) bytes apart, so a wavefront's store of
@@ -2788,6 +2961,112 @@ int sweepk_rows(const Geom &g, int rows, int K) {
         r++;
     }
     return std::min(r, lx);
+}
+
+// Where it pays: up to 2^18 nodes in FP64 and 3 * 2^16 in FP32 and FP16 (time
+// of a step, this kernel / the faster of one and two steps per launch, channels
+// with walls: FP64 300x300 2.33 / 4.4 us, 420x180 2.57 / 5.0, 700x250 4.6 / 6.4,
+// 500x500 7.9 / 8.2, 5000x50 8.1 / 10.6, 700x700 14.0 / 11.8; FP32 420x180 1.8 /
+// 4.5, 700x250 2.8 / 4.5, 500x500 5.9 / 5.2, 700x700 9.7 / 7.7; 20x30 FP64 1.6 /
+// 4.1, FP16 50x97 with the pressure fix 1.8 / 4.4).  Larger lattices need several
+// rounds of blocks, whose halos cost more than the launches they save.
+// Time of a launch, from the kernel's own timings on one round of blocks: 3.3
+// us of launch, first loads and last stores, and for each step 0.35 us of
+// barrier and LDS latency and, for every wave that a SIMD holds, 0.4 us of
+// arithmetic in FP64 or 0.12 us in FP32 and FP16.
+TileShape tile_shape(int storage, const Geom &g, const BcView &bc) {
+    TileShape best;
+    const bool f64 = storage == LBM_STORE_F64;
+    if (bc.codes && bc.nclasses > kSweepMaxClasses) return best;
+    if (g.N > (f64 ? 1u << 18 : 3u << 16)) return best;
+    const bool pressure = (bc.flags & kProgPressure) != 0;
+    const size_t elem = f64 ? 8 : (storage == LBM_STORE_F32 ? 4 : 2);
+    const uint32_t tmax = (uint32_t)tile_threads(elem, pressure);
+    const uint32_t wmax = f64 ? (pressure ? 8 : 12) : (pressure ? 12 : 24);  // resident waves a CU (registers)
+    double t_best = 1e30;  // us a step
+    for (int K = 1; K <= 8; K++) {
+        // what a node depends on may cross the seam of the fix only once
+        if (pressure && (uint32_t)K + 4 > g.lx) break;
+        const uint32_t hx = 2 * (K - 1 + (pressure ? 2 : 0)), hy = 2 * (K - 1);  // both sides
+        for (uint32_t ty = 1; ty <= g.ly && ty + hy <= 64 && (ty + hy) * (hx + 1) <= tmax; ty++) {
+            const uint32_t ny = (g.ly + ty - 1) / ty;
+            if (ty < g.ly && (g.ly + ty) / (ty + 1) == ny) continue;  // as many tiles as a wider one
+            for (uint32_t tx = std::min(g.lx, tmax / (ty + hy) - hx); tx >= 1; tx--) {
+                const uint32_t nx = (g.lx + tx - 1) / tx;
+                const uint32_t waves = ((tx + hx) * (ty + hy) + 63) / 64;
+                const uint32_t tiles = nx * ny;
+                if (tiles > 4096) break;  // ever more with fewer rows
+                const uint32_t fit = std::max(1u, wmax / waves);  // blocks a CU
+                const uint32_t rounds = (tiles + 256 * fit - 1) / (256 * fit);
+                const uint32_t per_cu = std::min(fit, (tiles + 255) / 256);
+                const double step = 0.35 + (f64 ? 0.4 : 0.12) * ((waves * per_cu + 3) / 4);
+                const double t = rounds * (3.3 + K * step) / K;
+                if (t < t_best) {
+                    t_best = t;
+                    best.K = K;
+                    best.tx = tx;
+                    best.ty = ty;
+                }
+            }
+        }
+    }
+    return best;
+}
+
+namespace {
+template <class S>
+hipError_t tile_typed(const TileShape &sh, const Geom &g, const StateView &st, int src, const BcView &bc, double omega,
+                      const ProbeView &pr, int64_t slot, hipStream_t s) {
+    using C = typename Io<S>::C;
+    TileParams<S> p;
+    p.src = static_cast<const S *>(st.plane[src]);
+    p.dst = static_cast<S *>(st.plane[src ^ 1]);
+    p.side_prev = static_cast<const C *>(st.side[src]);
+    p.side_next = static_cast<C *>(st.side[src ^ 1]);
+    p.g = g;
+    p.bc = bc;
+    p.omega = omega;
+    const bool probing = pr.cell >= 0 && pr.ring && pr.capacity > 0 && slot + sh.K - 1 >= 0;
+    p.probe_cell = probing ? pr.cell : -1;
+    p.probe_ring = pr.ring;
+    p.probe_cap = pr.capacity;
+    p.probe_slot = slot;
+    p.K = (uint32_t)sh.K;
+    p.tx = sh.tx;
+    p.ty = sh.ty;
+    p.hx = sh.K - 1 + (bc.flags & kProgPressure ? 2 : 0);
+    p.hy = sh.K - 1;
+    p.offx = (p.hx + g.lx - 1) / g.lx * g.lx - p.hx;
+    p.offy = (p.hy + g.ly - 1) / g.ly * g.ly - p.hy;
+    p.tiles_y = (g.ly + p.ty - 1) / p.ty;
+    const uint32_t rx = p.tx + 2 * p.hx, ry = p.ty + 2 * p.hy;
+    p.copies = (rx + g.lx - 1) / g.lx + 1;
+    const uint64_t nodes = (uint64_t)rx * ry;
+    const size_t lds = TileLds<S>((uint32_t)nodes, ry, p.copies, bc.codes ? bc.nclasses : 0).total;
+    if (sh.K < 1 || p.tx < 1 || p.ty < 1 || nodes > 1024 || lds > kLdsLimit) return hipErrorInvalidValue;
+    if ((bc.flags & kProgPressure) && (uint32_t)sh.K + 4 > g.lx) return hipErrorInvalidValue;
+    const unsigned grid = (g.lx + p.tx - 1) / p.tx * p.tiles_y;
+    const unsigned threads = ((unsigned)nodes + 63) / 64 * 64;
+    const bool pressure = (bc.flags & kProgPressure) != 0;
+    if (nodes > (uint64_t)tile_threads(sizeof(S), pressure)) return hipErrorInvalidValue;
+    const void *fn = pressure ? reinterpret_cast<const void *>(k_tile<S, true>)
+                              : reinterpret_cast<const void *>(k_tile<S, false>);
+    hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsLimit);
+    if (e != hipSuccess) return e;
+    void *args[] = {&p};
+    e = hipLaunchKernel(fn, dim3(grid), dim3(threads), args, lds, s);
+    return e != hipSuccess ? e : hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_tile(int storage, const TileShape &sh, const Geom &g, const StateView &st, int src, const BcView &bc,
+                       double omega, const ProbeView &pr, int64_t slot, hipStream_t s) {
+    switch (storage) {
+        case LBM_STORE_F64: return tile_typed<double>(sh, g, st, src, bc, omega, pr, slot, s);
+        case LBM_STORE_F32: return tile_typed<float>(sh, g, st, src, bc, omega, pr, slot, s);
+        case LBM_STORE_F16: return tile_typed<__half>(sh, g, st, src, bc, omega, pr, slot, s);
+    }
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_sweepk(int storage, int K, const Geom &g, const StateView &st, int src, const BcView &bc,

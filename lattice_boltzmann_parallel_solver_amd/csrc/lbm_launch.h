@@ -54,6 +54,13 @@ hipError_t launch_sweepk(int storage, int K, const Geom &g, const StateView &st,
 // As sweep_supported(), and ly <= 1024, FP32 or FP16, its LDS (K - 1 stages of
 // exchange and outlet buffers) within 160 KiB.
 bool sweepk_supported(int storage, const Geom &g, const BcView &bc, int K);
+// K steps in one launch on tiles held in registers and LDS (small lattices).
+// The samples of step s (1-based) go to ring slot probe_slot + s - 1.
+// tile_shape: the fastest tiling of a lattice (K = 0: it has none); a launch
+// may take fewer steps than its K.
+TileShape tile_shape(int storage, const Geom &g, const BcView &bc);
+hipError_t launch_tile(int storage, const TileShape &sh, const Geom &g, const StateView &st, int src, const BcView &bc,
+                       double omega, const ProbeView &pr, int64_t probe_slot, hipStream_t s);
 // Rows per block of the K-step kernel: `rows`, raised until every block
 // (the last one included) holds at least K - 1 rows.
 int sweepk_rows(const Geom &g, int rows, int K);

@@ -61,11 +61,12 @@ struct LaunchCfg {
     int cells_per_thread = 0;  // 0: 16-byte kernel (needs ly % (16/sizeof) == 0), else 1, 2, 4
     int xcd_remap = 1;
     int nt_stores = 0;
-    int steps_per_launch = 1;  // 2: two-step row-sweep kernel where supported
+    int steps_per_launch = 0;  // 0: the library's choice; 1; 2: two-step row sweep where supported; 3, 4
     int sweep_rows = 0;        // output rows per block of the sweep kernel (0: automatic)
     int sweep_tile = 0;        // threads per column tile of the sweep kernel (0: whole rows up to one block)
     int sweep_v = 0;           // columns per thread of column tiles (0: two for FP32/FP16, one for FP64)
     int row_interleave = 1;    // long two-step runs move the state to the range-interleaved row order
+    bool shape_given = false;  // lbm_set_launch was called: steps_per_launch 0 means 1
     int sweep_il = 0;          // (per launch) the buffers are in that order for sweep_rows-row ranges
 };
 
@@ -75,6 +76,12 @@ struct LaunchCfg {
 struct SweepShape {
     int v = 1;
     uint32_t ntiles = 1, tw = 0, lw = 0, threads = 0;
+};
+
+// Steps per launch and output nodes per block of the tile kernel.
+struct TileShape {
+    int K = 0;
+    uint32_t tx = 0, ty = 0;
 };
 
 // One lattice of a batch, with its buffers already resolved for the step

@@ -160,9 +160,12 @@ class Lattice:
         more steps keep the intermediate states on chip (identical results,
         1/K of the population traffic per step).  Rows wider than one kernel
         block run as column tiles with two steps; three and four need FP32 or
-        FP16 rows of at most 1024 columns.  Raises LbmError where the kernel
-        does not apply (pressure fix, fewer than three rows, more than 128
-        boundary classes, LDS)."""
+        FP16 rows of at most 1024 columns.  With 2 or more and automatic rows,
+        small lattices (2^18 nodes FP64, 3 * 2^16 else) take up to eight per
+        launch on tiles.  A lattice on which neither this nor `set_launch` was
+        called takes the number that measured fastest for it.  Raises LbmError
+        where the kernel does not apply (pressure fix, fewer than three rows,
+        more than 128 boundary classes, LDS)."""
         check(_lib.load().lbm_set_temporal(self._h, int(steps_per_launch), int(rows_per_block)))
 
     def set_sweep_tile(self, threads: int = 0, cols_per_thread: int = 0) -> None:

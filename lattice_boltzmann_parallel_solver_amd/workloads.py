@@ -98,6 +98,8 @@ def run_sequential(jobs: Sequence[ChannelJob], steps: int, storage: str = "f32",
                 lat.set_temporal(2)
             except LbmError:
                 pass
+        else:
+            lat.set_temporal(1)
         lat.synchronize()
         t0 = time.perf_counter()
         lat.run(job.omega, steps)
