@@ -125,6 +125,7 @@ struct lbm_ctx {
     double *partials = nullptr;
     double *sums = nullptr;
     LaunchCfg cfg;
+    uint8_t *codes8 = nullptr;  // bc.view.codes8
     // tiling of the tile kernel, worked out by the first run that may take it
     TileShape tile;
     bool tile_ready = false;
@@ -159,6 +160,7 @@ void release(lbm_ctx *c) {
     (void)hipFree(c->stage_rho);
     (void)hipFree(c->stage_u);
     (void)hipFree(c->bc.mem);
+    (void)hipFree(c->codes8);
     (void)hipFree(c->probe.ring);
     (void)hipFree(c->partials);
     (void)hipFree(c->sums);
@@ -300,7 +302,7 @@ int lbm_set_launch(lbm_ctx *c, int v, int xcd, int nt) {
     c->cfg.cells_per_thread = v;
     c->cfg.xcd_remap = xcd ? 1 : 0;
     c->cfg.nt_stores = nt ? 1 : 0;
-    c->cfg.shape_given = true;
+    c->cfg.shape_given = v != 1 || !xcd || nt;  // (the default shape is no request)
     return LBM_OK;
 }
 
@@ -387,9 +389,18 @@ int lbm_set_bc(lbm_ctx *c, const lbm_bc_prog *prog) {
     }
     LBM_HIP_CHECK(hipStreamSynchronize(c->stream), "lbm_set_bc");
     (void)hipFree(c->bc.mem);
+    (void)hipFree(c->codes8);
+    c->codes8 = nullptr;
     c->bc = BcUpload{};
     c->tile_ready = false;
-    if (prog) LBM_HIP_CHECK(upload_bc(*prog, c->bc), "lbm_set_bc: upload");
+    if (prog) {
+        LBM_HIP_CHECK(upload_bc(*prog, c->bc), "lbm_set_bc: upload");
+        if (c->bc.view.nclasses <= 256) {
+            LBM_HIP_CHECK(hipMalloc(reinterpret_cast<void **>(&c->codes8), (size_t)c->g.lx * c->g.pitch), "lbm_set_bc: upload");
+            LBM_HIP_CHECK(launch_codes8(c->g, c->bc.view.codes, c->codes8, c->stream), "lbm_set_bc: byte codes");
+            c->bc.view.codes8 = c->codes8;
+        }
+    }
     return LBM_OK;
 }
 
@@ -478,8 +489,8 @@ int lbm_run(lbm_ctx *c, double omega, int64_t nsteps) {
     const bool probing = c->probe.cell >= 0;
     const int K = run_steps_per_launch(c);
     // Small lattices: several steps per launch on tiles.  A step alone, one
-    // step per launch and row counts or column tiles that the caller chose keep
-    // their kernels.
+    // step per launch and launch shapes, row counts or column tiles that the
+    // caller chose keep their kernels.
     const bool tiles = K != 1 && !c->cfg.shape_given && c->cfg.sweep_rows == 0 && c->cfg.sweep_tile == 0;
     if (tiles && !c->tile_ready) {
         c->tile = tile_shape(c->storage, c->g, c->bc.view);
@@ -494,6 +505,19 @@ int lbm_run(lbm_ctx *c, double omega, int64_t nsteps) {
         c->cur ^= 1;
         c->steps += sh.K;
         left -= sh.K;
+    }
+    // Full rows of two (FP32) or one (FP64) column per thread: three steps per
+    // launch with adjacent columns per lane, under the same conditions.
+    if (tiles && K >= 2) {
+        const SweepVShape sh = sweepv_shape(c->storage, c->g, c->bc.view);
+        for (; sh.K > 0 && left >= sh.K; left -= sh.K) {
+            const int64_t slot = probing ? c->steps - c->probe_base - 1 : -1;
+            LBM_HIP_CHECK(launch_sweepv(c->storage, sh, c->g, c->st, c->cur, c->bc.view, omega, c->probe, slot,
+                                        c->stream),
+                          "three-step sweep kernel");
+            c->cur ^= 1;
+            c->steps += sh.K;
+        }
     }
     if (K >= 3 && sweepk_supported(c->storage, c->g, c->bc.view, K)) {
         for (; left >= K; left -= K) {

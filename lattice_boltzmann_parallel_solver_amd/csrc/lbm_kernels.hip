@@ -1775,6 +1775,545 @@ __global__ __launch_bounds__(kSweepThreads, K == 3 ? 5 : 4) void k_sweepk_batch(
     sweepk_block<S, K, false>(p, (blk - j.block0) * j.rows, smem);
 }
 
+// Stores through a buffer descriptor: lanes whose offset lies past its end
+// store nothing, without a branch (a branch would leave the compiler unable to
+// count the stores in flight, and every wait for a load would drain them).
+using BufRsrc = __amdgpu_buffer_rsrc_t;
+__device__ __forceinline__ BufRsrc run_rsrc(void *base, uint32_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(base);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(((uint64_t)hi << 32) | lo), 0,
+                                             __builtin_amdgcn_readfirstlane(bytes), 0x00027000);
+}
+__device__ __forceinline__ void buf_store(BufRsrc r, uint32_t off, double v) {
+    using V2 = uint32_t __attribute__((ext_vector_type(2)));
+    const V2 d = {(uint32_t)__double2loint(v), (uint32_t)__double2hiint(v)};
+    __builtin_amdgcn_raw_buffer_store_b64(d, r, off, 0, 0);
+}
+
+// ---------------------------------------------------------------------------
+// K steps per launch, V adjacent columns per lane
+//
+// The row sweep again (in iteration it, stage s collides row xa - (K-1) + it -
+// (s-1)), laid out so that the row stays in
+// registers: lane l of wave w holds V adjacent columns, 16 bytes of a plane,
+// so a pull is nine aligned 16-byte loads, a y shift moves V - 1 of its values
+// between a lane's own registers and one over a DPP shift, and only the values
+// at the waves' edges (three each way) pass through LDS.  The kernels with one
+// or two separate columns per thread publish and read six values a node there,
+// which at 2048 columns leaves LDS for one intermediate stage; here a third
+// step fits (24 bytes a node and step in FP32, 48 in FP64), and with V nodes
+// sharing every address and boundary test the row costs fewer instructions.
+//
+// Per iteration: stage 1 (from the prefetched row), the loads of the next row,
+// then each later stage, after a barrier behind which the wave edges of the one
+// before are in LDS.  (One barrier an iteration, later stages taking the last
+// iteration's row as in k_sweepk, keeps another row of all nine directions: 36
+// registers that a third step has not.)  A stage carries, per column, directions 1, 5, 8 of two rows and 0, 2, 4 of one.  A reflecting
+// node's own populations are at hand when its row is passed on, so they
+// replace the streamed ones there and then (directions 3, 6, 7, which the next
+// row still has to bring, wait in LDS).
+//
+// Iterations before the first and after the last output row run every stage
+// on rows whose results are not kept: their stores go to an empty buffer range.
+// So the loop body has no branch around its loads and stores, and the wait for
+// the prefetched row does not drain the stores behind it.
+//
+// Each wave takes one of two loops: the waves with boundary nodes in the
+// block's rows one that looks classes up, the others one without that code.
+// ---------------------------------------------------------------------------
+template <class S>
+struct SweepVParams {
+    const S *src;
+    S *dst;
+    const typename Io<S>::C *side_prev;
+    typename Io<S>::C *side_next;
+    Geom g;
+    BcView bc;
+    double omega;
+    uint32_t probe_row, probe_col;  // probe_row = ~0: no probe
+    double *probe_out[3];           // where the sample of step s = 1 .. K goes, or null
+    uint32_t rows;                  // output rows per block
+};
+
+struct SweepVLds {
+    uint32_t edge, refl, side, cls, flag, total;
+};
+
+// A boundary class as the kernel applies it: `a` is what a reflection
+// subtracts, or the constant in the storage's representation.
+template <class C>
+struct ClassV {
+    uint32_t src, flags;
+    C a[9];
+};
+constexpr uint32_t kFlagHasOutlet = 1u << 30;  // (ClassV) some direction copies the outlet
+
+// `cols`: columns a block holds (V times its threads).
+template <class S, int K>
+__host__ __device__ inline SweepVLds sweepv_lds(uint32_t cols, uint32_t waves, uint32_t nclasses, bool outlet, uint32_t rows) {
+    using C = typename Io<S>::C;
+    SweepVLds L;
+    L.edge = 0;  // per stage < K and parity: 4 values for each of waves + 1 upward and waves downward slots
+    L.refl = (uint32_t)align16((K - 1) * 2 * (2 * waves + 1) * 4 * sizeof(C));
+    L.side = L.refl + (nclasses ? (K - 1) * 3 * cols * (uint32_t)sizeof(C) : 0);
+    L.cls = L.side + (outlet ? (K - 1) * 3 * cols * (uint32_t)sizeof(C) : 0);
+    L.flag = (uint32_t)align16(L.cls + nclasses * sizeof(ClassV<C>));
+    L.total = L.flag + (nclasses ? (rows + 2 * (K - 1)) * waves : 0);
+    return L;
+}
+
+constexpr int kSweepVSteps = 3;
+
+// One value over the wave: lane n from lane n - 1 (n + 1), lane 0 (63) `edge`.
+template <bool kUp>
+__device__ __forceinline__ float wave_shift(float v, float edge) {
+    constexpr int ctrl = kUp ? 0x138 : 0x130;  // wave_shr:1 / wave_shl:1
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(edge), __float_as_int(v), ctrl, 0xf, 0xf, false));
+}
+template <bool kUp>
+__device__ __forceinline__ double wave_shift(double v, double edge) {
+    constexpr int ctrl = kUp ? 0x138 : 0x130;
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(v), ctrl, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(v), ctrl, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ float lane_value(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// V values of 16 bytes.
+template <class S>
+struct Quad {
+    static constexpr int V = 16 / sizeof(S);
+    using W4 = uint32_t __attribute__((ext_vector_type(4)));
+    S v[V];
+    __device__ void load(BufRsrc r, uint32_t voff, uint32_t soff) {
+        const W4 w = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+        if constexpr (sizeof(S) == 4) {
+#pragma unroll
+            for (int j = 0; j < V; j++) v[j] = __uint_as_float(w[j]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < V; j++) v[j] = __hiloint2double((int)w[2 * j + 1], (int)w[2 * j]);
+        }
+    }
+    __device__ void load_one(int j, BufRsrc r, uint32_t voff) {
+        if constexpr (sizeof(S) == 4) {
+            v[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0));
+        } else {
+            using W2 = uint32_t __attribute__((ext_vector_type(2)));
+            const W2 w = __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, 0);
+            v[j] = __hiloint2double((int)w[1], (int)w[0]);
+        }
+    }
+    // The offset goes into the vector operand.  With it in a scalar register
+    // the compiler puts no wait state between a 16-byte store and an
+    // instruction that overwrites the stored registers, and single lanes then
+    // stored the new values here.
+    __device__ static void store(BufRsrc r, uint32_t off, const S x[V]) {
+        W4 w;
+        if constexpr (sizeof(S) == 4) {
+#pragma unroll
+            for (int j = 0; j < V; j++) w[j] = __float_as_uint(x[j]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < V; j++) {
+                w[2 * j] = (uint32_t)__double2loint(x[j]);
+                w[2 * j + 1] = (uint32_t)__double2hiint(x[j]);
+            }
+        }
+        __builtin_amdgcn_raw_buffer_store_b128(w, r, off, 0, 0);
+    }
+};
+
+template <class S, int K>
+__global__ __launch_bounds__(512) void k_sweepv(SweepVParams<S> p) {
+    using C = typename Io<S>::C;
+    constexpr int V = Quad<S>::V;
+    constexpr int NB = K - 1;  // hand-overs between stages
+    extern __shared__ __align__(16) unsigned char smem[];
+    const Geom &g = p.g;
+    const uint32_t lx = g.lx, ly = g.ly, pitch = g.pitch;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, NW = blockDim.x >> 6;
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t blk = xcd_block(blockIdx.x, gridDim.x);
+    const uint32_t xa = blk * p.rows, R = min(p.rows, lx - xa);
+    const uint32_t cols = blockDim.x * V;
+    const uint32_t l0 = tid * V;  // the lane's first column
+    const bool has_bc = p.bc.chunk != nullptr;
+    const bool outlet = has_bc && (p.bc.flags & kProgOutlet);
+    const SweepVLds L = sweepv_lds<S, K>(cols, NW, has_bc ? p.bc.nclasses : 0, outlet, p.rows);
+    C *edge = reinterpret_cast<C *>(smem);
+    C *refl = reinterpret_cast<C *>(smem + L.refl);
+    C *side = reinterpret_cast<C *>(smem + L.side);
+    ClassV<C> *cls = reinterpret_cast<ClassV<C> *>(smem + L.cls);
+    uint8_t *wflag = smem + L.flag;
+    // edge slots: up(b, par, w) what wave w takes from below (three values),
+    // dn(b, par, w) what wave w - 1 takes from wave w
+    auto up = [&](int b, uint32_t par, uint32_t w) { return edge + ((b * 2 + par) * (2 * NW + 1) + w) * 4; };
+    auto dn = [&](int b, uint32_t par, uint32_t w) { return edge + ((b * 2 + par) * (2 * NW + 1) + NW + 1 + w) * 4; };
+    // row of iteration `it` back by `b` rows: kept as wrapped counters
+    auto wrap_back = [&](uint32_t x, uint32_t b) { return x >= b ? x - b : x + lx - b; };
+    const uint32_t nrows1 = R + 2 * NB;  // stage-1 rows that are used
+    if (has_bc) {
+        for (uint32_t i = tid; i < p.bc.nclasses; i += blockDim.x) {
+            const ClassEntry &ce = p.bc.classes[i];
+            uint32_t f = ce.flags;
+#pragma unroll
+            for (int d = 0; d < 9; d++) {
+                const uint32_t kind = (ce.src >> (2 * d)) & 3u;
+                if (kind == kSrcOutlet) f |= kFlagHasOutlet;
+                cls[i].a[d] = Io<S>::kDev && kind == kSrcConst ? (C)(ce.k[d] - kWd[d]) : (C)ce.k[d];
+            }
+            cls[i].src = ce.src;
+            cls[i].flags = f;
+        }
+        for (uint32_t i = tid; i < nrows1 * NW; i += blockDim.x) {
+            const uint32_t rr = i / NW, w = i - rr * NW;
+            const uint32_t r = (xa + rr + lx - NB) % lx;
+            const uint8_t *wr = p.bc.wave + (size_t)r * g.wpr;
+            uint8_t f = 0;
+            for (uint32_t c = w * V; c < min((w + 1) * V, g.wpr); c++) f |= wr[c];
+            wflag[i] = f;
+        }
+    }
+    __syncthreads();
+    // the lane's vector in memory (lanes past the row repeat the last one) and
+    // its place in a stored row (or past every row's end)
+    const uint32_t g0 = min(l0, (ly - 1) / V * V);
+    const uint32_t voff = g0 * (uint32_t)sizeof(S);
+    const uint32_t vst = l0 < pitch ? l0 * (uint32_t)sizeof(S) : 0x7ffffff0u;
+    const uint32_t plane = pitch * (uint32_t)sizeof(S), row_bytes = 9 * plane;
+    auto row_rsrc = [&](const S *base, uint32_t slot, uint32_t bytes) {
+        return run_rsrc(const_cast<S *>(base) + (size_t)slot * 9 * pitch, bytes);
+    };
+    // the wave-edge values of a pulled row: lane a < 6 fetches direction 2, 5,
+    // 6 (from the column before the wave's first) or 4, 7, 8 (after its last)
+    const uint32_t ea = min(lane, 5u);
+    const uint32_t edir = ea < 3 ? (ea == 0 ? 2 : 4 + ea) : (ea == 3 ? 4 : 3 + ea);
+    const bool wlast = wv == NW - 1;
+    const uint32_t ecol = ea < 3 ? (wv == 0 ? ly - 1 : wv * 64 * V - 1) : (wlast ? 0 : (wv + 1) * 64 * V);
+    auto special = [&](uint32_t rr) -> bool {
+        return has_bc && __builtin_amdgcn_readfirstlane(wflag[min(rr, nrows1 - 1) * NW + wv]) != 0;
+    };
+    // class codes of the lane's columns in one row, a byte each
+    // l0 computed anew: what boundary branches derive from it is not kept in
+    // registers over the loop
+    auto fresh_l0 = [&]() {
+        uint32_t l = l0;
+        asm volatile("" : "+v"(l));
+        return l;
+    };
+    auto load_codes = [&](uint32_t rr, uint32_t x) -> uint32_t {
+        if (!special(rr)) return 0;
+        const uint8_t *at = p.bc.codes8 + (size_t)x * pitch + g0;
+        if constexpr (V == 4) return *reinterpret_cast<const uint32_t *>(at);
+        else return *reinterpret_cast<const uint16_t *>(at);
+    };
+    auto code_of = [](uint32_t c, int j) { return (c >> (8 * j)) & 255u; };
+
+    Quad<S> pf[9];
+    Quad<S> eg;  // (one value of it)
+    const BufRsrc rsrc_all = run_rsrc(const_cast<S *>(p.src), lx * row_bytes);  // below 4 GiB
+    auto prefetch = [&](auto sp_tag, uint32_t rr, uint32_t x, uint32_t codes) {
+        const uint32_t xm = x == 0 ? lx - 1 : x - 1, xp = x + 1 == lx ? 0 : x + 1;
+        if (decltype(sp_tag)::value && special(rr)) {
+            // value by value, shifted, a reflected direction from the node's own
+            // opposite population
+            const uint32_t l = fresh_l0();
+#pragma unroll
+            for (int j = 0; j < V; j++) {
+                const uint32_t y = min(l + j, ly - 1), ym = y == 0 ? ly - 1 : y - 1, yp = y + 1 == ly ? 0 : y + 1;
+                const uint32_t c = code_of(codes, j);
+                const uint32_t w = c ? cls[c].src : 0u;
+                const uint32_t oy = y * (uint32_t)sizeof(S), om = ym * (uint32_t)sizeof(S), op = yp * (uint32_t)sizeof(S);
+#pragma unroll
+                for (int i = 0; i < 9; i++) {
+                    const uint32_t row = kCX[i] == 1 ? xm : (kCX[i] == -1 ? xp : x);
+                    const uint32_t pulled = row * row_bytes + i * plane + (kCY[i] == 1 ? om : (kCY[i] == -1 ? op : oy));
+                    const uint32_t own = x * row_bytes + kOpp[i] * plane + oy;
+                    pf[i].load_one(j, rsrc_all, ((w >> (2 * i)) & 3u) == kSrcReflect ? own : pulled);
+                }
+            }
+        } else {
+            const BufRsrc r0 = row_rsrc(p.src, x, row_bytes), rm = row_rsrc(p.src, xm, row_bytes), rp = row_rsrc(p.src, xp, row_bytes);
+#pragma unroll
+            for (int i = 0; i < 9; i++) pf[i].load(kCX[i] == 1 ? rm : (kCX[i] == -1 ? rp : r0), voff, i * plane);
+            const uint32_t es = edir == 2 || edir == 4 ? x : (edir == 5 || edir == 8 ? xm : xp);
+            eg.load_one(0, rsrc_all, es * row_bytes + edir * plane + ecol * (uint32_t)sizeof(S));
+        }
+    };
+    // apply a node's class: v holds the streamed values, refl(d, v[d]) the
+    // reflected ones, out(q) the outlet's
+    auto apply = [&](uint32_t c, C v[9], auto out, auto refl_value) {
+        const ClassV<C> &ce = cls[c];
+        const uint32_t w = ce.src, flags = ce.flags;
+        C o3[3] = {0, 0, 0};
+        if (flags & kFlagHasOutlet) {
+#pragma unroll
+            for (int q = 0; q < 3; q++) o3[q] = out(q);
+        }
+#pragma unroll
+        for (int d = 0; d < 9; d++) {
+            const uint32_t kind = (w >> (2 * d)) & 3u;
+            const C a = ce.a[d], rv = refl_value(d, v[d]);
+            C n = kind == kSrcReflect ? rv - a : v[d];
+            n = kind == kSrcConst ? a : n;
+            if (d == 3 || d == 6 || d == 7) n = kind == kSrcOutlet ? o3[outlet_slot(d)] : n;
+            v[d] = n;
+        }
+        return flags;
+    };
+    auto probe = [&](int s, uint32_t col, const NodeOut<S> &o) {
+        double *pr = p.probe_out[s - 1];
+        if (col == p.probe_col && pr) {
+            pr[0] = o.rho;
+            pr[1] = (double)o.ux;
+            pr[2] = (double)o.uy;
+        }
+    };
+    // column of the lane's value j where it is an output column, else ~0
+    auto out_col = [&](int j) -> uint32_t {
+        const uint32_t l = fresh_l0() + j;
+        return l < ly ? l : ~0u;
+    };
+
+    C A[NB][V][3], B[NB][V][3], Cc[NB][V][3];  // per hand-over, as in sweepk_block
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int j = 0; j < V; j++)
+#pragma unroll
+            for (int q = 0; q < 3; q++) A[b][j][q] = B[b][j][q] = Cc[b][j][q] = 0;
+
+    // publish the wave-edge values of one stage's row
+    auto put_edges = [&](int b, uint32_t par, const C s[V][9]) {
+        if (lane == 63) {
+            C *u = up(b, par, wv + 1);
+            u[0] = s[V - 1][2];
+            u[1] = s[V - 1][5];
+            u[2] = s[V - 1][6];
+        }
+        if (lane == 0) {
+            C *d = dn(b, par, wv);
+            d[0] = s[0][4];
+            d[1] = s[0][7];
+            d[2] = s[0][8];
+        }
+        if (wlast) {  // column ly - 1 is what wave 0 takes from below
+            C *u = up(b, par, 0);
+            const uint32_t l = fresh_l0();
+#pragma unroll
+            for (int j = 0; j < V; j++)
+                if (l + j == ly - 1) {
+                    u[0] = s[j][2];
+                    u[1] = s[j][5];
+                    u[2] = s[j][6];
+                }
+        }
+    };
+    // y[j][i] = s streamed in y; lower / upper: the edge values of directions
+    // 2, 5, 6 / 4, 7, 8.  In the last wave the value past the row's
+    // last (a pad column, not used itself) becomes column 0's.
+    auto stream_y = [&](C s[V][9], const C lower[3], const C upper[3], C y[V][9]) {
+        constexpr int kUp[3] = {2, 5, 6}, kDn[3] = {4, 7, 8};
+        if (wlast) {
+            const uint32_t l = fresh_l0();
+#pragma unroll
+            for (int j = 0; j < V; j++)
+#pragma unroll
+                for (int q = 0; q < 3; q++) s[j][kDn[q]] = l + j == ly ? upper[q] : s[j][kDn[q]];
+        }
+#pragma unroll
+        for (int j = 0; j < V; j++) {
+            y[j][0] = s[j][0];
+            y[j][1] = s[j][1];
+            y[j][3] = s[j][3];
+        }
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            const C lo = wave_shift<true>(s[V - 1][kUp[q]], lower[q]);
+            const C hi = wave_shift<false>(s[0][kDn[q]], upper[q]);
+#pragma unroll
+            for (int j = 0; j < V; j++) {
+                y[j][kUp[q]] = j == 0 ? lo : s[j > 0 ? j - 1 : 0][kUp[q]];
+                y[j][kDn[q]] = j == V - 1 ? hi : s[j < V - 1 ? j + 1 : j][kDn[q]];
+            }
+        }
+    };
+
+    auto sweep = [&](auto sp_tag) {
+        constexpr bool kSp = decltype(sp_tag)::value;
+        uint32_t x = wrap_back(xa, NB);  // stage-1 row of the iteration
+        auto next_row = [&](uint32_t r) { return r + 1 == lx ? 0 : r + 1; };
+        uint32_t c0 = kSp ? load_codes(0, x) : 0, c1 = kSp ? load_codes(1, next_row(x)) : 0, c2 = 0;
+        uint32_t hist[NB];  // codes of rows x - 1, x - 2, ..
+#pragma unroll
+        for (int j = 0; j < NB; j++) hist[j] = 0;
+        prefetch(sp_tag, 0, x, c0);
+        for (uint32_t it = 0; it < nrows1; it++) {
+            const uint32_t par = it & 1;
+            const uint32_t x1 = it + 1 < nrows1 ? next_row(x) : x;  // the row to prefetch (the last one again)
+            // ---- stage 1 on row x
+            C cur[V][9];  // the last stage's output
+            {
+                C v[V][9];
+                if (kSp && special(it)) {
+#pragma unroll
+                    for (int j = 0; j < V; j++)
+#pragma unroll
+                        for (int i = 0; i < 9; i++) v[j][i] = pf[i].v[j];
+                } else {
+                    C raw[V][9];
+#pragma unroll
+                    for (int j = 0; j < V; j++)
+#pragma unroll
+                        for (int i = 0; i < 9; i++) raw[j][i] = pf[i].v[j];
+                    const C lower[3] = {lane_value(eg.v[0], 0), lane_value(eg.v[0], 1), lane_value(eg.v[0], 2)};
+                    const C upper[3] = {lane_value(eg.v[0], 3), lane_value(eg.v[0], 4), lane_value(eg.v[0], 5)};
+                    stream_y(raw, lower, upper, v);
+                }
+                const bool own_row = it >= NB && it < R + NB;
+#pragma unroll
+                for (int j = 0; j < V; j++) {
+                    uint32_t flags = 0;
+                    const uint32_t c = code_of(c0, j);
+                    if (kSp && c) {
+                        const uint32_t l = fresh_l0() + j;
+                        flags = apply(c, v[j], [&](int q) { return p.side_prev[(size_t)min(l, ly - 1) * 3 + q]; },
+                                      [&](int, C own) { return own; });
+                        if (flags & kFlagOutletSide) {
+                            side[0 * cols + l] = v[j][3];
+                            side[1 * cols + l] = v[j][6];
+                            side[2 * cols + l] = v[j][7];
+                        }
+                    }
+                    NodeOut<S> o;
+                    collide_node<S>(v[j], p.omega, o);
+#pragma unroll
+                    for (int i = 0; i < 9; i++) cur[j][i] = round_to_storage<S>(o.s[i]);
+                    if (x == p.probe_row && own_row) probe(1, out_col(j), o);
+                }
+            }
+            put_edges(0, par, cur);
+            c2 = kSp && it + 2 < nrows1 ? load_codes(it + 2, next_row(x1)) : 0u;
+            prefetch(sp_tag, it + 1, x1, c1);
+            // ---- stages 2 .. K, each on the row that the one before passes on
+#pragma unroll
+            for (int s = 2; s <= K; s++) {
+                __syncthreads();
+                const int b = s - 2;
+                C(*in)[9] = cur;
+                C lower[3], upper[3], Y[V][9];
+                const C *lo = up(b, par, wv), *hi = dn(b, par, wlast ? 0 : wv + 1);
+#pragma unroll
+                for (int q = 0; q < 3; q++) {
+                    lower[q] = lo[q];
+                    upper[q] = hi[q];
+                }
+                stream_y(in, lower, upper, Y);
+                const uint32_t back = s - 1;
+                const uint32_t r = wrap_back(x, back);
+                const uint32_t codes = hist[s - 2];                            // of row r
+                const uint32_t codes_in = s == 2 ? c0 : hist[s > 2 ? s - 3 : 0];  // of the arriving row r + 1
+                const bool own_row = it >= back + NB && it < back + NB + R;
+                C out[V][9];
+#pragma unroll
+                for (int j = 0; j < V; j++) {
+                    C v[9] = {B[b][j][0], A[b][j][0], B[b][j][1], Y[j][3], B[b][j][2], A[b][j][1], Y[j][6], Y[j][7], A[b][j][2]};
+                    uint32_t flags = 0;
+                    const uint32_t c = code_of(codes, j);
+                    if (kSp && c) {
+                        const uint32_t l = fresh_l0() + j;
+                        flags = apply(c, v, [&](int q) { return side[(b * 3 + q) * cols + l]; },
+                                      [&](int d, C own) {
+                                          return d == 3 || d == 6 || d == 7 ? refl[(b * 3 + outlet_slot(d)) * cols + l] : own;
+                                      });
+                        if (flags & kFlagOutletSide) {
+                            if (s < K) {
+                                side[((b + 1) * 3 + 0) * cols + l] = v[3];
+                                side[((b + 1) * 3 + 1) * cols + l] = v[6];
+                                side[((b + 1) * 3 + 2) * cols + l] = v[7];
+                            } else if (own_row && out_col(j) != ~0u) {
+                                C *sn = p.side_next + (size_t)out_col(j) * 3;
+                                sn[0] = v[3];
+                                sn[1] = v[6];
+                                sn[2] = v[7];
+                            }
+                        }
+                    }
+                    NodeOut<S> o;
+                    collide_node<S>(v, p.omega, o);
+#pragma unroll
+                    for (int i = 0; i < 9; i++) out[j][i] = s < K ? round_to_storage<S>(o.s[i]) : o.s[i];
+                    if (r == p.probe_row && own_row) probe(s, out_col(j), o);
+                    // hand the arriving row over; where its nodes reflect, their own
+                    // populations take the streamed ones' places
+                    A[b][j][0] = Cc[b][j][0];
+                    A[b][j][1] = Cc[b][j][1];
+                    A[b][j][2] = Cc[b][j][2];
+                    B[b][j][0] = Y[j][0];
+                    B[b][j][1] = Y[j][2];
+                    B[b][j][2] = Y[j][4];
+                    Cc[b][j][0] = Y[j][1];
+                    Cc[b][j][1] = Y[j][5];
+                    Cc[b][j][2] = Y[j][8];
+                    const uint32_t ci = code_of(codes_in, j);
+                    if (kSp && ci) {
+                        const uint32_t w = cls[ci].src;
+                        auto is = [&](int d) { return ((w >> (2 * d)) & 3u) == kSrcReflect; };
+                        A[b][j][0] = is(1) ? in[j][3] : A[b][j][0];
+                        A[b][j][1] = is(5) ? in[j][7] : A[b][j][1];
+                        A[b][j][2] = is(8) ? in[j][6] : A[b][j][2];
+                        B[b][j][1] = is(2) ? in[j][4] : B[b][j][1];
+                        B[b][j][2] = is(4) ? in[j][2] : B[b][j][2];
+                        const uint32_t l = fresh_l0() + j;
+                        refl[(b * 3 + 0) * cols + l] = in[j][1];
+                        refl[(b * 3 + 1) * cols + l] = in[j][8];
+                        refl[(b * 3 + 2) * cols + l] = in[j][5];
+                    }
+                }
+                if (s == K) {
+                    const BufRsrc rd = row_rsrc(p.dst, r, own_row ? row_bytes : 0);
+#pragma unroll
+                    for (int i = 0; i < 9; i++) {
+                        S o[V];
+#pragma unroll
+                        for (int j = 0; j < V; j++) o[j] = out[j][i];
+                        Quad<S>::store(rd, vst + i * plane, o);
+                    }
+                } else {
+                    put_edges(b + 1, par, out);
+#pragma unroll
+                    for (int j = 0; j < V; j++)
+#pragma unroll
+                        for (int i = 0; i < 9; i++) cur[j][i] = out[j][i];
+                }
+            }
+#pragma unroll
+            for (int j = NB - 1; j > 0; j--) hist[j] = hist[j - 1];
+            hist[0] = c0;
+            c0 = c1;
+            c1 = c2;
+            x = next_row(x);
+        }
+    };
+    bool any = false;
+    if (has_bc) {
+        uint32_t f = 0;
+        for (uint32_t rr = lane; rr < nrows1; rr += 64) f |= wflag[rr * NW + wv];
+        any |= __builtin_amdgcn_ballot_w64(f != 0) != 0;
+    }
+    if (__builtin_amdgcn_readfirstlane(any)) sweep(Flag<true>{});
+    else sweep(Flag<false>{});
+}
+
 // ---------------------------------------------------------------------------
 // K steps per launch on tiles held in registers and LDS, for small lattices
 //
@@ -2220,23 +2759,6 @@ struct StepAosParams {
     uint32_t strips;  // column strips of W output columns
     uint32_t W;       // at most kBlock - 2
 };
-
-// Stores through a buffer descriptor: lanes whose offset lies past its end
-// store nothing, without a branch (a branch would leave the compiler unable to
-// count the stores in flight, and every wait for a load would drain them).
-using BufRsrc = __amdgpu_buffer_rsrc_t;
-__device__ __forceinline__ BufRsrc run_rsrc(void *base, uint32_t bytes) {
-    const uint64_t a = reinterpret_cast<uint64_t>(base);
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
-    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(((uint64_t)hi << 32) | lo), 0,
-                                             __builtin_amdgcn_readfirstlane(bytes), 0x00027000);
-}
-__device__ __forceinline__ void buf_store(BufRsrc r, uint32_t off, double v) {
-    using V2 = uint32_t __attribute__((ext_vector_type(2)));
-    const V2 d = {(uint32_t)__double2loint(v), (uint32_t)__double2hiint(v)};
-    __builtin_amdgcn_raw_buffer_store_b64(d, r, off, 0, 0);
-}
 
 constexpr uint32_t kStepClasses = 64;  // classes kept in LDS (all composites have fewer)
 
@@ -2963,6 +3485,74 @@ int sweepk_rows(const Geom &g, int rows, int K) {
     return std::min(r, lx);
 }
 
+// Where it beats the kernels with separate columns: rows that fill seven or
+// eight waves of adjacent columns (FP32 1537 to 2048 columns, FP64 769 to 1024)
+// and twelve or more rows a block.  Time of a step, channels with walls, this
+// kernel with three steps / two steps per launch: FP32 8192x2048 93 us / 118,
+// 4200x1800 55.8 / 63.1, 2048x2048 (8 rows a block) 34.1 / 34.2, 8192x1300 84 /
+// 82, 1024x2048 24.7 / 18.7; FP64 8192x1024 99 / 124, 4096x1024 58.6 / 65.5,
+// 4096x768 54.0 / 50.7, 2000x1000 35.8 / 34.2.  An iteration's three barriers
+// and its chain of stages take 7 us whatever the row's width, which the memory
+// traffic of a full row covers (8192x2048 periodic: 81 us, 5.9 TB/s with the
+// halo rows) and a narrower one's does not; column tiles with halos lost too
+// (FP64 4200x1800 142 / 118).  With two steps it lost everywhere (FP32
+// 8192x2048 130).
+SweepVShape sweepv_shape(int storage, const Geom &g, const BcView &bc) {
+    SweepVShape sh;
+    if (storage == LBM_STORE_F16 || (bc.flags & kProgPressure) || sweep_big(storage, g)) return sh;
+    const bool f64 = storage == LBM_STORE_F64;
+    const uint32_t ncls = bc.chunk ? bc.nclasses : 0, V = f64 ? 2 : 4;
+    if (ncls > kSweepMaxClasses || (ncls && !bc.codes8)) return sh;
+    const uint32_t waves = (g.ly + 64 * V - 1) / (64 * V);
+    if (waves < 7 || waves > 8) return sh;
+    // one block a CU, in the fewest rounds
+    const uint32_t slots = 256, rounds = (g.lx + slots * kSweepMaxRows - 1) / (slots * kSweepMaxRows);
+    sh.rows = (g.lx + rounds * slots - 1) / (rounds * slots);
+    if (sh.rows < 12) return sh;
+    const bool outlet = ncls && (bc.flags & kProgOutlet);
+    sh.threads = 64 * waves;
+    sh.lds = f64 ? sweepv_lds<double, kSweepVSteps>(sh.threads * V, waves, ncls, outlet, sh.rows).total
+                 : sweepv_lds<float, kSweepVSteps>(sh.threads * V, waves, ncls, outlet, sh.rows).total;
+    if (sh.lds <= kLdsLimit) sh.K = kSweepVSteps;
+    return sh;
+}
+
+namespace {
+template <class S>
+hipError_t sweepv_typed(const SweepVShape &sh, const Geom &g, const StateView &st, int src, const BcView &bc, double omega,
+                        const ProbeView &pr, int64_t slot, hipStream_t s) {
+    using C = typename Io<S>::C;
+    SweepVParams<S> p;
+    p.src = static_cast<const S *>(st.plane[src]);
+    p.dst = static_cast<S *>(st.plane[src ^ 1]);
+    p.side_prev = static_cast<const C *>(st.side[src]);
+    p.side_next = static_cast<C *>(st.side[src ^ 1]);
+    p.g = g;
+    p.bc = bc;
+    p.omega = omega;
+    const bool probing = pr.cell >= 0 && pr.ring && pr.capacity > 0;
+    p.probe_row = probing ? (uint32_t)(pr.cell / g.ly) : ~0u;
+    p.probe_col = probing ? (uint32_t)(pr.cell % g.ly) : ~0u;
+    for (int q = 0; q < kSweepVSteps; q++)
+        p.probe_out[q] = probing && slot + q >= 0 ? pr.ring + 3 * ((slot + q) % pr.capacity) : nullptr;
+    p.rows = sh.rows;
+    const void *fn = reinterpret_cast<const void *>(k_sweepv<S, kSweepVSteps>);
+    hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsLimit);
+    if (e != hipSuccess) return e;
+    void *args[] = {&p};
+    e = hipLaunchKernel(fn, dim3((g.lx + sh.rows - 1) / sh.rows), dim3(sh.threads), args, sh.lds, s);
+    return e != hipSuccess ? e : hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_sweepv(int storage, const SweepVShape &sh, const Geom &g, const StateView &st, int src, const BcView &bc,
+                         double omega, const ProbeView &pr, int64_t slot, hipStream_t s) {
+    if (sh.K != kSweepVSteps) return hipErrorInvalidValue;
+    if (storage == LBM_STORE_F64) return sweepv_typed<double>(sh, g, st, src, bc, omega, pr, slot, s);
+    if (storage == LBM_STORE_F32) return sweepv_typed<float>(sh, g, st, src, bc, omega, pr, slot, s);
+    return hipErrorInvalidValue;
+}
+
 // Where it pays: up to 2^18 nodes in FP64 and 3 * 2^16 in FP32 and FP16 (time
 // of a step, this kernel / the faster of one and two steps per launch, channels
 // with walls: FP64 300x300 2.33 / 4.4 us, 420x180 2.57 / 5.0, 700x250 4.6 / 6.4,
@@ -3270,6 +3860,20 @@ hipError_t launch_row_sweep_probe(const void *src, void *dst, uint32_t lx, uint3
         else
             hipLaunchKernelGGL((k_row_sweep_probe<2, false>), dim3(grid), dim3(1024), 0, s, in, out, lx, pitch2, rows, L);
     }
+    return hipGetLastError();
+}
+
+namespace {
+__global__ __launch_bounds__(kBlock) void k_codes8(Geom g, const uint16_t *__restrict__ codes, uint8_t *__restrict__ out) {
+    const uint32_t y = blockIdx.x * kBlock + threadIdx.x;
+    if (y >= g.pitch) return;
+    for (uint32_t x = blockIdx.y; x < g.lx; x += gridDim.y)
+        out[(size_t)x * g.pitch + y] = y < g.ly ? (uint8_t)codes[(size_t)x * g.ly + y] : 0;
+}
+}  // namespace
+
+hipError_t launch_codes8(const Geom &g, const uint16_t *codes, uint8_t *codes8, hipStream_t s) {
+    hipLaunchKernelGGL(k_codes8, dim3((g.pitch + kBlock - 1) / kBlock, std::min(g.lx, 4096u)), dim3(kBlock), 0, s, g, codes, codes8);
     return hipGetLastError();
 }
 

@@ -54,6 +54,14 @@ hipError_t launch_sweepk(int storage, int K, const Geom &g, const StateView &st,
 // As sweep_supported(), and ly <= 1024, FP32 or FP16, its LDS (K - 1 stages of
 // exchange and outlet buffers) within 160 KiB.
 bool sweepk_supported(int storage, const Geom &g, const BcView &bc, int K);
+// codes (lx rows of ly 16-bit codes) to codes8 (rows of pitch bytes, the pad 0).
+hipError_t launch_codes8(const Geom &g, const uint16_t *codes, uint8_t *codes8, hipStream_t s);
+// Three steps in one launch, adjacent columns per lane (FP64, FP32; no pressure
+// fix, at most 128 classes, state buffers below 4 GiB): the shape, K = 0 where it
+// does not apply or another kernel is faster.  Probe slots as launch_sweepk.
+SweepVShape sweepv_shape(int storage, const Geom &g, const BcView &bc);
+hipError_t launch_sweepv(int storage, const SweepVShape &sh, const Geom &g, const StateView &st, int src, const BcView &bc,
+                         double omega, const ProbeView &pr, int64_t probe_slot, hipStream_t s);
 // K steps in one launch on tiles held in registers and LDS (small lattices).
 // The samples of step s (1-based) go to ring slot probe_slot + s - 1.
 // tile_shape: the fastest tiling of a lattice (K = 0: it has none); a launch

@@ -23,6 +23,9 @@ struct BcView {
     double rho_in = 0, rho_out = 0;        // pressure fix
     uint32_t d1 = 0, d2 = 0;
     uint32_t flags = 0;                    // kProg*
+    // codes as bytes, rows `pitch` apart as the state's (with a context's own
+    // tables of at most 256 classes; the pad holds 0)
+    const uint8_t *codes8 = nullptr;
 };
 
 // Geometry with a precomputed divisor for node -> (x, y).  Node n = x*ly + y
@@ -82,6 +85,12 @@ struct SweepShape {
 struct TileShape {
     int K = 0;
     uint32_t tx = 0, ty = 0;
+};
+
+// Launch shape of the three-step sweep with adjacent columns per lane.
+struct SweepVShape {
+    int K = 0;  // steps per launch; 0: another kernel is faster, or it does not apply
+    uint32_t threads = 0, rows = 0, lds = 0;
 };
 
 // One lattice of a batch, with its buffers already resolved for the step
