@@ -144,6 +144,10 @@ bool three_steps_pay(int storage, unsigned waves) {
 // order (moving the state there and back costs about two launches).
 constexpr int64_t kInterleaveMinPairs = 32;
 constexpr int kInterleaveMinRows = 16;
+// Smallest lattice with the pressure fix that sweeps several steps per launch.
+uint32_t seam_nodes(int storage) {
+    return storage == LBM_STORE_F64 ? 1u << 20 : (storage == LBM_STORE_F32 ? 3u << 20 : 1u << 22);
+}
 
 // Bytes of one state buffer: nine planes of lx rows, `pitch` elements a row.
 size_t plane_bytes(const lbm_ctx *c) { return 9 * (size_t)c->g.lx * c->g.pitch * plane_elem(c->storage); }
@@ -395,7 +399,7 @@ int lbm_set_bc(lbm_ctx *c, const lbm_bc_prog *prog) {
     c->tile_ready = false;
     if (prog) {
         LBM_HIP_CHECK(upload_bc(*prog, c->bc), "lbm_set_bc: upload");
-        if (c->bc.view.nclasses <= 256) {
+        if (c->bc.view.nclasses <= 256 && sweepv_fits(c->storage, c->g)) {
             LBM_HIP_CHECK(hipMalloc(reinterpret_cast<void **>(&c->codes8), (size_t)c->g.lx * c->g.pitch), "lbm_set_bc: upload");
             LBM_HIP_CHECK(launch_codes8(c->g, c->bc.view.codes, c->codes8, c->stream), "lbm_set_bc: byte codes");
             c->bc.view.codes8 = c->codes8;
@@ -505,6 +509,35 @@ int lbm_run(lbm_ctx *c, double omega, int64_t nsteps) {
         c->cur ^= 1;
         c->steps += sh.K;
         left -= sh.K;
+    }
+    // The pressure fix reaches K rows to each side of the periodic seam in K
+    // steps.  A lattice that was given no launch setting sweeps K steps at once
+    // as if it had no fix, and puts those 2 K rows right from the same source.
+    // The seam's launch costs 11 us, so it pays from a size on (us a step, one
+    // step per launch / sweep and seam: FP64 2048x2048 107 / 80, 4096x1000 106 /
+    // 61, 1500x1500 58 / 47, 1100x1000 25.9 / 24.5; FP32 2048x2048 48 / 38,
+    // 4096x1000 51 / 39, 1500x1500 25.8 / 24.1, 2048x1024 24.1 / 24.5; FP16
+    // 3000x2048 43 / 39, 2048x2048 31.6 / 30.0, 4096x1000 33 / 34).
+    if (K == 0 && tiles && (c->bc.view.flags & kProgPressure) && c->g.N >= seam_nodes(c->storage)) {
+        BcView walls = c->bc.view;
+        walls.flags &= ~(uint32_t)kProgPressure;
+        const SweepVShape sv = sweepv_shape(c->storage, c->g, walls);
+        const SweepShape sh = sweep_shape(c->storage, c->g.ly);
+        LaunchCfg cfg = c->cfg;
+        const int step = sv.K > 0 ? sv.K
+                         : sweep_supported(c->storage, c->g, walls) && (uint64_t)c->g.lx * sh.ntiles >= 256 ? 2 : 0;
+        for (; step > 0 && left >= step; left -= step) {
+            const int64_t slot = probing ? c->steps - c->probe_base - 1 : -1;
+            LBM_HIP_CHECK(step == 2 ? launch_sweep2(c->storage, c->g, c->st, c->cur, walls, omega, c->probe, slot,
+                                                    probing ? slot + 1 : -1, cfg, c->stream)
+                                    : launch_sweepv(c->storage, sv, c->g, c->st, c->cur, walls, omega, c->probe, slot,
+                                                    c->stream),
+                          "sweep kernel");
+            LBM_HIP_CHECK(launch_seam(c->storage, step, c->g, c->st, c->cur, c->bc.view, omega, c->probe, slot, c->stream),
+                          "seam kernel");
+            c->cur ^= 1;
+            c->steps += step;
+        }
     }
     // Full rows of two (FP32) or one (FP64) column per thread: three steps per
     // launch with adjacent columns per lane, under the same conditions.

@@ -2348,6 +2348,7 @@ struct TileParams {
     uint32_t tx, ty;          // output nodes of a tile
     uint32_t hx, hy;          // halo on each side
     uint32_t offx, offy;      // multiples of lx, ly at least hx, hy, less hx, hy
+    uint32_t x_first, nx;     // the output rows: nx from x_first on, periodic
     uint32_t tiles_y;         // tiles along y
     uint32_t copies;          // times a row can appear in a tile's region
 };
@@ -2377,10 +2378,10 @@ __global__ __launch_bounds__(tile_threads(sizeof(S), kPressure)) void k_tile(Til
     const bool active = threadIdx.x < nodes;
     const uint32_t t = min(threadIdx.x, nodes - 1);
     const uint32_t i = t / ry, j = t - i * ry;
-    const uint32_t ux = x0 + i + p.offx;
+    const uint32_t ux = p.x_first + x0 + i + p.offx;
     const uint32_t x = ux % lx, y = (y0 + j + p.offy) % ly;
-    const uint32_t copy = ux / lx - (x0 + p.offx) / lx;
-    const bool owned = active && i >= p.hx && j >= p.hy && i - p.hx < min(p.tx, lx - x0) && j - p.hy < min(p.ty, ly - y0);
+    const uint32_t copy = ux / lx - (p.x_first + x0 + p.offx) / lx;
+    const bool owned = active && i >= p.hx && j >= p.hy && i - p.hx < min(p.tx, p.nx - x0) && j - p.hy < min(p.ty, ly - y0);
     const bool has_bc = p.bc.codes != nullptr;
     const TileLds<S> L(nodes, ry, p.copies, has_bc ? p.bc.nclasses : 0);
     S *ex = reinterpret_cast<S *>(smem);
@@ -3497,18 +3498,32 @@ int sweepk_rows(const Geom &g, int rows, int K) {
 // halo rows) and a narrower one's does not; column tiles with halos lost too
 // (FP64 4200x1800 142 / 118).  With two steps it lost everywhere (FP32
 // 8192x2048 130).
+namespace {
+// One block a CU, in the fewest rounds.
+uint32_t sweepv_rows(const Geom &g) {
+    const uint32_t slots = 256, rounds = (g.lx + slots * kSweepMaxRows - 1) / (slots * kSweepMaxRows);
+    return (g.lx + rounds * slots - 1) / (rounds * slots);
+}
+uint32_t sweepv_waves(int storage, const Geom &g) {
+    const uint32_t cols = 64 * (storage == LBM_STORE_F64 ? 2 : 4);
+    return (g.ly + cols - 1) / cols;
+}
+}  // namespace
+
+bool sweepv_fits(int storage, const Geom &g) {
+    if (storage == LBM_STORE_F16 || sweep_big(storage, g)) return false;
+    const uint32_t waves = sweepv_waves(storage, g);
+    return waves >= 7 && waves <= 8 && sweepv_rows(g) >= 12;
+}
+
 SweepVShape sweepv_shape(int storage, const Geom &g, const BcView &bc) {
     SweepVShape sh;
-    if (storage == LBM_STORE_F16 || (bc.flags & kProgPressure) || sweep_big(storage, g)) return sh;
-    const bool f64 = storage == LBM_STORE_F64;
-    const uint32_t ncls = bc.chunk ? bc.nclasses : 0, V = f64 ? 2 : 4;
+    const uint32_t ncls = bc.chunk ? bc.nclasses : 0;
+    if (!sweepv_fits(storage, g) || (bc.flags & kProgPressure)) return sh;
     if (ncls > kSweepMaxClasses || (ncls && !bc.codes8)) return sh;
-    const uint32_t waves = (g.ly + 64 * V - 1) / (64 * V);
-    if (waves < 7 || waves > 8) return sh;
-    // one block a CU, in the fewest rounds
-    const uint32_t slots = 256, rounds = (g.lx + slots * kSweepMaxRows - 1) / (slots * kSweepMaxRows);
-    sh.rows = (g.lx + rounds * slots - 1) / (rounds * slots);
-    if (sh.rows < 12) return sh;
+    const bool f64 = storage == LBM_STORE_F64;
+    const uint32_t V = f64 ? 2 : 4, waves = sweepv_waves(storage, g);
+    sh.rows = sweepv_rows(g);
     const bool outlet = ncls && (bc.flags & kProgOutlet);
     sh.threads = 64 * waves;
     sh.lds = f64 ? sweepv_lds<double, kSweepVSteps>(sh.threads * V, waves, ncls, outlet, sh.rows).total
@@ -3606,7 +3621,7 @@ TileShape tile_shape(int storage, const Geom &g, const BcView &bc) {
 namespace {
 template <class S>
 hipError_t tile_typed(const TileShape &sh, const Geom &g, const StateView &st, int src, const BcView &bc, double omega,
-                      const ProbeView &pr, int64_t slot, hipStream_t s) {
+                      const ProbeView &pr, int64_t slot, uint32_t x_first, uint32_t nx, hipStream_t s) {
     using C = typename Io<S>::C;
     TileParams<S> p;
     p.src = static_cast<const S *>(st.plane[src]);
@@ -3628,6 +3643,8 @@ hipError_t tile_typed(const TileShape &sh, const Geom &g, const StateView &st, i
     p.hy = sh.K - 1;
     p.offx = (p.hx + g.lx - 1) / g.lx * g.lx - p.hx;
     p.offy = (p.hy + g.ly - 1) / g.ly * g.ly - p.hy;
+    p.x_first = x_first;
+    p.nx = nx;
     p.tiles_y = (g.ly + p.ty - 1) / p.ty;
     const uint32_t rx = p.tx + 2 * p.hx, ry = p.ty + 2 * p.hy;
     p.copies = (rx + g.lx - 1) / g.lx + 1;
@@ -3635,7 +3652,7 @@ hipError_t tile_typed(const TileShape &sh, const Geom &g, const StateView &st, i
     const size_t lds = TileLds<S>((uint32_t)nodes, ry, p.copies, bc.codes ? bc.nclasses : 0).total;
     if (sh.K < 1 || p.tx < 1 || p.ty < 1 || nodes > 1024 || lds > kLdsLimit) return hipErrorInvalidValue;
     if ((bc.flags & kProgPressure) && (uint32_t)sh.K + 4 > g.lx) return hipErrorInvalidValue;
-    const unsigned grid = (g.lx + p.tx - 1) / p.tx * p.tiles_y;
+    const unsigned grid = (nx + p.tx - 1) / p.tx * p.tiles_y;
     const unsigned threads = ((unsigned)nodes + 63) / 64 * 64;
     const bool pressure = (bc.flags & kProgPressure) != 0;
     if (nodes > (uint64_t)tile_threads(sizeof(S), pressure)) return hipErrorInvalidValue;
@@ -3649,14 +3666,34 @@ hipError_t tile_typed(const TileShape &sh, const Geom &g, const StateView &st, i
 }
 }  // namespace
 
-hipError_t launch_tile(int storage, const TileShape &sh, const Geom &g, const StateView &st, int src, const BcView &bc,
-                       double omega, const ProbeView &pr, int64_t slot, hipStream_t s) {
+namespace {
+hipError_t tile_rows(int storage, const TileShape &sh, const Geom &g, const StateView &st, int src, const BcView &bc,
+                     double omega, const ProbeView &pr, int64_t slot, uint32_t x_first, uint32_t nx, hipStream_t s) {
     switch (storage) {
-        case LBM_STORE_F64: return tile_typed<double>(sh, g, st, src, bc, omega, pr, slot, s);
-        case LBM_STORE_F32: return tile_typed<float>(sh, g, st, src, bc, omega, pr, slot, s);
-        case LBM_STORE_F16: return tile_typed<__half>(sh, g, st, src, bc, omega, pr, slot, s);
+        case LBM_STORE_F64: return tile_typed<double>(sh, g, st, src, bc, omega, pr, slot, x_first, nx, s);
+        case LBM_STORE_F32: return tile_typed<float>(sh, g, st, src, bc, omega, pr, slot, x_first, nx, s);
+        case LBM_STORE_F16: return tile_typed<__half>(sh, g, st, src, bc, omega, pr, slot, x_first, nx, s);
     }
     return hipErrorInvalidValue;
+}
+}  // namespace
+
+hipError_t launch_tile(int storage, const TileShape &sh, const Geom &g, const StateView &st, int src, const BcView &bc,
+                       double omega, const ProbeView &pr, int64_t slot, hipStream_t s) {
+    return tile_rows(storage, sh, g, st, src, bc, omega, pr, slot, 0, g.lx, s);
+}
+
+hipError_t launch_seam(int storage, int K, const Geom &g, const StateView &st, int src, const BcView &bc, double omega,
+                       const ProbeView &pr, int64_t slot, hipStream_t s) {
+    TileShape sh;
+    sh.K = K;
+    sh.tx = 2 * K;
+    if (K < 1 || g.lx < (uint32_t)(2 * K)) return hipErrorInvalidValue;
+    const size_t elem = storage == LBM_STORE_F64 ? 8 : (storage == LBM_STORE_F32 ? 4 : 2);
+    const uint32_t ry = (uint32_t)tile_threads(elem, true) / (2 * K + 2 * (K + 1));
+    // narrow tiles: one wave a SIMD and the whole GPU, since nothing runs beside
+    sh.ty = std::min(std::min(g.ly, ry - 2 * (K - 1)), std::max(8u, (g.ly + 255) / 256));
+    return tile_rows(storage, sh, g, st, src, bc, omega, pr, slot, g.lx - K, 2 * K, s);
 }
 
 hipError_t launch_sweepk(int storage, int K, const Geom &g, const StateView &st, int src, const BcView &bc,

@@ -60,6 +60,8 @@ hipError_t launch_codes8(const Geom &g, const uint16_t *codes, uint8_t *codes8, 
 // fix, at most 128 classes, state buffers below 4 GiB): the shape, K = 0 where it
 // does not apply or another kernel is faster.  Probe slots as launch_sweepk.
 SweepVShape sweepv_shape(int storage, const Geom &g, const BcView &bc);
+// Whether the lattice's size is one it takes (its boundary tables then need codes8).
+bool sweepv_fits(int storage, const Geom &g);
 hipError_t launch_sweepv(int storage, const SweepVShape &sh, const Geom &g, const StateView &st, int src, const BcView &bc,
                          double omega, const ProbeView &pr, int64_t probe_slot, hipStream_t s);
 // K steps in one launch on tiles held in registers and LDS (small lattices).
@@ -69,6 +71,11 @@ hipError_t launch_sweepv(int storage, const SweepVShape &sh, const Geom &g, cons
 TileShape tile_shape(int storage, const Geom &g, const BcView &bc);
 hipError_t launch_tile(int storage, const TileShape &sh, const Geom &g, const StateView &st, int src, const BcView &bc,
                        double omega, const ProbeView &pr, int64_t probe_slot, hipStream_t s);
+// K steps of the rows that the pressure fix reaches in them, lx - K to K - 1
+// across the periodic seam: run after a K-step sweep of the whole lattice
+// without the fix, from the same source, it puts those rows right.
+hipError_t launch_seam(int storage, int K, const Geom &g, const StateView &st, int src, const BcView &bc, double omega,
+                       const ProbeView &pr, int64_t probe_slot, hipStream_t s);
 // Rows per block of the K-step kernel: `rows`, raised until every block
 // (the last one included) holds at least K - 1 rows.
 int sweepk_rows(const Geom &g, int rows, int K);

@@ -109,3 +109,33 @@ def test_many_classes(walls):
         lat.close()
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("storage,lx,ly,kind", [("f64", 1030, 1030, "poiseuille"), ("f64", 1040, 1040, "poiseuille_y"),
+                                                ("f64", 2830, 1000, "poiseuille"), ("f64", 300, 4000, "poiseuille"),
+                                                ("f32", 2820, 1700, "poiseuille"), ("f32", 2000, 1700, "poiseuille"),
+                                                ("f32", 1800, 1800, "poiseuille_y"), ("f16", 2050, 2048, "poiseuille")])
+@pytest.mark.parametrize("at", [(0, 0), (-2, -1), (2, 5)])
+def test_pressure_fix_beside_sweeps(storage, lx, ly, kind, at):
+    """the rows the fix reaches are put right after a sweep without it; probes in and beside them"""
+    import torch
+
+    rng = np.random.default_rng(lx + ly)
+    rho = torch.from_numpy(1 + 0.02 * rng.random((lx, ly))).cuda()
+    u = torch.from_numpy(0.03 * rng.standard_normal((lx, ly, 2))).cuda()
+    outs = []
+    for temporal in (None, 1):
+        lat = Lattice(lx, ly, boundary=_boundary(kind, lx, ly), storage=storage)
+        if temporal:
+            lat.set_temporal(temporal)
+        lat.set_probe(at[0] % lx, at[1] % ly, 20)
+        lat.set_equilibrium(rho, u)
+        for n in (1, 6, 5):
+            lat.run(1.3, n)
+        out = [torch.empty(s, dtype=torch.float64, device="cuda") for s in ((lx, ly, 9), (lx, ly), (lx, ly, 2))]
+        lat.state_into(*out)
+        outs.append((out, lat.probe(20)))
+        lat.close()
+    for a, b in zip(outs[0][0], outs[1][0]):
+        assert torch.equal(a, b)
+    assert np.array_equal(outs[0][1], outs[1][1])
