@@ -304,10 +304,12 @@ int lbm_collide(const void *f, const void *rho, const void *u, double omega, voi
  * prog NULL = fully periodic.  The outputs overlap no input. */
 int lbm_step(const lbm_bc_prog *prog, const double *f, const double *rho, const double *u, double omega,
              int nx, int ny, double *f_out, double *rho_out, double *u_out, void *stream);
-/* The same on host arrays, through `work` (device memory, 24*nx*ny doubles).
- * Synchronous. */
+/* The same on host arrays, through `work` (device memory, 24*nx*ny doubles)
+ * and `stage` (pinned host memory, stage_bytes of it: a multiple of 256, at
+ * least 1024; a few MB are enough for any lattice).  Synchronous. */
 int lbm_step_host(const lbm_bc_prog *prog, const double *f, const double *rho, const double *u, double omega,
-                  int nx, int ny, double *f_out, double *rho_out, double *u_out, double *work, void *stream);
+                  int nx, int ny, double *f_out, double *rho_out, double *u_out, double *work, void *stage,
+                  int64_t stage_bytes, void *stream);
 /* Post-streaming boundary rules of a program applied in place to f_post
  * (the closures of boundary_conditions.py:93-111, 138-165, 192-212, 239-252,
  * 267-281).  f_prev is read only if the program has an outlet. FP64 only. */

@@ -13,13 +13,22 @@ import numpy as np
 from . import _lib
 
 
+_torch = None      # the torch module, once a HIP device has been seen
+_raw_stream = None  # device index -> its current stream's handle
+
+
 def torch_cuda():
     """The torch module, after checking that a HIP device is visible."""
-    import torch
+    global _torch, _raw_stream
+    if _torch is None:
+        import torch
 
-    if not torch.cuda.is_available():
-        raise RuntimeError("no HIP device is visible: the lattice-Boltzmann kernels have no CPU fallback")
-    return torch
+        if not torch.cuda.is_available():
+            raise RuntimeError("no HIP device is visible: the lattice-Boltzmann kernels have no CPU fallback")
+        # the handle alone, without a Stream object around it, where torch has it
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        _torch = torch
+    return _torch
 
 
 def to_device(a, dtype=None):
@@ -55,7 +64,10 @@ def dtype_code(t) -> int:
 
 
 def stream() -> int:
-    return torch_cuda().cuda.current_stream().cuda_stream
+    torch = torch_cuda()
+    if _raw_stream is not None:
+        return _raw_stream(torch.cuda.current_device())
+    return torch.cuda.current_stream().cuda_stream
 
 
 def write_back(dst, t) -> None:

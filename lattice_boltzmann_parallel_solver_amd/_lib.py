@@ -109,7 +109,7 @@ _SIGNATURES = {
     "lbm_velocity": (_I, [_P, _P, _P, _I64, _I, _P]),
     "lbm_collide": (_I, [_P, _P, _P, _D, _P, _I64, _I, _P]),
     "lbm_step": (_I, [_P, _P, _P, _P, _D, _I, _I, _P, _P, _P, _P]),
-    "lbm_step_host": (_I, [_P, _P, _P, _P, _D, _I, _I, _P, _P, _P, _P, _P]),
+    "lbm_step_host": (_I, [_P, _P, _P, _P, _D, _I, _I, _P, _P, _P, _P, _P, _I64, _P]),
     "lbm_bc_apply": (_I, [_P, _P, _P, _P, _P]),
     "lbm_bc_pressure": (_I, [_P, _P, _P, _P, _P]),
     "lbm_moments_sum_noalloc": (_I, [_P, _I64, _P, _P]),
@@ -125,6 +125,8 @@ _lock = threading.Lock()
 def load():
     """Load liblbm_hip.so (raises if it has not been built)."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is None:
             if not os.path.exists(LIB_PATH):

@@ -135,6 +135,9 @@ def lattice_boltzmann_step(f, density, velocity, omega: float,
     ins = [np.ascontiguousarray(a, dtype=np.float64) for a in (f, density, velocity)]
     outs = tuple(np.empty(a.shape) for a in ins)
     work = torch.empty(24 * lx * ly, dtype=torch.float64, device="cuda")
+    # four pinned quarters of 64 KiB to 2 MiB (torch keeps and hands them out again)
+    stage = torch.empty(4 * min(2 << 20, max(1 << 16, -(-96 * lx * ly // 2048) * 256)), dtype=torch.uint8, pin_memory=True)
     check(_lib.load().lbm_step_host(handle, *(a.ctypes.data for a in ins), float(omega), lx, ly,
-                                    *(a.ctypes.data for a in outs), work.data_ptr(), stream()))
+                                    *(a.ctypes.data for a in outs), work.data_ptr(), stage.data_ptr(), stage.numel(),
+                                    stream()))
     return outs
