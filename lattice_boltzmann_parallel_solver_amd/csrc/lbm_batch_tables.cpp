@@ -149,6 +149,13 @@ int batch_group_rows(int threads, int k, int base_rows, bool rows_auto, int64_t 
     return rows;
 }
 
+int batch_spread_rows(int rows, int threads, int k, bool f64, int64_t rows_total, int cus) {
+    const int per_cu = k == 3 ? 6 : (threads >= 512 ? 8 : 16) / (f64 ? 2 : 1);
+    const int64_t spread = rows_total / ((int64_t)per_cu * std::max(cus, 1));
+    if (4 * spread >= 3 * (int64_t)rows) return rows;  // too little to gain for another split
+    return (int)std::min<int64_t>(rows, std::max<int64_t>(2, spread));
+}
+
 bool batch_three_steps_fill(int64_t rows_total, int cus) { return rows_total / (4 * (int64_t)std::max(cus, 1)) >= 8; }
 
 }  // namespace lbm

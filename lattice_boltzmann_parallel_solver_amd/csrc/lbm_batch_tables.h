@@ -89,6 +89,16 @@ int pick_wide_rows(const std::vector<WideLattice> &lattices, int cus, int max_ro
 // batch's rows_total rows about four blocks per CU (two for wide rows).
 int batch_group_rows(int threads, int k, int base_rows, bool rows_auto, int64_t rows_total, int cus, int wide_rows);
 
+// Fewer rows per block for batches of a few dozen lattices, whose groups run
+// side by side and each end with their slowest block: no more rows than leave
+// the whole batch 16 blocks a CU (8 of 512 threads or more, half of both in
+// FP64; 6 of three steps), but 2.  120 steps of seeded channels, FP32, two / three
+// steps per launch, ms before -> after: 20 channels 7.4 -> 6.2 / 6.8 -> 6.0 (another
+// draw 9.9 -> 8.0 / 10.0 -> 8.2), 12 7.1 -> 4.3 / 6.6 -> 4.7, 8 4.9 -> 3.2; FP64 20
+// channels 15.0 -> 13.9, 10 8.3 -> 7.6 (and 10.4 at the FP32 counts).  At twice
+// as many blocks FP32 lost again (7.5 / 7.1).  Large batches keep their counts.
+int batch_spread_rows(int rows, int threads, int k, bool f64, int64_t rows_total, int cus);
+
 // With automatic rows, three steps per launch only where the batch's rows
 // make at least 8 per block at four blocks per CU.
 bool batch_three_steps_fill(int64_t rows_total, int cus);

@@ -1163,6 +1163,9 @@ int batch_run_sweep(lbm_batch *b, int64_t nsteps) {
             LaunchCfg cfg = c->cfg;
             cfg.sweep_rows =
                 batch_group_rows((int)bk.threads, bk.k, b->sweep_rows, b->rows_auto, rows_total, cus, wide_rows);
+            if (b->rows_auto && !(bk.k == 2 && bk.threads >= 512 && wide_rows > 0))
+                cfg.sweep_rows = batch_spread_rows(cfg.sweep_rows, (int)bk.threads, bk.k, b->storage == LBM_STORE_F64,
+                                                   rows_total, cus);
             uint32_t rows = (uint32_t)sweep_rows_for(c->g, cfg, 0);
             // the three-step kernel needs two rows in every block; the same
             // tables also serve its two-step launches
