@@ -129,6 +129,7 @@ struct lbm_ctx {
     // tiling of the tile kernel, worked out by the first run that may take it
     TileShape tile;
     bool tile_ready = false;
+    bool stage_eq = false;  // pending: stage_f is the equilibrium of stage_rho and stage_u
 };
 
 namespace {
@@ -178,6 +179,16 @@ int check_ctx(lbm_ctx *c, const char *fn) {
     }
     LBM_HIP_CHECK(hipSetDevice(c->device), fn);
     return LBM_OK;
+}
+
+// Whether p is device memory of `device` (a kernel there can read it in place).
+bool in_memory_of(int device, const void *p) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type == hipMemoryTypeDevice && a.device == device;
 }
 
 hipMemcpyKind kind_in(int where) { return where == LBM_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice; }
@@ -390,6 +401,7 @@ int lbm_set_bc(lbm_ctx *c, const lbm_bc_prog *prog) {
         rc = finalize_into(c, c->stage_f, c->stage_rho, c->stage_u);
         if (rc) return rc;
         c->phase = kPending;
+        c->stage_eq = false;
     }
     LBM_HIP_CHECK(hipStreamSynchronize(c->stream), "lbm_set_bc");
     (void)hipFree(c->bc.mem);
@@ -416,6 +428,7 @@ int lbm_set_state(lbm_ctx *c, const double *f, const double *rho, const double *
         return LBM_ERR_ARG;
     }
     const size_t N = c->g.N;
+    c->stage_eq = false;
     LBM_HIP_CHECK(hipMemcpyAsync(c->stage_f, f, 9 * N * sizeof(double), kind_in(where), c->stream), "lbm_set_state");
     LBM_HIP_CHECK(hipMemcpyAsync(c->stage_rho, rho, N * sizeof(double), kind_in(where), c->stream), "lbm_set_state");
     LBM_HIP_CHECK(hipMemcpyAsync(c->stage_u, u, 2 * N * sizeof(double), kind_in(where), c->stream), "lbm_set_state");
@@ -434,14 +447,25 @@ int lbm_set_state_equilibrium(lbm_ctx *c, const double *rho, const double *u, in
         return LBM_ERR_ARG;
     }
     const size_t N = c->g.N;
-    LBM_HIP_CHECK(hipMemcpyAsync(c->stage_rho, rho, N * sizeof(double), kind_in(where), c->stream),
-                  "lbm_set_state_equilibrium");
-    LBM_HIP_CHECK(hipMemcpyAsync(c->stage_u, u, 2 * N * sizeof(double), kind_in(where), c->stream),
-                  "lbm_set_state_equilibrium");
-    LBM_HIP_CHECK(launch_equilibrium_aos(c->stage_rho, c->stage_u, c->stage_f, (int64_t)N, LBM_DT_F64, c->stream),
+    c->stage_eq = false;
+    const double *src_rho = rho, *src_u = u;
+    // arrays in this device's memory are copied by the kernel that reads them
+    const bool here = where == LBM_DEVICE && in_memory_of(c->device, rho) && in_memory_of(c->device, u);
+    if (!here) {
+        LBM_HIP_CHECK(hipMemcpyAsync(c->stage_rho, rho, N * sizeof(double), kind_in(where), c->stream),
+                      "lbm_set_state_equilibrium");
+        LBM_HIP_CHECK(hipMemcpyAsync(c->stage_u, u, 2 * N * sizeof(double), kind_in(where), c->stream),
+                      "lbm_set_state_equilibrium");
+        src_rho = c->stage_rho;
+        src_u = c->stage_u;
+    }
+    LBM_HIP_CHECK(here ? launch_load_equilibrium(src_rho, src_u, c->stage_f, c->stage_rho, c->stage_u,
+                                                                (int64_t)N, c->stream)
+                                      : launch_equilibrium_aos(src_rho, src_u, c->stage_f, (int64_t)N, LBM_DT_F64, c->stream),
                   "equilibrium kernel");
     LBM_HIP_CHECK(hipStreamSynchronize(c->stream), "lbm_set_state_equilibrium");
     c->phase = kPending;
+    c->stage_eq = true;
     c->steps = 0;
     c->probe_base = 0;
     return LBM_OK;
@@ -484,7 +508,7 @@ int lbm_run(lbm_ctx *c, double omega, int64_t nsteps) {
     int64_t left = nsteps;
     if (c->phase == kPending) {
         LBM_HIP_CHECK(launch_collide_first(c->storage, c->g, c->stage_f, c->stage_rho, c->stage_u, c->st, c->cur,
-                                           c->bc.view, omega, c->stream),
+                                           c->bc.view, omega, c->stage_eq, c->stream),
                       "first-collision kernel");
         c->phase = kRunning;
         c->steps++;
@@ -564,9 +588,11 @@ int lbm_run(lbm_ctx *c, double omega, int64_t nsteps) {
         }
     }
     if (K >= 2 && sweep_supported(c->storage, c->g, c->bc.view, c->cfg.sweep_tile, c->cfg.sweep_v)) {
-        // A long run moves the state into the range-interleaved row order of
-        // the sweep's row ranges (the rows all blocks touch at once become
-        // neighbours in memory) and back at its end: two copies of the state.
+        // A long run keeps the state in the range-interleaved row order of the
+        // sweep's row ranges (the rows all blocks touch at once become
+        // neighbours in memory): its first launch reads the plain order and
+        // writes that one, its last the other way round (two separate copies
+        // of the state cost 410 us a run at 4200 x 1800 FP64).
         // Measured where it pays: FP32 rows of two columns per thread and FP64
         // column tiles, with 16 or more rows per block and at most two rounds
         // of resident row ranges (8192 x 2048 FP32 137.3 -> 147.4 GLUPS, FP64
@@ -585,11 +611,7 @@ int lbm_run(lbm_ctx *c, double omega, int64_t nsteps) {
             const int resident = sweep2_resident_ranges(c->storage, c->g, c->bc.view, cfg);
             if (rows >= kInterleaveMinRows && rows <= (int)kRowLayoutMaxRows && rows < (int)c->g.lx &&
                 resident > 0 && ranges <= 2 * (int64_t)resident) {
-                LBM_HIP_CHECK(launch_row_layout(c->storage, c->g, c->st, c->cur, (uint32_t)rows, true, c->stream),
-                              "row order kernel");
-                c->cur ^= 1;
                 cfg.sweep_rows = rows;
-                cfg.sweep_il = 1;
                 ilv = true;
             }
         }
@@ -597,15 +619,17 @@ int lbm_run(lbm_ctx *c, double omega, int64_t nsteps) {
         for (; left >= 2; left -= 2) {
             // materialises f_{steps} and f_{steps+1}
             const int64_t slot = probing ? c->steps - c->probe_base - 1 : -1;
+            cfg.sweep_il_src = cfg.sweep_il_dst;
+            cfg.sweep_il_dst = ilv && left >= 4;
             e = launch_sweep2(c->storage, c->g, c->st, c->cur, c->bc.view, omega, c->probe, slot,
                               probing ? slot + 1 : -1, cfg, c->stream);
             if (e != hipSuccess) break;
             c->cur ^= 1;
             c->steps += 2;
         }
-        // back to the plain order, also after a failed launch (the state then
-        // holds the steps done so far)
-        if (ilv) {
+        // after a failed launch the state, with the steps done so far, may still
+        // be in the other order (what the failed launch would have read)
+        if (e != hipSuccess && cfg.sweep_il_src) {
             const hipError_t eb = launch_row_layout(c->storage, c->g, c->st, c->cur, (uint32_t)cfg.sweep_rows, false,
                                                     c->stream);
             if (eb == hipSuccess) c->cur ^= 1;
@@ -880,6 +904,7 @@ int lbm_checkpoint_load(lbm_ctx *c, const void *host, int64_t bytes) {
         LBM_HIP_CHECK(hipMemcpyAsync(c->st.side[0], src + pb, sb, hipMemcpyHostToDevice, c->stream), "lbm_checkpoint_load");
         c->cur = 0;
     } else {
+        c->stage_eq = false;
         LBM_HIP_CHECK(hipMemcpyAsync(c->stage_f, src, 9 * N * sizeof(double), hipMemcpyHostToDevice, c->stream), "lbm_checkpoint_load");
         LBM_HIP_CHECK(hipMemcpyAsync(c->stage_rho, src + 9 * N * sizeof(double), N * sizeof(double), hipMemcpyHostToDevice, c->stream), "lbm_checkpoint_load");
         LBM_HIP_CHECK(hipMemcpyAsync(c->stage_u, src + 10 * N * sizeof(double), 2 * N * sizeof(double), hipMemcpyHostToDevice, c->stream), "lbm_checkpoint_load");
@@ -1638,7 +1663,7 @@ int batch_run_body(lbm_batch *b, int64_t nsteps) {
             lbm_ctx *c = b->ctxs[j];
             if (c->phase == kPending) {
                 LBM_HIP_CHECK(launch_collide_first(c->storage, c->g, c->stage_f, c->stage_rho, c->stage_u, c->st,
-                                                   c->cur, c->bc.view, b->omegas[j], b->stream),
+                                                   c->cur, c->bc.view, b->omegas[j], c->stage_eq, b->stream),
                               "lbm_batch_run: first collision");
                 c->phase = kRunning;
             } else {

@@ -800,7 +800,7 @@ struct SweepParams {
     int nt;
     int xcd;         // XCD-aware block order (neighbouring row ranges share an L2)
     S *scratch;      // 9 V blockDim.x values, written and never read
-    RowLayout il;    // row order of src and dst (rows = 0: plain)
+    RowLayout il, ild;  // row orders of src and of dst (rows = 0: plain)
 };
 
 template <class S>
@@ -1142,7 +1142,7 @@ __device__ __forceinline__ void sweep_block(const SweepParams<S> &p, uint32_t xa
             if constexpr (kS2) {
                 // step 2 on row r = x - 1 (stored at slot sr2)
                 const uint32_t r = row_at(it - 1);
-                const uint32_t sr2 = row_slot(p.il, r);
+                const uint32_t sr2 = row_slot(p.ild, r);
                 C v2[9];
                 v2[0] = B[k][0];
                 v2[2] = B[k][1];
@@ -1304,6 +1304,7 @@ __global__ __launch_bounds__(kSweepThreads, sizeof(S) < 8 && V == 1 && !kBig ? 8
         p.il.ranges = j.il_ranges;
         p.il.whole = j.il_whole;
         p.il.magic = j.il_magic;
+        p.ild = p.il;
     }
     sweep_block<S, V, true, false, kBig>(p, (blk - j.block0) * j.rows, 0, SweepLanes{threadIdx.x, blockDim.x, smem, 0});
 }
@@ -2542,7 +2543,9 @@ __device__ __forceinline__ void store_records(T *out, uint32_t cnt, const T v[9]
 // ---------------------------------------------------------------------------
 // first collision (from the AoS FP64 step input)
 // ---------------------------------------------------------------------------
-template <class S>
+// kEq: f holds the equilibrium of (rho, u), so it is computed and not read
+// (8192x2048 FP32: 410 -> 190 us).
+template <class S, bool kEq>
 __global__ __launch_bounds__(kBlock) void k_collide_first(const double *__restrict__ f,
                                                           const double *__restrict__ rho,
                                                           const double *__restrict__ u, S *__restrict__ dst,
@@ -2553,10 +2556,16 @@ __global__ __launch_bounds__(kBlock) void k_collide_first(const double *__restri
     if (n >= g.N) return;
     const uint32_t x = row_of(g, n), y = n - x * g.ly;
     double fi[9], e[9], s[9];
-#pragma unroll
-    for (int i = 0; i < 9; i++) fi[i] = f[(size_t)n * 9 + i];
     const double r = rho[n], ux = u[2 * (size_t)n], uy = u[2 * (size_t)n + 1];
+    if constexpr (!kEq) {
+#pragma unroll
+        for (int i = 0; i < 9; i++) fi[i] = f[(size_t)n * 9 + i];
+    }
     feq_f64(r, ux, uy, e);
+    if constexpr (kEq) {
+#pragma unroll
+        for (int i = 0; i < 9; i++) fi[i] = e[i];
+    }
 #pragma unroll
     for (int i = 0; i < 9; i++) s[i] = fi[i] + (e[i] - fi[i]) * omega;
     const uint32_t flags = bc.codes ? bc.classes[bc.codes[n]].flags : 0;
@@ -2942,15 +2951,23 @@ __global__ __launch_bounds__(kBlock, 3) void k_step_aos(StepAosParams p) {
     for (uint32_t it = 2; it < R + 2; it++) body(it, Flag<true>{});
 }
 
+// rho_out, u_out: where the moments are also copied to, or null.
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_equilibrium_aos(const T *__restrict__ rho, const T *__restrict__ u,
-                                                            T *__restrict__ feq, int64_t n) {
+                                                            T *__restrict__ feq, int64_t n, T *__restrict__ rho_out,
+                                                            T *__restrict__ u_out) {
     __shared__ __align__(16) T rec[kBlock / 64][kRecLds];
     const int64_t w0 = (int64_t)blockIdx.x * kBlock + (threadIdx.x & ~63u);
     if (w0 >= n) return;
     const int64_t c = min(w0 + (threadIdx.x & 63), n - 1);
+    const T r = rho[c], ux = u[2 * c], uy = u[2 * c + 1];
+    if (rho_out && w0 + (threadIdx.x & 63) < n) {
+        rho_out[c] = r;
+        u_out[2 * c] = ux;
+        u_out[2 * c + 1] = uy;
+    }
     T e[9];
-    feq_t<T>(rho[c], u[2 * c], u[2 * c + 1], e);
+    feq_t<T>(r, ux, uy, e);
     store_records(feq + w0 * 9, (uint32_t)min((int64_t)64, n - w0), e, rec[threadIdx.x >> 6]);
 }
 
@@ -3221,10 +3238,12 @@ hipError_t sweep_typed(const Geom &g, const StateView &st, int src, const BcView
     if (V != 1 && V != V2) return hipErrorInvalidValue;
     auto pick = [&](bool probe) { return V == 1 ? sweep_fn<S, 1>(probe, tiled, big) : sweep_fn<S, V2>(probe, tiled, big); };
     p.rows = sweep_rows_typed<S>(g, bc, cfg);
-    // the buffers in the range-interleaved order of exactly these row ranges
-    if (cfg.sweep_il) {
-        p.il = row_layout(g.lx, p.rows);
-        if (p.il.rows != p.rows) return hipErrorInvalidValue;
+    // buffers in the range-interleaved order of exactly these row ranges
+    if (cfg.sweep_il_src || cfg.sweep_il_dst) {
+        const RowLayout il = row_layout(g.lx, p.rows);
+        if (il.rows != p.rows) return hipErrorInvalidValue;
+        if (cfg.sweep_il_src) p.il = il;
+        if (cfg.sweep_il_dst) p.ild = il;
     }
     const unsigned grid = (g.lx + p.rows - 1) / p.rows * sh.ntiles;
     const size_t lds = sweep_lds_layout<S>(sh.lw, bc.chunk ? bc.nclasses : 0, p.rows).total;
@@ -3936,25 +3955,26 @@ hipError_t launch_speed(const double *u, double *out, int64_t n, hipStream_t s) 
     return hipGetLastError();
 }
 
+namespace {
+template <class S>
+void collide_first(const Geom &g, const double *f, const double *rho, const double *u, const StateView &st, int dst,
+                   const BcView &bc, double omega, bool equilibrium, hipStream_t s) {
+    const void *fn = equilibrium ? reinterpret_cast<const void *>(k_collide_first<S, true>)
+                                 : reinterpret_cast<const void *>(k_collide_first<S, false>);
+    S *plane = static_cast<S *>(st.plane[dst]);
+    auto *side = static_cast<typename Io<S>::C *>(st.side[dst]);
+    void *args[] = {&f, &rho, &u, &plane, &side, const_cast<Geom *>(&g), const_cast<BcView *>(&bc), &omega};
+    (void)hipLaunchKernel(fn, dim3(grid_for(g.N)), dim3(kBlock), args, 0, s);
+}
+}  // namespace
+
 hipError_t launch_collide_first(int storage, const Geom &g, const double *f, const double *rho, const double *u,
-                                const StateView &st, int dst, const BcView &bc, double omega, hipStream_t s) {
-    const unsigned grid = grid_for(g.N);
+                                const StateView &st, int dst, const BcView &bc, double omega, bool equilibrium,
+                                hipStream_t s) {
     switch (storage) {
-        case LBM_STORE_F64:
-            hipLaunchKernelGGL(k_collide_first<double>, dim3(grid), dim3(kBlock), 0, s, f, rho, u,
-                               static_cast<double *>(st.plane[dst]), static_cast<double *>(st.side[dst]), g, bc,
-                               omega);
-            break;
-        case LBM_STORE_F32:
-            hipLaunchKernelGGL(k_collide_first<float>, dim3(grid), dim3(kBlock), 0, s, f, rho, u,
-                               static_cast<float *>(st.plane[dst]), static_cast<float *>(st.side[dst]), g, bc,
-                               omega);
-            break;
-        case LBM_STORE_F16:
-            hipLaunchKernelGGL(k_collide_first<__half>, dim3(grid), dim3(kBlock), 0, s, f, rho, u,
-                               static_cast<__half *>(st.plane[dst]), static_cast<float *>(st.side[dst]), g, bc,
-                               omega);
-            break;
+        case LBM_STORE_F64: collide_first<double>(g, f, rho, u, st, dst, bc, omega, equilibrium, s); break;
+        case LBM_STORE_F32: collide_first<float>(g, f, rho, u, st, dst, bc, omega, equilibrium, s); break;
+        case LBM_STORE_F16: collide_first<__half>(g, f, rho, u, st, dst, bc, omega, equilibrium, s); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -4038,11 +4058,17 @@ hipError_t launch_equilibrium_aos(const void *rho, const void *u, void *feq, int
     if (dtype == LBM_DT_F64)
         hipLaunchKernelGGL(k_equilibrium_aos<double>, dim3(grid_for(n)), dim3(kBlock), 0, s,
                            static_cast<const double *>(rho), static_cast<const double *>(u),
-                           static_cast<double *>(feq), n);
+                           static_cast<double *>(feq), n, (double *)nullptr, (double *)nullptr);
     else
         hipLaunchKernelGGL(k_equilibrium_aos<float>, dim3(grid_for(n)), dim3(kBlock), 0, s,
                            static_cast<const float *>(rho), static_cast<const float *>(u), static_cast<float *>(feq),
-                           n);
+                           n, (float *)nullptr, (float *)nullptr);
+    return hipGetLastError();
+}
+
+hipError_t launch_load_equilibrium(const double *rho, const double *u, double *f, double *rho_out, double *u_out, int64_t n,
+                                   hipStream_t s) {
+    hipLaunchKernelGGL(k_equilibrium_aos<double>, dim3(grid_for(n)), dim3(kBlock), 0, s, rho, u, f, n, rho_out, u_out);
     return hipGetLastError();
 }
 

@@ -34,8 +34,8 @@ int sweep2_rows(int storage, const Geom &g, const BcView &bc, const LaunchCfg &c
 int sweep2_resident_ranges(int storage, const Geom &g, const BcView &bc, const LaunchCfg &cfg);
 // planes[src] -> planes[src^1] and side[src] -> side[src^1], rows moved to
 // (to_ilv) or from their slots in the range-interleaved order of `rows`-row
-// ranges (lbm_rowlayout.h); launch_sweep2 with cfg.sweep_il and cfg.sweep_rows
-// = rows then runs on buffers in that order.
+// ranges (lbm_rowlayout.h); launch_sweep2 with cfg.sweep_rows = rows and
+// cfg.sweep_il_src / sweep_il_dst reads / writes buffers in that order.
 hipError_t launch_row_layout(int storage, const Geom &g, const StateView &st, int src, uint32_t rows, bool to_ilv,
                              hipStream_t s);
 // The sweep kernel needs no pressure fix, at most 128 boundary classes,
@@ -151,9 +151,13 @@ hipError_t launch_copy16(const void *src, void *dst, int64_t n16, hipStream_t s)
 hipError_t launch_add_step(int64_t *step, int64_t k, hipStream_t s);
 
 // First collision from AoS FP64 (f, rho, u) into planes[dst] / side[dst].
+// equilibrium: f holds the equilibrium of (rho, u) and need not be read.
 hipError_t launch_collide_first(int storage, const Geom &g, const double *f, const double *rho,
                                 const double *u, const StateView &st, int dst, const BcView &bc,
-                                double omega, hipStream_t s);
+                                double omega, bool equilibrium, hipStream_t s);
+// f = equilibrium(rho, u) and copies of rho and u, in one pass.
+hipError_t launch_load_equilibrium(const double *rho, const double *u, double *f, double *rho_out, double *u_out, int64_t n,
+                                   hipStream_t s);
 
 // Stream + boundary + moments from planes[src] into AoS FP64 outputs (any may
 // be null); partials != nullptr adds the per-block moment sums.
