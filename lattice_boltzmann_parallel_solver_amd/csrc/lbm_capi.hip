@@ -548,8 +548,9 @@ int lbm_run(lbm_ctx *c, double omega, int64_t nsteps) {
         const SweepVShape sv = sweepv_shape(c->storage, c->g, walls);
         const SweepShape sh = sweep_shape(c->storage, c->g.ly);
         LaunchCfg cfg = c->cfg;
-        const int step = sv.K > 0 ? sv.K
-                         : sweep_supported(c->storage, c->g, walls) && (uint64_t)c->g.lx * sh.ntiles >= 256 ? 2 : 0;
+        int step = sv.K > 0 ? sv.K
+                   : sweep_supported(c->storage, c->g, walls) && (uint64_t)c->g.lx * sh.ntiles >= 256 ? 2 : 0;
+        if (!seam_supported(step, c->g)) step = 0;
         for (; step > 0 && left >= step; left -= step) {
             const int64_t slot = probing ? c->steps - c->probe_base - 1 : -1;
             LBM_HIP_CHECK(step == 2 ? launch_sweep2(c->storage, c->g, c->st, c->cur, walls, omega, c->probe, slot,

@@ -877,6 +877,9 @@ struct Flag {
 // one run of its waves (tid counts from the run's first thread; T threads;
 // its LDS area from smem), and the row iterations every wave of the block
 // runs (packed blocks: the longest range's rows + 2).
+// Instances that can run in the range-interleaved row order.
+constexpr bool sweep_interleaves(size_t elem, int v, bool tiled) { return elem >= 4 && (v == 2 || tiled); }
+
 struct SweepLanes {
     uint32_t tid, T;
     unsigned char *smem;
@@ -931,6 +934,10 @@ __device__ __forceinline__ void sweep_block(const SweepParams<S> &p, uint32_t xa
     auto row_at = [&](uint32_t it) {
         const uint32_t r = xa + it + lx - 1;
         return r >= lx ? (r - lx >= lx ? r - 2 * lx : r - lx) : r;
+    };
+    auto slot_of = [&](const RowLayout &il, uint32_t x) {
+        if constexpr (sweep_interleaves(sizeof(S), V, kTiled)) return row_slot(il, x);
+        else return x;
     };
     if (has_bc) {
         const uint32_t words = p.bc.nclasses * (uint32_t)(sizeof(ClassEntry) / 4);
@@ -1012,7 +1019,7 @@ __device__ __forceinline__ void sweep_block(const SweepParams<S> &p, uint32_t xa
     auto pull_row = [&](uint32_t rr, const uint32_t code[V], C out[V][9], auto k0_tag, auto k1_tag) {
         constexpr int k0 = decltype(k0_tag)::value, k1 = decltype(k1_tag)::value;
         const uint32_t xr = row_at(rr), xm = xr == 0 ? lx - 1 : xr - 1, xp = xr + 1 == lx ? 0 : xr + 1;
-        const uint32_t sr = row_slot(p.il, xr), sm = row_slot(p.il, xm), sp = row_slot(p.il, xp);
+        const uint32_t sr = slot_of(p.il, xr), sm = slot_of(p.il, xm), sp = slot_of(p.il, xp);
 #pragma unroll
         for (int k = k0; k < k1; k++) {
             if (special(rr, k)) {
@@ -1142,7 +1149,7 @@ __device__ __forceinline__ void sweep_block(const SweepParams<S> &p, uint32_t xa
             if constexpr (kS2) {
                 // step 2 on row r = x - 1 (stored at slot sr2)
                 const uint32_t r = row_at(it - 1);
-                const uint32_t sr2 = row_slot(p.ild, r);
+                const uint32_t sr2 = slot_of(p.ild, r);
                 C v2[9];
                 v2[0] = B[k][0];
                 v2[2] = B[k][1];
@@ -1245,8 +1252,11 @@ __device__ __forceinline__ void sweep_block(const SweepParams<S> &p, uint32_t xa
         for (uint32_t it = R + 2; it < ln.r_block + 2; it++) __syncthreads();
 }
 
+// Whole rows of one column per thread in FP32 and FP16: two 1024-thread blocks a CU, which
+// takes at most 64 vector and 80 scalar registers (with 88 scalar registers,
+// one block: 1531x1023 FP16 23.6 us a launch instead of 30.9).
 template <class S, int V, bool kProbe, bool kTiled, bool kBig>
-__global__ __launch_bounds__(kSweepThreads) void k_sweep2(SweepParams<S> p) {
+__global__ __launch_bounds__(kSweepThreads, sizeof(S) < 8 && V == 1 && !kBig && !kTiled ? 8 : 4) void k_sweep2(SweepParams<S> p) {
     extern __shared__ __align__(16) unsigned char smem[];
     const uint32_t blk = p.xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
     const SweepLanes ln{threadIdx.x, blockDim.x, smem, 0};
@@ -3240,6 +3250,7 @@ hipError_t sweep_typed(const Geom &g, const StateView &st, int src, const BcView
     p.rows = sweep_rows_typed<S>(g, bc, cfg);
     // buffers in the range-interleaved order of exactly these row ranges
     if (cfg.sweep_il_src || cfg.sweep_il_dst) {
+        if (!sweep_interleaves(sizeof(S), (int)V, tiled)) return hipErrorInvalidValue;
         const RowLayout il = row_layout(g.lx, p.rows);
         if (il.rows != p.rows) return hipErrorInvalidValue;
         if (cfg.sweep_il_src) p.il = il;
@@ -3702,12 +3713,14 @@ hipError_t launch_tile(int storage, const TileShape &sh, const Geom &g, const St
     return tile_rows(storage, sh, g, st, src, bc, omega, pr, slot, 0, g.lx, s);
 }
 
+bool seam_supported(int K, const Geom &g) { return K >= 1 && g.lx >= (uint32_t)(2 * K) && g.lx >= (uint32_t)K + 4; }
+
 hipError_t launch_seam(int storage, int K, const Geom &g, const StateView &st, int src, const BcView &bc, double omega,
                        const ProbeView &pr, int64_t slot, hipStream_t s) {
     TileShape sh;
     sh.K = K;
     sh.tx = 2 * K;
-    if (K < 1 || g.lx < (uint32_t)(2 * K)) return hipErrorInvalidValue;
+    if (!seam_supported(K, g)) return hipErrorInvalidValue;
     const size_t elem = storage == LBM_STORE_F64 ? 8 : (storage == LBM_STORE_F32 ? 4 : 2);
     const uint32_t ry = (uint32_t)tile_threads(elem, true) / (2 * K + 2 * (K + 1));
     // narrow tiles: one wave a SIMD and the whole GPU, since nothing runs beside

@@ -74,6 +74,8 @@ hipError_t launch_tile(int storage, const TileShape &sh, const Geom &g, const St
 // K steps of the rows that the pressure fix reaches in them, lx - K to K - 1
 // across the periodic seam: run after a K-step sweep of the whole lattice
 // without the fix, from the same source, it puts those rows right.
+// Needs K + 4 rows, for a node's dependencies to cross the seam only once.
+bool seam_supported(int K, const Geom &g);
 hipError_t launch_seam(int storage, int K, const Geom &g, const StateView &st, int src, const BcView &bc, double omega,
                        const ProbeView &pr, int64_t probe_slot, hipStream_t s);
 // Rows per block of the K-step kernel: `rows`, raised until every block

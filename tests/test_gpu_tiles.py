@@ -139,3 +139,10 @@ def test_pressure_fix_beside_sweeps(storage, lx, ly, kind, at):
     for a, b in zip(outs[0][0], outs[1][0]):
         assert torch.equal(a, b)
     assert np.array_equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("storage,lx,ly", [("f64", 3, 349530), ("f64", 4, 262147), ("f64", 5, 209733), ("f64", 6, 174771),
+                                           ("f32", 4, 786440)])
+def test_pressure_fix_of_few_long_rows(storage, lx, ly):
+    """large by their columns, but too few rows for the seam's launch (it needs K + 4)"""
+    test_pressure_fix_beside_sweeps(storage, lx, ly, "poiseuille", (1, 7))
