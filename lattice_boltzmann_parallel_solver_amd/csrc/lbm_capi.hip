@@ -2107,9 +2107,10 @@ struct RingEvents {
 
 // The copies and the kernel of lbm_step_host.  A pageable copy of 5.4 MB took
 // the runtime 168 us in and 310 us out, one from pinned memory 103 and 105 with
-// a 70 us memcpy beside it, so the arrays go through `stage` in quarters, the
-// memcpy of one beside the transfer of the others (and small lattices in one
-// transfer each way instead of three): four 420x180 calls 3.0 -> 2.7 ms.
+// a 70 us memcpy beside it, so the arrays go through `stage` in its quarters, the
+// memcpy of one beside the transfer of the others, and small lattices in one
+// transfer each way instead of three (us a call: 88x68 123 -> 90, 420x180 700 ->
+// 572, 420x300 1042 -> 867).
 int step_host_body(const lbm_bc_prog *prog, char *const in[3], char *const out[3], double omega, int nx, int ny,
                    char *work, char *stage, size_t stage_bytes, hipStream_t s) {
     const size_t N = (size_t)nx * ny, total = 96 * N, chunk = stage_bytes / 4;

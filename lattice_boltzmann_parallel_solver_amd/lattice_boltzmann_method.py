@@ -135,8 +135,12 @@ def lattice_boltzmann_step(f, density, velocity, omega: float,
     ins = [np.ascontiguousarray(a, dtype=np.float64) for a in (f, density, velocity)]
     outs = tuple(np.empty(a.shape) for a in ins)
     work = torch.empty(24 * lx * ly, dtype=torch.float64, device="cuda")
-    # four pinned quarters of 64 KiB to 2 MiB (torch keeps and hands them out again)
-    stage = torch.empty(4 * min(2 << 20, max(1 << 16, -(-96 * lx * ly // 2048) * 256)), dtype=torch.uint8, pin_memory=True)
+    # four pinned quarters (torch keeps and hands them out again): arrays of up
+    # to 2 MiB go in one piece, since each piece costs 25 us (88x68: 90 us a call
+    # in one, 182 in four), larger ones in four or more (420x180: 649 and 572)
+    total = 96 * lx * ly
+    piece = total if total <= 2 << 20 else min(2 << 20, -(-total // 4))
+    stage = torch.empty(4 * max(256, -(-piece // 256) * 256), dtype=torch.uint8, pin_memory=True)
     check(_lib.load().lbm_step_host(handle, *(a.ctypes.data for a in ins), float(omega), lx, ly,
                                     *(a.ctypes.data for a in outs), work.data_ptr(), stage.data_ptr(), stage.numel(),
                                     stream()))
