@@ -209,6 +209,7 @@ def autotune_lattice(lat: Lattice, omega: float, steps: int = 30) -> Tuple[int, 
         u[..., 0] = 0.05
         scratch.set_equilibrium(rho, u)
         scratch.run(omega, 2)
+        scratch.set_temporal(1)  # (a lattice without a setting may run several steps per launch)
         timings = []
         for cand in lattice_candidates(lat.ly, lat.storage):
             scratch.set_launch(*cand)
