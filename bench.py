@@ -75,8 +75,8 @@ TRAFFIC_JSON = os.path.join(ROOT, "profiles", "fused_step_8192x2048_hbm_traffic.
 def measured_traffic(storage, steps_per_launch=1):
     """HBM bytes per launch of the step kernel from the committed rocprofv3
     counter runs (keys "f32", "f64", "f16" for one step per launch,
-    "f32_sweep2", ... for the two-step kernel)."""
-    key = storage if steps_per_launch == 1 else f"{storage}_sweep2"
+    "f32_sweep2", ... for the two-step kernel, "f32_sweepv" for the three-step one)."""
+    key = storage + {1: "", 2: "_sweep2", 3: "_sweepv"}[steps_per_launch]
     try:
         with open(TRAFFIC_JSON) as fh:
             return float(json.load(fh)[key]["traffic_bytes"])
@@ -532,6 +532,9 @@ def main():
         torch.cuda.empty_cache()
     spl = lat.steps_per_launch
     steps = -(-args.steps // spl) * spl  # whole launches
+    # full FP32 rows take three steps per launch from a setting of two on,
+    # unless rows per block are given (the same results)
+    taken = 3 if spl >= 2 and args.storage == "f32" and not (tuned and tuned["rows_per_block"]) else spl
     ms = time_steps(lat, steps, args.warmup, torch)
     m, jx, _ = lat.moments_sum()
     assert m == m and abs(m / N - 1.0) < 0.1, "unstable run"
@@ -540,7 +543,7 @@ def main():
     torch.cuda.empty_cache()
     sec = ms / 1e3
     mlups = N * steps / sec / 1e6
-    launch_s = sec / (steps / spl)
+    launch_s = sec / (steps / taken)
     # one launch reads and writes every population once, whatever its step count
     bytes_launch = BYTES_PER_NODE[args.storage] * N
     achieved = bytes_launch / launch_s / 1e9
@@ -559,7 +562,7 @@ def main():
                 "steps_per_launch": spl_, "roofline_achieved_gbs": ach, "roofline_frac": ach / HBM_PEAK_GBS,
                 "bytes_per_node_step": BYTES_PER_NODE[storage] // spl_, "traffic": measured_traffic(storage, spl_)}
 
-    single = leg(args.storage, args.single_steps, 1) if spl == 2 else None
+    single = leg(args.storage, args.single_steps, 1) if spl >= 2 else None
     if single is not None and not args.no_extra:
         single["periodic_lattice"] = periodic_single_step_leg(torch, args.storage)
     fp64 = leg("f64", args.fp64_steps, args.temporal) if args.storage != "f64" else None
@@ -594,14 +597,15 @@ def main():
         "data": "synthetic",
         "config": {"workload": f"von Karman channel {LX}x{LY}, plate {PLATE} at x={LX // 4} (+1 y offset), "
                                f"rigid walls, inlet u={U_IN}, Re={RE:g}, {args.storage} population storage",
-                   "lx": LX, "ly": LY, "storage": args.storage, "omega": omega(), "steps_per_launch": spl,
+                   "lx": LX, "ly": LY, "storage": args.storage, "omega": omega(), "steps_per_launch": taken,
                    "launch_shape": tuned or "default",
                    "parallelism": "single GPU (whole lattice resident)"},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS, "traffic": measured_traffic(args.storage, spl),
-                     "kernel": "k_sweep2 (two steps per launch)" if spl == 2 else "k_fused (one step per launch)",
+                     "frac": achieved / HBM_PEAK_GBS, "traffic": measured_traffic(args.storage, taken),
+                     "kernel": {1: "k_fused (one step per launch)", 2: "k_sweep2 (two steps per launch)",
+                                3: "k_sweepv (three steps per launch)"}[taken],
                      "bytes_per_node_launch": BYTES_PER_NODE[args.storage],
-                     "bytes_per_node_step": BYTES_PER_NODE[args.storage] // spl,
+                     "bytes_per_node_step": BYTES_PER_NODE[args.storage] // taken,
                      "single_step_equivalent_gbs": mlups * 1e6 * BYTES_PER_NODE[args.storage] / 1e9,
                      "copy_gbs": copy, "frac_of_copy": achieved / copy,
                      "row_sweep_pattern_gbs": sweep_pattern, "frac_of_row_sweep_pattern": achieved / sweep_pattern,
