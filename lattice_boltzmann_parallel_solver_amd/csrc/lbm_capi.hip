@@ -213,9 +213,14 @@ int lbm_device_count(int *n) {
 }
 
 int lbm_bc_destroy(lbm_bc_prog *prog) {
-    if (prog && prog->dev_mem) {
-        (void)hipSetDevice(prog->dev_id);
-        (void)hipFree(prog->dev_mem);
+    if (prog && !prog->copies.empty()) {
+        int dev = -1;
+        const bool known = hipGetDevice(&dev) == hipSuccess;
+        for (const auto &d : prog->copies) {
+            (void)hipSetDevice(d.id);
+            (void)hipFree(d.mem);
+        }
+        if (known) (void)hipSetDevice(dev);
     }
     delete prog;
     return LBM_OK;
@@ -2008,29 +2013,27 @@ static int prog_on_device(const lbm_bc_prog *prog, BcView &view, const char *fn)
     int dev = 0;
     LBM_HIP_CHECK(hipGetDevice(&dev), fn);
     auto *p = const_cast<lbm_bc_prog *>(prog);
-    if (p->dev_mem && p->dev_id != dev) {
-        (void)hipSetDevice(p->dev_id);
-        (void)hipFree(p->dev_mem);
-        (void)hipSetDevice(dev);
-        p->dev_mem = nullptr;
-    }
-    if (!p->dev_mem) {
+    const lbm_bc_prog::DeviceCopy *at = nullptr;
+    for (const auto &d : p->copies)
+        if (d.id == dev) at = &d;
+    if (!at) {
+        try {
+            p->copies.reserve(p->copies.size() + 1);
+        } catch (const std::bad_alloc &) {
+            set_error(std::string(fn) + ": out of host memory");
+            return LBM_ERR_NOMEM;
+        }
         BcUpload up;
         LBM_HIP_CHECK(upload_bc(*p, up), fn);
-        p->dev_mem = up.mem;
-        p->dev_id = dev;
-        p->dev_codes = up.view.codes;
-        p->dev_chunk = up.view.chunk;
-        p->dev_wave = up.view.wave;
-        p->dev_classes = up.view.classes;
-        p->dev_special = up.view.special;
+        p->copies.push_back({dev, up.mem, up.view.codes, up.view.chunk, up.view.wave, up.view.classes, up.view.special});
+        at = &p->copies.back();
     }
-    view.codes = p->dev_codes;
-    view.chunk = p->dev_chunk;
-    view.wave = p->dev_wave;
-    view.classes = p->dev_classes;
+    view.codes = at->codes;
+    view.chunk = at->chunk;
+    view.wave = at->wave;
+    view.classes = at->classes;
+    view.special = at->special;
     view.nclasses = (uint32_t)p->classes.size();
-    view.special = p->dev_special;
     view.nspecial = (int64_t)p->special.size();
     view.rho_in = p->rho_in;
     view.rho_out = p->rho_out;

@@ -59,15 +59,19 @@ struct lbm_bc_prog {
     std::vector<uint32_t> special;          // nodes with a nonzero class
     double rho_in = 0, rho_out = 0;         // pressure fix densities
     uint32_t d1 = 0, d2 = 0;                // pressure fix direction sets
-    // device copy used by the stateless lbm_bc_apply / lbm_bc_pressure
-    // (uploaded on first use, released by lbm_bc_destroy)
-    int dev_id = -1;
-    void *dev_mem = nullptr;
-    const uint16_t *dev_codes = nullptr;
-    const uint8_t *dev_chunk = nullptr;
-    const uint8_t *dev_wave = nullptr;
-    const lbm::ClassEntry *dev_classes = nullptr;
-    const uint32_t *dev_special = nullptr;
+    // device copies used by the stateless calls: one for each device that a call
+    // ran on, uploaded by the first and kept until lbm_bc_destroy (another
+    // device's kernels may be reading theirs)
+    struct DeviceCopy {
+        int id = -1;
+        void *mem = nullptr;
+        const uint16_t *codes = nullptr;
+        const uint8_t *chunk = nullptr;
+        const uint8_t *wave = nullptr;
+        const lbm::ClassEntry *classes = nullptr;
+        const uint32_t *special = nullptr;
+    };
+    std::vector<DeviceCopy> copies;
 };
 
 namespace lbm {
