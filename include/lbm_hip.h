@@ -176,6 +176,19 @@ int lbm_set_launch(lbm_ctx *ctx, int cells_per_thread, int xcd_remap, int nt_sto
  * every setting.  No counterpart in the reference (a launch setting of this
  * library). */
 int lbm_set_temporal(lbm_ctx *ctx, int steps_per_launch, int rows_per_block);
+/* The kernel that lbm_run(ctx, omega, nsteps) would launch first in the
+ * context's present state and settings, and the steps that this launch
+ * advances (a run is the launches for nsteps, nsteps - steps, ...).  Launches
+ * nothing.  No counterpart in the reference. */
+#define LBM_LAUNCH_FIRST 0       /* the collision of a loaded state */
+#define LBM_LAUNCH_STEP 1        /* one step */
+#define LBM_LAUNCH_TILE 2        /* several steps on tiles held on chip */
+#define LBM_LAUNCH_SWEEP2 3      /* two-step row sweep */
+#define LBM_LAUNCH_SWEEPK 4      /* three- or four-step row sweep, one column per thread */
+#define LBM_LAUNCH_SWEEPV 5      /* three-step row sweep, adjacent columns per lane */
+#define LBM_LAUNCH_SWEEP2_SEAM 6 /* SWEEP2 without the pressure fix, then the rows that it reaches */
+#define LBM_LAUNCH_SWEEPV_SEAM 7 /* the same with SWEEPV */
+int lbm_next_launch(lbm_ctx *ctx, int64_t nsteps, int *kernel, int *steps);
 /* Column tiles of the two-step kernel: blocks of at most `threads` threads (a
  * multiple of 64 up to 1024; 0 = whole rows up to 1024 threads, the default),
  * each sweeping a tile of columns plus one halo column each side, so that the

@@ -33,6 +33,8 @@ BC_RIGID_OBJECT = 3
 BC_INLET = 4
 BC_OUTLET = 5
 BC_PRESSURE_PERIODIC = 6
+# the kernels of lbm_next_launch, in the order of their numbers
+LAUNCHES = ("first", "step", "tile", "sweep2", "sweepk", "sweepv", "sweep2_seam", "sweepv_seam")
 
 
 class LbmError(RuntimeError):
@@ -95,6 +97,7 @@ _SIGNATURES = {
     "lbm_steps_done": (_I, [_P, ctypes.POINTER(_I64)]),
     "lbm_set_launch": (_I, [_P, _I, _I, _I]),
     "lbm_set_temporal": (_I, [_P, _I, _I]),
+    "lbm_next_launch": (_I, [_P, _I64, ctypes.POINTER(_I), ctypes.POINTER(_I)]),
     "lbm_set_sweep_tile": (_I, [_P, _I, _I]),
     "lbm_set_row_layout": (_I, [_P, _I]),
     "lbm_batch_create": (_I, [ctypes.POINTER(_P), ctypes.POINTER(_P), ctypes.POINTER(ctypes.c_double), _I]),

@@ -109,6 +109,19 @@ hipError_t upload_bc(const lbm_bc_prog &p, BcUpload &up) {
 
 }  // namespace
 
+namespace lbm {
+// What the launches of a run may take.
+struct RunPlan {
+    bool ready = false;
+    int K = 1;            // steps per launch asked for, or the library's choice; 0: tiles, the seam path or single steps
+    TileShape tile;       // K = 0: no tiles
+    int seam = 0;         // steps of a sweep that the pressure fix's rows are put right after; 0: not taken
+    BcView nofix;         // the boundary without the fix, for those sweeps
+    SweepVShape v;        // K = 0: not taken
+    bool sweepk = false, sweep2 = false;
+};
+}  // namespace lbm
+
 struct lbm_ctx {
     int nx = 0, ny = 0, storage = 0, device = 0;
     Geom g;
@@ -126,9 +139,7 @@ struct lbm_ctx {
     double *sums = nullptr;
     LaunchCfg cfg;
     uint8_t *codes8 = nullptr;  // bc.view.codes8
-    // tiling of the tile kernel, worked out by the first run that may take it
-    TileShape tile;
-    bool tile_ready = false;
+    RunPlan plan;  // (cleared with each change of boundary or settings)
     bool stage_eq = false;  // pending: stage_f is the equilibrium of stage_rho and stage_u
 };
 
@@ -323,6 +334,7 @@ int lbm_set_launch(lbm_ctx *c, int v, int xcd, int nt) {
     c->cfg.xcd_remap = xcd ? 1 : 0;
     c->cfg.nt_stores = nt ? 1 : 0;
     c->cfg.shape_given = v != 1 || !xcd || nt;  // (the default shape is no request)
+    c->plan.ready = false;
     return LBM_OK;
 }
 
@@ -350,6 +362,7 @@ int lbm_set_temporal(lbm_ctx *c, int steps_per_launch, int rows_per_block) {
     }
     c->cfg.steps_per_launch = steps_per_launch;
     c->cfg.sweep_rows = rows_per_block;
+    c->plan.ready = false;
     return LBM_OK;
 }
 
@@ -371,6 +384,7 @@ int lbm_set_sweep_tile(lbm_ctx *c, int threads, int cols_per_thread) {
     }
     c->cfg.sweep_tile = threads;
     c->cfg.sweep_v = cols_per_thread;
+    c->plan.ready = false;
     return LBM_OK;
 }
 
@@ -413,7 +427,7 @@ int lbm_set_bc(lbm_ctx *c, const lbm_bc_prog *prog) {
     (void)hipFree(c->codes8);
     c->codes8 = nullptr;
     c->bc = BcUpload{};
-    c->tile_ready = false;
+    c->plan.ready = false;
     if (prog) {
         LBM_HIP_CHECK(upload_bc(*prog, c->bc), "lbm_set_bc: upload");
         if (c->bc.view.nclasses <= 256 && sweepv_fits(c->storage, c->g)) {
@@ -494,6 +508,116 @@ static int run_steps_per_launch(const lbm_ctx *c) {
     return 2;
 }
 
+// The kernels that a run of this context may take, worked out once for its
+// boundary and settings.
+static const RunPlan &run_plan(lbm_ctx *c) {
+    RunPlan &p = c->plan;
+    if (p.ready) return p;
+    p = RunPlan{};
+    p.K = run_steps_per_launch(c);
+    // Small lattices: several steps per launch on tiles.  One step per launch
+    // and launch shapes, row counts or column tiles that the caller chose keep
+    // their kernels.
+    const bool free = p.K != 1 && !c->cfg.shape_given && c->cfg.sweep_rows == 0 && c->cfg.sweep_tile == 0;
+    if (free) p.tile = tile_shape(c->storage, c->g, c->bc.view);
+    // The pressure fix reaches K rows to each side of the periodic seam in K
+    // steps.  A lattice that was given no launch setting sweeps K steps at once
+    // as if it had no fix, and puts those 2 K rows right from the same source.
+    // The seam's launch costs 11 us, so it pays from a size on (us a step, one
+    // step per launch / sweep and seam: FP64 2048x2048 107 / 80, 4096x1000 106 /
+    // 61, 1500x1500 58 / 47, 1100x1000 25.9 / 24.5; FP32 2048x2048 48 / 38,
+    // 4096x1000 51 / 39, 1500x1500 25.8 / 24.1, 2048x1024 24.1 / 24.5; FP16
+    // 3000x2048 43 / 39, 2048x2048 31.6 / 30.0, 4096x1000 33 / 34).
+    p.nofix = c->bc.view;
+    p.nofix.flags &= ~(uint32_t)kProgPressure;
+    if (p.K == 0 && free && (c->bc.view.flags & kProgPressure) && c->g.N >= seam_nodes(c->storage)) {
+        const SweepVShape v = sweepv_shape(c->storage, c->g, p.nofix);
+        const SweepShape sh = sweep_shape(c->storage, c->g.ly);
+        const int k = v.K > 0 ? v.K
+                      : sweep_supported(c->storage, c->g, p.nofix) && (uint64_t)c->g.lx * sh.ntiles >= 256 ? 2 : 0;
+        if (seam_supported(k, c->g)) {
+            p.seam = k;
+            p.v = v;
+        }
+    }
+    // Full rows of two (FP32) or one (FP64) column per thread: three steps per
+    // launch with adjacent columns per lane, under the same conditions.
+    if (free && p.K >= 2) p.v = sweepv_shape(c->storage, c->g, c->bc.view);
+    p.sweepk = p.K >= 3 && sweepk_supported(c->storage, c->g, c->bc.view, p.K);
+    p.sweep2 = p.K >= 2 && sweep_supported(c->storage, c->g, c->bc.view, c->cfg.sweep_tile, c->cfg.sweep_v);
+    p.ready = true;
+    return p;
+}
+
+// The kernel of a run's next launch with `left` steps to go, and its steps.
+struct Launch {
+    int kernel, steps;
+};
+static Launch next_launch(lbm_ctx *c, int64_t left) {
+    if (c->phase == kPending) return {LBM_LAUNCH_FIRST, 1};
+    if (left < 2) return {LBM_LAUNCH_STEP, 1};
+    const RunPlan &p = run_plan(c);
+    if (p.tile.K > 0) return {LBM_LAUNCH_TILE, (int)std::min<int64_t>(p.tile.K, left)};
+    if (p.seam > 0) {
+        if (left >= p.seam) return {p.seam == 2 ? LBM_LAUNCH_SWEEP2_SEAM : LBM_LAUNCH_SWEEPV_SEAM, p.seam};
+        return {LBM_LAUNCH_STEP, 1};
+    }
+    if (p.v.K > 0 && left >= p.v.K) return {LBM_LAUNCH_SWEEPV, p.v.K};
+    if (p.sweepk && left >= p.K) return {LBM_LAUNCH_SWEEPK, p.K};
+    if (p.sweep2) return {LBM_LAUNCH_SWEEP2, 2};
+    return {LBM_LAUNCH_STEP, 1};
+}
+
+// Launch settings of a run's two-step sweeps.
+//
+// A long run keeps the state in the range-interleaved row order of the sweep's
+// row ranges (the rows all blocks touch at once become neighbours in memory):
+// its first launch reads the plain order and writes that one, its last the
+// other way round (two separate copies of the state cost 410 us a run at 4200
+// x 1800 FP64).
+// Measured where it pays: FP32 rows of two columns per thread and FP64 column
+// tiles, with 16 or more rows per block and at most two rounds of resident row
+// ranges (8192 x 2048 FP32 137.3 -> 147.4 GLUPS, FP64 67.7 -> 69.4, 4200 x
+// 1800 FP32 125.5 -> 128.3, 65536 x 2048 FP32 in two rounds 141.8 -> 144.1).
+// It lost on one column per thread (8192 x 1024 FP32 130.1 -> 121.5), at 8
+// rows per block (2048 x 2048 FP32 125.7 -> 122.9), in FP16 (220.5 -> 214.4)
+// and over seven rounds (65536 x 2048 FP64 69.1 -> 65.1), which keep the plain
+// order.
+static LaunchCfg sweep2_settings(const lbm_ctx *c, int64_t left, bool &interleave) {
+    LaunchCfg cfg = c->cfg;
+    interleave = false;
+    const SweepShape sh = sweep_shape(c->storage, c->g.ly, cfg.sweep_tile, cfg.sweep_v);
+    if (cfg.row_interleave && left / 2 >= kInterleaveMinPairs && c->g.lx < kRowLayoutMaxLx &&
+        c->storage != LBM_STORE_F16 && (sh.v == 2 || sh.ntiles > 1)) {
+        const int rows = sweep2_rows(c->storage, c->g, c->bc.view, cfg);
+        const int64_t ranges = rows > 0 ? ((int64_t)c->g.lx + rows - 1) / rows : 0;
+        const int resident = sweep2_resident_ranges(c->storage, c->g, c->bc.view, cfg);
+        if (rows >= kInterleaveMinRows && rows <= (int)kRowLayoutMaxRows && rows < (int)c->g.lx && resident > 0 &&
+            ranges <= 2 * (int64_t)resident) {
+            cfg.sweep_rows = rows;
+            interleave = true;
+        }
+    }
+    return cfg;
+}
+
+int lbm_next_launch(lbm_ctx *c, int64_t nsteps, int *kernel, int *steps) {
+    int rc = check_ctx(c, "lbm_next_launch");
+    if (rc) return rc;
+    if (nsteps < 1 || !kernel || !steps) {
+        set_error("lbm_next_launch: need nsteps >= 1, kernel and steps");
+        return LBM_ERR_ARG;
+    }
+    if (c->phase == kEmpty) {
+        set_error("lbm_next_launch: no state loaded (call lbm_set_state first)");
+        return LBM_ERR_STATE;
+    }
+    const Launch l = next_launch(c, nsteps);
+    *kernel = l.kernel;
+    *steps = l.steps;
+    return LBM_OK;
+}
+
 int lbm_run(lbm_ctx *c, double omega, int64_t nsteps) {
     int rc = check_ctx(c, "lbm_run");
     if (rc) return rc;
@@ -511,150 +635,81 @@ int lbm_run(lbm_ctx *c, double omega, int64_t nsteps) {
     }
     if (nsteps == 0) return LBM_OK;
     int64_t left = nsteps;
-    if (c->phase == kPending) {
-        LBM_HIP_CHECK(launch_collide_first(c->storage, c->g, c->stage_f, c->stage_rho, c->stage_u, c->st, c->cur,
-                                           c->bc.view, omega, c->stage_eq, c->stream),
-                      "first-collision kernel");
-        c->phase = kRunning;
-        c->steps++;
-        left--;
-    }
     const bool probing = c->probe.cell >= 0;
-    const int K = run_steps_per_launch(c);
-    // Small lattices: several steps per launch on tiles.  A step alone, one
-    // step per launch and launch shapes, row counts or column tiles that the
-    // caller chose keep their kernels.
-    const bool tiles = K != 1 && !c->cfg.shape_given && c->cfg.sweep_rows == 0 && c->cfg.sweep_tile == 0;
-    if (tiles && !c->tile_ready) {
-        c->tile = tile_shape(c->storage, c->g, c->bc.view);
-        c->tile_ready = true;
-    }
-    while (tiles && left > 1 && c->tile.K > 0) {
-        TileShape sh = c->tile;
-        sh.K = (int)std::min<int64_t>(sh.K, left);
+    const BcView &bc = c->bc.view;
+    LaunchCfg cfg2 = c->cfg;  // of the two-step sweeps
+    bool cfg2_set = false, interleave = false;
+    while (left > 0) {
+        const Launch l = next_launch(c, left);
+        // a launch of s steps materialises f_{steps} .. f_{steps+s-1} on chip:
+        // it records them if probed
         const int64_t slot = probing ? c->steps - c->probe_base - 1 : -1;
-        LBM_HIP_CHECK(launch_tile(c->storage, sh, c->g, c->st, c->cur, c->bc.view, omega, c->probe, slot, c->stream),
-                      "tile kernel");
-        c->cur ^= 1;
-        c->steps += sh.K;
-        left -= sh.K;
-    }
-    // The pressure fix reaches K rows to each side of the periodic seam in K
-    // steps.  A lattice that was given no launch setting sweeps K steps at once
-    // as if it had no fix, and puts those 2 K rows right from the same source.
-    // The seam's launch costs 11 us, so it pays from a size on (us a step, one
-    // step per launch / sweep and seam: FP64 2048x2048 107 / 80, 4096x1000 106 /
-    // 61, 1500x1500 58 / 47, 1100x1000 25.9 / 24.5; FP32 2048x2048 48 / 38,
-    // 4096x1000 51 / 39, 1500x1500 25.8 / 24.1, 2048x1024 24.1 / 24.5; FP16
-    // 3000x2048 43 / 39, 2048x2048 31.6 / 30.0, 4096x1000 33 / 34).
-    if (K == 0 && tiles && (c->bc.view.flags & kProgPressure) && c->g.N >= seam_nodes(c->storage)) {
-        BcView walls = c->bc.view;
-        walls.flags &= ~(uint32_t)kProgPressure;
-        const SweepVShape sv = sweepv_shape(c->storage, c->g, walls);
-        const SweepShape sh = sweep_shape(c->storage, c->g.ly);
-        LaunchCfg cfg = c->cfg;
-        int step = sv.K > 0 ? sv.K
-                   : sweep_supported(c->storage, c->g, walls) && (uint64_t)c->g.lx * sh.ntiles >= 256 ? 2 : 0;
-        if (!seam_supported(step, c->g)) step = 0;
-        for (; step > 0 && left >= step; left -= step) {
-            const int64_t slot = probing ? c->steps - c->probe_base - 1 : -1;
-            LBM_HIP_CHECK(step == 2 ? launch_sweep2(c->storage, c->g, c->st, c->cur, walls, omega, c->probe, slot,
-                                                    probing ? slot + 1 : -1, cfg, c->stream)
-                                    : launch_sweepv(c->storage, sv, c->g, c->st, c->cur, walls, omega, c->probe, slot,
-                                                    c->stream),
-                          "sweep kernel");
-            LBM_HIP_CHECK(launch_seam(c->storage, step, c->g, c->st, c->cur, c->bc.view, omega, c->probe, slot, c->stream),
-                          "seam kernel");
-            c->cur ^= 1;
-            c->steps += step;
-        }
-    }
-    // Full rows of two (FP32) or one (FP64) column per thread: three steps per
-    // launch with adjacent columns per lane, under the same conditions.
-    if (tiles && K >= 2) {
-        const SweepVShape sh = sweepv_shape(c->storage, c->g, c->bc.view);
-        for (; sh.K > 0 && left >= sh.K; left -= sh.K) {
-            const int64_t slot = probing ? c->steps - c->probe_base - 1 : -1;
-            LBM_HIP_CHECK(launch_sweepv(c->storage, sh, c->g, c->st, c->cur, c->bc.view, omega, c->probe, slot,
-                                        c->stream),
-                          "three-step sweep kernel");
-            c->cur ^= 1;
-            c->steps += sh.K;
-        }
-    }
-    if (K >= 3 && sweepk_supported(c->storage, c->g, c->bc.view, K)) {
-        for (; left >= K; left -= K) {
-            // materialises f_{steps} .. f_{steps+K-1}
-            const int64_t slot = probing ? c->steps - c->probe_base - 1 : -1;
-            LBM_HIP_CHECK(launch_sweepk(c->storage, K, c->g, c->st, c->cur, c->bc.view, omega, c->probe, slot,
-                                        c->cfg, c->stream),
-                          "K-step sweep kernel");
-            c->cur ^= 1;
-            c->steps += K;
-        }
-    }
-    if (K >= 2 && sweep_supported(c->storage, c->g, c->bc.view, c->cfg.sweep_tile, c->cfg.sweep_v)) {
-        // A long run keeps the state in the range-interleaved row order of the
-        // sweep's row ranges (the rows all blocks touch at once become
-        // neighbours in memory): its first launch reads the plain order and
-        // writes that one, its last the other way round (two separate copies
-        // of the state cost 410 us a run at 4200 x 1800 FP64).
-        // Measured where it pays: FP32 rows of two columns per thread and FP64
-        // column tiles, with 16 or more rows per block and at most two rounds
-        // of resident row ranges (8192 x 2048 FP32 137.3 -> 147.4 GLUPS, FP64
-        // 67.7 -> 69.4, 4200 x 1800 FP32 125.5 -> 128.3, 65536 x 2048 FP32 in
-        // two rounds 141.8 -> 144.1).  It lost on one column per thread (8192
-        // x 1024 FP32 130.1 -> 121.5), at 8 rows per block (2048 x 2048 FP32
-        // 125.7 -> 122.9), in FP16 (220.5 -> 214.4) and over seven rounds
-        // (65536 x 2048 FP64 69.1 -> 65.1), which keep the plain order.
-        LaunchCfg cfg = c->cfg;
-        bool ilv = false;
-        const SweepShape sh = sweep_shape(c->storage, c->g.ly, cfg.sweep_tile, cfg.sweep_v);
-        if (cfg.row_interleave && left / 2 >= kInterleaveMinPairs && c->g.lx < kRowLayoutMaxLx &&
-            c->storage != LBM_STORE_F16 && (sh.v == 2 || sh.ntiles > 1)) {
-            const int rows = sweep2_rows(c->storage, c->g, c->bc.view, cfg);
-            const int64_t ranges = rows > 0 ? ((int64_t)c->g.lx + rows - 1) / rows : 0;
-            const int resident = sweep2_resident_ranges(c->storage, c->g, c->bc.view, cfg);
-            if (rows >= kInterleaveMinRows && rows <= (int)kRowLayoutMaxRows && rows < (int)c->g.lx &&
-                resident > 0 && ranges <= 2 * (int64_t)resident) {
-                cfg.sweep_rows = rows;
-                ilv = true;
+        switch (l.kernel) {
+            case LBM_LAUNCH_FIRST:
+                LBM_HIP_CHECK(launch_collide_first(c->storage, c->g, c->stage_f, c->stage_rho, c->stage_u, c->st, c->cur, bc,
+                                                   omega, c->stage_eq, c->stream),
+                              "first-collision kernel");
+                c->phase = kRunning;
+                break;
+            case LBM_LAUNCH_TILE: {
+                TileShape sh = c->plan.tile;
+                sh.K = l.steps;
+                LBM_HIP_CHECK(launch_tile(c->storage, sh, c->g, c->st, c->cur, bc, omega, c->probe, slot, c->stream),
+                              "tile kernel");
+                break;
             }
+            case LBM_LAUNCH_SWEEP2_SEAM:
+            case LBM_LAUNCH_SWEEPV_SEAM: {
+                const BcView &walls = c->plan.nofix;
+                LBM_HIP_CHECK(l.kernel == LBM_LAUNCH_SWEEP2_SEAM
+                                  ? launch_sweep2(c->storage, c->g, c->st, c->cur, walls, omega, c->probe, slot,
+                                                  probing ? slot + 1 : -1, c->cfg, c->stream)
+                                  : launch_sweepv(c->storage, c->plan.v, c->g, c->st, c->cur, walls, omega, c->probe, slot,
+                                                  c->stream),
+                              "sweep kernel");
+                LBM_HIP_CHECK(launch_seam(c->storage, l.steps, c->g, c->st, c->cur, bc, omega, c->probe, slot, c->stream),
+                              "seam kernel");
+                break;
+            }
+            case LBM_LAUNCH_SWEEPV:
+                LBM_HIP_CHECK(launch_sweepv(c->storage, c->plan.v, c->g, c->st, c->cur, bc, omega, c->probe, slot, c->stream),
+                              "three-step sweep kernel");
+                break;
+            case LBM_LAUNCH_SWEEPK:
+                LBM_HIP_CHECK(launch_sweepk(c->storage, l.steps, c->g, c->st, c->cur, bc, omega, c->probe, slot, c->cfg,
+                                            c->stream),
+                              "K-step sweep kernel");
+                break;
+            case LBM_LAUNCH_SWEEP2: {
+                // (the two-step launches of a run follow one another to its last step or two)
+                if (!cfg2_set) cfg2 = sweep2_settings(c, left, interleave);
+                cfg2_set = true;
+                cfg2.sweep_il_src = cfg2.sweep_il_dst;
+                cfg2.sweep_il_dst = interleave && left >= 4;
+                const hipError_t e = launch_sweep2(c->storage, c->g, c->st, c->cur, bc, omega, c->probe, slot,
+                                                   probing ? slot + 1 : -1, cfg2, c->stream);
+                // after a failed launch the state, with the steps done so far, may
+                // still be in the other order (what the failed launch would have read)
+                if (e != hipSuccess && cfg2.sweep_il_src) {
+                    const hipError_t eb = launch_row_layout(c->storage, c->g, c->st, c->cur, (uint32_t)cfg2.sweep_rows, false,
+                                                            c->stream);
+                    if (eb == hipSuccess) c->cur ^= 1;
+                    LBM_HIP_CHECK(eb, "row order kernel");
+                }
+                LBM_HIP_CHECK(e, "two-step sweep kernel");
+                break;
+            }
+            default:
+                LBM_HIP_CHECK(launch_fused(c->storage, c->g, c->st, c->cur, bc, omega, c->probe, slot, nullptr, c->cfg,
+                                           c->stream, nullptr),
+                              "fused step kernel");
         }
-        hipError_t e = hipSuccess;
-        for (; left >= 2; left -= 2) {
-            // materialises f_{steps} and f_{steps+1}
-            const int64_t slot = probing ? c->steps - c->probe_base - 1 : -1;
-            cfg.sweep_il_src = cfg.sweep_il_dst;
-            cfg.sweep_il_dst = ilv && left >= 4;
-            e = launch_sweep2(c->storage, c->g, c->st, c->cur, c->bc.view, omega, c->probe, slot,
-                              probing ? slot + 1 : -1, cfg, c->stream);
-            if (e != hipSuccess) break;
-            c->cur ^= 1;
-            c->steps += 2;
-        }
-        // after a failed launch the state, with the steps done so far, may still
-        // be in the other order (what the failed launch would have read)
-        if (e != hipSuccess && cfg.sweep_il_src) {
-            const hipError_t eb = launch_row_layout(c->storage, c->g, c->st, c->cur, (uint32_t)cfg.sweep_rows, false,
-                                                    c->stream);
-            if (eb == hipSuccess) c->cur ^= 1;
-            LBM_HIP_CHECK(eb, "row order kernel");
-        }
-        LBM_HIP_CHECK(e, "two-step sweep kernel");
-    }
-    for (; left > 0; left--) {
-        // this launch materialises f_{steps} in registers: record it if probed
-        const int64_t slot = probing ? c->steps - c->probe_base - 1 : -1;
-        LBM_HIP_CHECK(launch_fused(c->storage, c->g, c->st, c->cur, c->bc.view, omega, c->probe, slot, nullptr,
-                                   c->cfg, c->stream, nullptr),
-                      "fused step kernel");
-        c->cur ^= 1;
-        c->steps++;
+        if (l.kernel != LBM_LAUNCH_FIRST) c->cur ^= 1;  // (the first collision writes planes[cur])
+        c->steps += l.steps;
+        left -= l.steps;
     }
     if (probing && c->steps > c->probe_base)
-        LBM_HIP_CHECK(launch_probe_cell(c->storage, c->g, c->st, c->cur, c->bc.view, c->probe,
-                                        c->steps - c->probe_base - 1, c->stream),
+        LBM_HIP_CHECK(launch_probe_cell(c->storage, c->g, c->st, c->cur, bc, c->probe, c->steps - c->probe_base - 1, c->stream),
                       "probe kernel");
     return LBM_OK;
 }

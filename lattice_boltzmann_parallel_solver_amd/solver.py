@@ -168,6 +168,14 @@ class Lattice:
         more than 128 boundary classes, LDS)."""
         check(_lib.load().lbm_set_temporal(self._h, int(steps_per_launch), int(rows_per_block)))
 
+    def next_launch(self, steps: int) -> Tuple[str, int]:
+        """The kernel that `run(omega, steps)` would launch first in the present
+        state and settings (one of `_lib.LAUNCHES`), and the steps that this
+        launch advances."""
+        kernel, k = ctypes.c_int(), ctypes.c_int()
+        check(_lib.load().lbm_next_launch(self._h, int(steps), ctypes.byref(kernel), ctypes.byref(k)))
+        return _lib.LAUNCHES[kernel.value], k.value
+
     def set_sweep_tile(self, threads: int = 0, cols_per_thread: int = 0) -> None:
         """Two-step launches in column tiles of blocks of at most `threads`
         threads (a multiple of 64; 0 = whole rows up to 1024 threads), each
