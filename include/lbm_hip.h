@@ -156,7 +156,11 @@ int lbm_steps_done(const lbm_ctx *ctx, int64_t *steps);
 /* Launch tuning of the fused step: nodes per thread (1, 2 or 4; 0 = aligned
  * 16-byte groups, needs ny divisible by 2/4/8 for FP64/FP32/FP16), XCD-aware
  * block order (0/1), non-temporal stores (0/1).  Default {1, 1, 0}, the
- * fastest measured on MI355X for every storage. */
+ * fastest measured on MI355X for every storage.  A context on which this was
+ * called (with the default too) and lbm_set_temporal was not runs one step per
+ * launch.  With lbm_set_temporal of 2 or more, another shape than the default
+ * keeps the row sweeps, which take its block order and stores, where tiles or
+ * the three-step sweep of full rows would run. */
 int lbm_set_launch(lbm_ctx *ctx, int cells_per_thread, int xcd_remap, int nt_stores);
 /* Temporal blocking of lbm_run: steps_per_launch = 2 advances two steps per
  * kernel launch (a row sweep that keeps the intermediate state on chip and

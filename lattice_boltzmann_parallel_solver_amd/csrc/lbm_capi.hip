@@ -333,7 +333,7 @@ int lbm_set_launch(lbm_ctx *c, int v, int xcd, int nt) {
     c->cfg.cells_per_thread = v;
     c->cfg.xcd_remap = xcd ? 1 : 0;
     c->cfg.nt_stores = nt ? 1 : 0;
-    c->cfg.shape_given = v != 1 || !xcd || nt;  // (the default shape is no request)
+    c->cfg.shape_given = true;
     c->plan.ready = false;
     return LBM_OK;
 }
@@ -508,6 +508,10 @@ static int run_steps_per_launch(const lbm_ctx *c) {
     return 2;
 }
 
+static bool default_shape(const LaunchCfg &cfg) {
+    return cfg.cells_per_thread == 1 && cfg.xcd_remap && !cfg.nt_stores;
+}
+
 // The kernels that a run of this context may take, worked out once for its
 // boundary and settings.
 static const RunPlan &run_plan(lbm_ctx *c) {
@@ -516,9 +520,9 @@ static const RunPlan &run_plan(lbm_ctx *c) {
     p = RunPlan{};
     p.K = run_steps_per_launch(c);
     // Small lattices: several steps per launch on tiles.  One step per launch
-    // and launch shapes, row counts or column tiles that the caller chose keep
-    // their kernels.
-    const bool free = p.K != 1 && !c->cfg.shape_given && c->cfg.sweep_rows == 0 && c->cfg.sweep_tile == 0;
+    // and row counts, column tiles or another launch shape than the default
+    // (the row sweep takes its block order and stores) keep their kernels.
+    const bool free = p.K != 1 && default_shape(c->cfg) && c->cfg.sweep_rows == 0 && c->cfg.sweep_tile == 0;
     if (free) p.tile = tile_shape(c->storage, c->g, c->bc.view);
     // The pressure fix reaches K rows to each side of the periodic seam in K
     // steps.  A lattice that was given no launch setting sweeps K steps at once

@@ -152,7 +152,10 @@ class Lattice:
 
     def set_launch(self, cells_per_thread: int = 1, xcd_remap: bool = True, nt_stores: bool = False) -> None:
         """Launch shape of the fused step: nodes per thread (1, 2, 4; 0 = aligned
-        16-byte groups), XCD-aware block order, non-temporal stores."""
+        16-byte groups), XCD-aware block order, non-temporal stores.  A lattice
+        on which this was called (with the default shape too) and
+        `set_temporal` was not runs one step per launch; with two or more, a
+        shape other than the default keeps the row sweeps."""
         check(_lib.load().lbm_set_launch(self._h, int(cells_per_thread), int(bool(xcd_remap)), int(bool(nt_stores))))
 
     def set_temporal(self, steps_per_launch: int = 2, rows_per_block: int = 0) -> None:

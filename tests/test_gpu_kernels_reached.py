@@ -135,6 +135,20 @@ def test_pressure_fix_beside_sweeps():
     assert _kernel(2048, 2048, "f64", "poiseuille", 1, 9) == ("step", 1)
 
 
+@pytest.mark.parametrize("shape", [(1, True, False), (2, True, False), (1, False, False), (1, True, True)])
+def test_a_launch_shape_means_single_steps(shape):
+    """also the default shape, called for; an explicit number of steps goes before it"""
+    lat = Lattice(300, 100)
+    lat.set_equilibrium(np.ones((300, 100)), np.zeros((300, 100, 2)))
+    lat.run(1.0, 1)
+    assert lat.next_launch(9)[0] == "tile"
+    lat.set_launch(*shape)
+    assert lat.next_launch(9) == ("step", 1)
+    lat.set_temporal(2)
+    assert lat.next_launch(9)[0] == ("tile" if shape == (1, True, False) else "sweep2")
+    lat.close()
+
+
 def test_next_launch_refuses_what_a_run_refuses():
     from lattice_boltzmann_parallel_solver_amd._lib import LbmError
 
