@@ -522,7 +522,8 @@ static const RunPlan &run_plan(lbm_ctx *c) {
     // Small lattices: several steps per launch on tiles.  One step per launch
     // and row counts, column tiles or another launch shape than the default
     // (the row sweep takes its block order and stores) keep their kernels.
-    const bool free = p.K != 1 && default_shape(c->cfg) && c->cfg.sweep_rows == 0 && c->cfg.sweep_tile == 0;
+    const bool free = p.K != 1 && default_shape(c->cfg) && c->cfg.sweep_rows == 0 && c->cfg.sweep_tile == 0 &&
+                      c->cfg.sweep_v == 0;
     if (free) p.tile = tile_shape(c->storage, c->g, c->bc.view);
     // The pressure fix reaches K rows to each side of the periodic seam in K
     // steps.  A lattice that was given no launch setting sweeps K steps at once
