@@ -26,6 +26,7 @@
 #include "lbm_batch_tables.h"
 #include "lbm_rowlayout.h"
 #include "lbm_launch.h"
+#include "lbm_plan.h"
 
 namespace lbm {
 namespace {
@@ -156,10 +157,6 @@ bool three_steps_pay(int storage, unsigned waves) {
 // order (moving the state there and back costs about two launches).
 constexpr int64_t kInterleaveMinPairs = 32;
 constexpr int kInterleaveMinRows = 16;
-// Smallest lattice with the pressure fix that sweeps several steps per launch.
-uint32_t seam_nodes(int storage) {
-    return storage == LBM_STORE_F64 ? 1u << 20 : (storage == LBM_STORE_F32 ? 3u << 20 : 1u << 22);
-}
 
 // Bytes of one state buffer: nine planes of lx rows, `pitch` elements a row.
 size_t plane_bytes(const lbm_ctx *c) { return 9 * (size_t)c->g.lx * c->g.pitch * plane_elem(c->storage); }
@@ -490,18 +487,24 @@ int lbm_set_state_equilibrium(lbm_ctx *c, const double *rho, const double *u, in
     return LBM_OK;
 }
 
+// Whether two steps per launch of the whole lattice beat single steps, with
+// extra_us a launch on top.
+static bool sweep_pays(const lbm_ctx *c, const BcView &bc, double extra_us) {
+    const LaunchCfg automatic{1, 1, 0};
+    return two_steps_pay(c->storage, c->g, bc.codes != nullptr, sweep_shape(c->storage, c->g.ly),
+                         sweep2_rows(c->storage, c->g, bc, automatic),
+                         sweep2_resident_ranges(c->storage, c->g, bc, automatic), extra_us);
+}
+
 // Steps per launch of a run: the caller's, or for a context that was given no
-// launch setting at all (0) what measured fastest.  Two wherever the row sweep
-// applies and one row a block fills the GPU (64x4000 FP32 has not the rows: 5.9
-// us a step with one, 9.7 with two; 1200x514 FP64 16.1 and 15.2, 8192x2048 FP32
-// 202 and 113); three for long FP32 lattices of the widths where they pay
-// (8192x1024: 131 GLUPS with two, 177 with three; 2000x1024: 15.9 us and 16.0).
-// 0 stays 0 where only tiles and single steps apply.
+// launch setting at all (0) what measured fastest.  Two where the row sweep
+// applies and is faster (two_steps_pay); three for long FP32 lattices of the
+// widths where they pay (8192x1024: 131 GLUPS with two, 177 with three;
+// 2000x1024: 15.9 us and 16.0).  0 stays 0 where only tiles and single steps apply.
 static int run_steps_per_launch(const lbm_ctx *c) {
     if (c->cfg.steps_per_launch > 0) return c->cfg.steps_per_launch;
     if (c->cfg.shape_given) return 1;
-    const SweepShape sh = sweep_shape(c->storage, c->g.ly);
-    if (!sweep_supported(c->storage, c->g, c->bc.view) || (uint64_t)c->g.lx * sh.ntiles < 256) return 0;
+    if (!sweep_supported(c->storage, c->g, c->bc.view) || !sweep_pays(c, c->bc.view, 0)) return 0;
     if (c->g.lx >= 4096 && three_steps_pay(c->storage, (c->g.ly + 63) / 64) &&
         sweepk_supported(c->storage, c->g, c->bc.view, 3))
         return 3;
@@ -528,18 +531,17 @@ static const RunPlan &run_plan(lbm_ctx *c) {
     // The pressure fix reaches K rows to each side of the periodic seam in K
     // steps.  A lattice that was given no launch setting sweeps K steps at once
     // as if it had no fix, and puts those 2 K rows right from the same source.
-    // The seam's launch costs 11 us, so it pays from a size on (us a step, one
-    // step per launch / sweep and seam: FP64 2048x2048 107 / 80, 4096x1000 106 /
-    // 61, 1500x1500 58 / 47, 1100x1000 25.9 / 24.5; FP32 2048x2048 48 / 38,
-    // 4096x1000 51 / 39, 1500x1500 25.8 / 24.1, 2048x1024 24.1 / 24.5; FP16
-    // 3000x2048 43 / 39, 2048x2048 31.6 / 30.0, 4096x1000 33 / 34).
+    // The seam's launch costs 11 us, so it pays where the sweep gains more (us a
+    // step, one step per launch / sweep and seam: FP64 2048x2048 107 / 73,
+    // 1500x1500 58 / 47, 300x4000 26.8 / 23.7, 1030x1030 24.4 / 27.6, 4000x300
+    // 27.4 / 31.4; FP32 2048x2048 47 / 38, 1100x2060 25.7 / 31; FP16 5000x900 31 /
+    // 26.5, 2048x2048 27.2 / 28.0).
     p.nofix = c->bc.view;
     p.nofix.flags &= ~(uint32_t)kProgPressure;
-    if (p.K == 0 && free && (c->bc.view.flags & kProgPressure) && c->g.N >= seam_nodes(c->storage)) {
+    if (p.K == 0 && free && (c->bc.view.flags & kProgPressure)) {
         const SweepVShape v = sweepv_shape(c->storage, c->g, p.nofix);
-        const SweepShape sh = sweep_shape(c->storage, c->g.ly);
         const int k = v.K > 0 ? v.K
-                      : sweep_supported(c->storage, c->g, p.nofix) && (uint64_t)c->g.lx * sh.ntiles >= 256 ? 2 : 0;
+                      : sweep_supported(c->storage, c->g, p.nofix) && sweep_pays(c, p.nofix, 11) ? 2 : 0;
         if (seam_supported(k, c->g)) {
             p.seam = k;
             p.v = v;

@@ -1,0 +1,40 @@
+// Which of the kernels with the same results a run takes: times of their
+// launches, from measurements on MI355X, compared.  Plain C++ (no HIP), so that
+// the rules can be tested on the host.
+#pragma once
+
+#include <stdint.h>
+
+#include "lbm_types.h"
+
+namespace lbm {
+
+// Time of a one-step launch among others, us.  Fitted to channels and boxes of
+// 500 to 7 million nodes (within 10 % from ly = 30 on, low rather than high): the
+// launch, 4.4 us with a boundary program and 3.3 without, and the planes read
+// and written at 7.9 TB/s (FP64), 8.2 to 10 (FP32, faster below 36 MB) and 6.5
+// (FP16, whose arithmetic is that of FP32); above 240 MB it is slower than this.
+double step_us(int storage, const Geom &g, bool program);
+
+// Time of a two-step launch of whole rows or column tiles, us: rounds of
+// `resident` row ranges of `rows` rows each.  A block walks its rows one after
+// another, so a range costs its rows and about three more (the halo rows and the
+// first loads), 3.7 to 5.1 us each whatever the storage, by the waves and columns
+// per thread of the block; 0.65 (FP64 0.7) of that without a boundary program.
+// Of blocks of five and of ten waves a CU holds one less than the runtime says
+// (five waves: two, not three, in FP64 and five, not six, else; ten: two, not
+// three), and the ranges left over start late: rows of 300 columns in FP16 take
+// 3.7 us each with 1250 ranges on 1536 places and 4.9 with 1397.
+double sweep2_us(int storage, const Geom &g, bool program, const SweepShape &sh, int rows, int resident);
+
+// Whether the library's own choice is two steps per launch, with extra_us a
+// launch on top (the rows that a pressure fix reaches).  us a step, one step per
+// launch / two, channels: FP16 400x1030 6.8 / 10.4, 1600x1030 15.0 / 19.6,
+// 520x640 6.3 / 8.1, 1332x284 6.9 / 8.2, 3300x400 14.9 / 12.6; FP32 300x1100 6.6 / 8.1, 400x900 6.7 /
+// 6.6, 1100x1800 22.6 / 21.1; FP64 270x1030 9.4 / 10.9, 1200x514 16.1 / 15.2.
+// Over 753 lattices of all storages this rule loses 3 % on one and nothing on the
+// others, and leaves 5 to 20 % on 39.
+bool two_steps_pay(int storage, const Geom &g, bool program, const SweepShape &sh, int rows, int resident,
+                   double extra_us);
+
+}  // namespace lbm
