@@ -115,6 +115,8 @@ namespace lbm {
 struct RunPlan {
     bool ready = false;
     int K = 1;            // steps per launch asked for, or the library's choice; 0: tiles, the seam path or single steps
+    bool tile_ready = false;
+    bool free = false;    // tiles and sweeps of adjacent columns may be taken
     TileShape tile;       // K = 0: no tiles
     int seam = 0;         // steps of a sweep that the pressure fix's rows are put right after; 0: not taken
     BcView nofix;         // the boundary without the fix, for those sweeps
@@ -140,6 +142,7 @@ struct lbm_ctx {
     double *sums = nullptr;
     LaunchCfg cfg;
     uint8_t *codes8 = nullptr;  // bc.view.codes8
+    int64_t single_steps = 0;  // launched by lbm_run
     RunPlan plan;  // (cleared with each change of boundary or settings)
     bool stage_eq = false;  // pending: stage_f is the equilibrium of stage_rho and stage_u
 };
@@ -525,9 +528,8 @@ static const RunPlan &run_plan(lbm_ctx *c) {
     // Small lattices: several steps per launch on tiles.  One step per launch
     // and row counts, column tiles or another launch shape than the default
     // (the row sweep takes its block order and stores) keep their kernels.
-    const bool free = p.K != 1 && default_shape(c->cfg) && c->cfg.sweep_rows == 0 && c->cfg.sweep_tile == 0 &&
+    const bool free = p.free = p.K != 1 && default_shape(c->cfg) && c->cfg.sweep_rows == 0 && c->cfg.sweep_tile == 0 &&
                       c->cfg.sweep_v == 0;
-    if (free) p.tile = tile_shape(c->storage, c->g, c->bc.view);
     // The pressure fix reaches K rows to each side of the periodic seam in K
     // steps.  A lattice that was given no launch setting sweeps K steps at once
     // as if it had no fix, and puts those 2 K rows right from the same source.
@@ -556,6 +558,11 @@ static const RunPlan &run_plan(lbm_ctx *c) {
     return p;
 }
 
+// The search for a tiling takes about 10 us, which some steps on tiles win back:
+// a run that comes to fewer since the context was made, this one included, goes
+// without (a new 300x300 FP64 lattice's first two steps: 24 us, 54 with a search).
+constexpr int64_t kTileSearchSteps = 4;
+
 // The kernel of a run's next launch with `left` steps to go, and its steps.
 struct Launch {
     int kernel, steps;
@@ -564,7 +571,14 @@ static Launch next_launch(lbm_ctx *c, int64_t left) {
     if (c->phase == kPending) return {LBM_LAUNCH_FIRST, 1};
     if (left < 2) return {LBM_LAUNCH_STEP, 1};
     const RunPlan &p = run_plan(c);
-    if (p.tile.K > 0) return {LBM_LAUNCH_TILE, (int)std::min<int64_t>(p.tile.K, left)};
+    if (p.free && !p.tile_ready && c->single_steps + left >= kTileSearchSteps) {
+        c->plan.tile = tile_shape(c->storage, c->g, c->bc.view);
+        c->plan.tile_ready = true;
+    }
+    if (p.tile.K > 0) {
+        const int k = (int)std::min<int64_t>(p.tile.K, left);
+        if (k == p.tile.K || tile_steps_pay(c->storage, c->g, c->bc.view, p.tile, k)) return {LBM_LAUNCH_TILE, k};
+    }
     if (p.seam > 0) {
         if (left >= p.seam) return {p.seam == 2 ? LBM_LAUNCH_SWEEP2_SEAM : LBM_LAUNCH_SWEEPV_SEAM, p.seam};
         return {LBM_LAUNCH_STEP, 1};
@@ -711,6 +725,7 @@ int lbm_run(lbm_ctx *c, double omega, int64_t nsteps) {
                                            c->stream, nullptr),
                               "fused step kernel");
         }
+        if (l.kernel == LBM_LAUNCH_STEP) c->single_steps++;
         if (l.kernel != LBM_LAUNCH_FIRST) c->cur ^= 1;  // (the first collision writes planes[cur])
         c->steps += l.steps;
         left -= l.steps;

@@ -27,6 +27,7 @@
 #include <type_traits>
 
 #include "lbm_launch.h"
+#include "lbm_plan.h"
 #include "lbm_rowlayout.h"
 
 namespace lbm {
@@ -2374,8 +2375,6 @@ struct TileLds {
     }
 };
 
-constexpr int tile_threads(size_t elem, bool pressure) { return elem == 8 ? (pressure ? 512 : 768) : (pressure ? 768 : 1024); }
-
 template <class S, bool kPressure>
 __global__ __launch_bounds__(tile_threads(sizeof(S), kPressure)) void k_tile(TileParams<S> p) {
     using C = typename Io<S>::C;
@@ -3163,6 +3162,15 @@ hipError_t launch_fused(int storage, const Geom &g, const StateView &st, int src
 
 namespace {
 
+// Compute units of the current device (256 if the runtime cannot say).
+int compute_units() {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        cus = 256;
+    return cus;
+}
+
 constexpr size_t kLdsLimit = 160 * 1024;
 
 size_t sweep_lds_for(int storage, uint32_t ly, uint32_t nclasses, uint32_t rows) {
@@ -3598,54 +3606,13 @@ hipError_t launch_sweepv(int storage, const SweepVShape &sh, const Geom &g, cons
     return hipErrorInvalidValue;
 }
 
-// Where it pays: up to 2^18 nodes in FP64 and 3 * 2^16 in FP32 and FP16 (time
-// of a step, this kernel / the faster of one and two steps per launch, channels
-// with walls: FP64 300x300 2.33 / 4.4 us, 420x180 2.57 / 5.0, 700x250 4.6 / 6.4,
-// 500x500 7.9 / 8.2, 5000x50 8.1 / 10.6, 700x700 14.0 / 11.8; FP32 420x180 1.8 /
-// 4.5, 700x250 2.8 / 4.5, 500x500 5.9 / 5.2, 700x700 9.7 / 7.7; 20x30 FP64 1.6 /
-// 4.1, FP16 50x97 with the pressure fix 1.8 / 4.4).  Larger lattices need several
-// rounds of blocks, whose halos cost more than the launches they save.
-// Time of a launch, from the kernel's own timings on one round of blocks: 3.3
-// us of launch, first loads and last stores, and for each step 0.35 us of
-// barrier and LDS latency and, for every wave that a SIMD holds, 0.4 us of
-// arithmetic in FP64 or 0.12 us in FP32 and FP16.
 TileShape tile_shape(int storage, const Geom &g, const BcView &bc) {
-    TileShape best;
-    const bool f64 = storage == LBM_STORE_F64;
-    if (bc.codes && bc.nclasses > kSweepMaxClasses) return best;
-    if (g.N > (f64 ? 1u << 18 : 3u << 16)) return best;
-    const bool pressure = (bc.flags & kProgPressure) != 0;
-    const size_t elem = f64 ? 8 : (storage == LBM_STORE_F32 ? 4 : 2);
-    const uint32_t tmax = (uint32_t)tile_threads(elem, pressure);
-    const uint32_t wmax = f64 ? (pressure ? 8 : 12) : (pressure ? 12 : 24);  // resident waves a CU (registers)
-    double t_best = 1e30;  // us a step
-    for (int K = 1; K <= 8; K++) {
-        // what a node depends on may cross the seam of the fix only once
-        if (pressure && (uint32_t)K + 4 > g.lx) break;
-        const uint32_t hx = 2 * (K - 1 + (pressure ? 2 : 0)), hy = 2 * (K - 1);  // both sides
-        for (uint32_t ty = 1; ty <= g.ly && ty + hy <= 64 && (ty + hy) * (hx + 1) <= tmax; ty++) {
-            const uint32_t ny = (g.ly + ty - 1) / ty;
-            if (ty < g.ly && (g.ly + ty) / (ty + 1) == ny) continue;  // as many tiles as a wider one
-            for (uint32_t tx = std::min(g.lx, tmax / (ty + hy) - hx); tx >= 1; tx--) {
-                const uint32_t nx = (g.lx + tx - 1) / tx;
-                const uint32_t waves = ((tx + hx) * (ty + hy) + 63) / 64;
-                const uint32_t tiles = nx * ny;
-                if (tiles > 4096) break;  // ever more with fewer rows
-                const uint32_t fit = std::max(1u, wmax / waves);  // blocks a CU
-                const uint32_t rounds = (tiles + 256 * fit - 1) / (256 * fit);
-                const uint32_t per_cu = std::min(fit, (tiles + 255) / 256);
-                const double step = 0.35 + (f64 ? 0.4 : 0.12) * ((waves * per_cu + 3) / 4);
-                const double t = rounds * (3.3 + K * step) / K;
-                if (t < t_best) {
-                    t_best = t;
-                    best.K = K;
-                    best.tx = tx;
-                    best.ty = ty;
-                }
-            }
-        }
-    }
-    return best;
+    if (bc.codes && bc.nclasses > kSweepMaxClasses) return TileShape{};
+    return pick_tile(storage, g, bc.codes != nullptr, (bc.flags & kProgPressure) != 0, compute_units());
+}
+
+bool tile_steps_pay(int storage, const Geom &g, const BcView &bc, const TileShape &sh, int k) {
+    return tile_pays(storage, g, bc.codes != nullptr, (bc.flags & kProgPressure) != 0, compute_units(), sh, k);
 }
 
 namespace {

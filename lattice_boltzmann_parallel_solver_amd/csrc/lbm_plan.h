@@ -37,4 +37,27 @@ double sweep2_us(int storage, const Geom &g, bool program, const SweepShape &sh,
 bool two_steps_pay(int storage, const Geom &g, bool program, const SweepShape &sh, int rows, int resident,
                    double extra_us);
 
+// Most threads of a block of the tile kernel (its registers).
+constexpr int tile_threads(size_t elem, bool pressure) { return elem == 8 ? (pressure ? 512 : 768) : (pressure ? 768 : 1024); }
+
+// Time of a launch of k steps of the tile kernel among others, us: the launch
+// with its first loads and last stores, 3 to 4 us for each further round of
+// blocks, and for every step of a round a barrier and LDS part and one for every
+// wave that a SIMD holds.  Fitted to 870 runs of 500 to 2^18 nodes, all storages
+// and kinds of boundary: within 7 % on nine of ten.
+double tile_us(int storage, const Geom &g, bool program, bool pressure, int cus, const TileShape &sh, int k);
+
+// The tiling with the least time a step, K = 0 where single steps are as fast (or
+// above 2^18 nodes in FP64, 3 * 2^16 in FP32 and FP16, where they always were).
+// us a step, single steps / tiles: FP64 channels 300x300 6.0 / 2.3, 203x494 6.1 /
+// 3.8, with the pressure fix 551x412 8.2 / 13.3, 1403x170 9.1 / 12.2, 56x838 5.3 /
+// 3.8; FP32 652x294 with the fix 5.9 / 5.3; FP16 1656x115 5.8 / 6.6.  Takes about
+// 10 us.
+TileShape pick_tile(int storage, const Geom &g, bool program, bool pressure, int cus);
+
+// Whether a launch of k <= sh.K steps of that tiling beats single steps (its
+// halos are those of k steps, its rounds of blocks those of the tiling: FP32
+// 67x2897, us a step with 2, 3 and 4: 7.3, 5.6 and 4.7, single steps 5.7).
+bool tile_pays(int storage, const Geom &g, bool program, bool pressure, int cus, const TileShape &sh, int k);
+
 }  // namespace lbm

@@ -135,3 +135,88 @@ def test_two_steps_need_rows_and_residency(tmp_path):
     run = _driver(tmp_path, DRIVER)
     assert run([(1, 8192, 2048, 2048, 1, 2, 1, 1024, 32, 256, 0), (1, 8192, 2048, 2048, 1, 2, 1, 1024, 32, 0, 0),
                 (1, 8192, 2048, 2048, 1, 2, 1, 1024, 0, 256, 0)]) == ["1", "0", "0"]
+
+
+TILE_DRIVER = r"""
+#include <cstdio>
+
+#include "lbm_plan.h"
+
+int main() {
+    int storage, program, pressure, cus, K, k;
+    unsigned lx, ly, pitch, tx, ty;
+    // K = 0: pick a tiling; else the time of k steps of the given one
+    while (std::scanf("%d %u %u %u %d %d %d %d %u %u %d", &storage, &lx, &ly, &pitch, &program, &pressure, &cus, &K, &tx, &ty,
+                      &k) == 11) {
+        lbm::Geom g;
+        g.lx = lx;
+        g.ly = ly;
+        g.N = lx * ly;
+        g.pitch = pitch;
+        lbm::TileShape sh;
+        sh.K = K;
+        sh.tx = tx;
+        sh.ty = ty;
+        if (K == 0) sh = lbm::pick_tile(storage, g, program != 0, pressure != 0, cus);
+        const int n = K == 0 ? sh.K : k;
+        std::printf("%d %u %u %.3f %d\n", sh.K, sh.tx, sh.ty,
+                    n > 0 ? lbm::tile_us(storage, g, program != 0, pressure != 0, cus, sh, n) : 0.0,
+                    n > 0 ? (int)lbm::tile_pays(storage, g, program != 0, pressure != 0, cus, sh, n) : 0);
+    }
+    return 0;
+}
+"""
+
+# storage, lx, ly, boundary (0: none, 1: walls, 2: with the pressure fix), tiling (steps, rows,
+# columns) and us of a launch of 2 steps and of all of them, us of a single step
+TILED = [
+    ("f64", 203, 494, 1, (4, 42, 10), 10.9, 15.2, 6.1), ("f64", 51, 1555, 1, (5, 28, 13), 10.0, 17.0, 5.9),
+    ("f64", 551, 412, 2, (2, 79, 4), 26.5, 26.5, 8.2), ("f64", 1403, 170, 2, (2, 67, 5), 24.4, 24.4, 9.1),
+    ("f64", 56, 838, 2, (4, 29, 7), 11.0, 15.2, 5.3), ("f32", 194, 545, 1, (6, 34, 13), 9.5, 14.5, 5.1),
+    ("f32", 652, 294, 2, (4, 30, 13), 16.5, 21.1, 5.9), ("f32", 67, 2897, 1, (4, 36, 12), 14.6, 19.0, 5.7),
+    ("f16", 357, 363, 1, (5, 40, 13), 9.0, 13.5, 5.4), ("f16", 1656, 115, 2, (3, 77, 5), 18.0, 19.9, 5.8),
+    ("f16", 88, 2278, 0, (4, 44, 8), 9.2, 17.4, 4.2),
+]
+
+
+def _tile_row(st, lx, ly, kind, K=0, tx=0, ty=0, k=0, cus=256):
+    return (STORAGE[st], lx, ly, -(-ly // LINE[st]) * LINE[st], int(kind > 0), int(kind == 2), cus, K, tx, ty, k)
+
+
+def test_tile_times_and_where_they_pay(tmp_path):
+    run = _driver(tmp_path, TILE_DRIVER)
+    for case in TILED[:-1]:
+        st, lx, ly, kind, (K, tx, ty), two, full, one = case
+        for k, us in ((2, two), (K, full)):
+            _, _, _, t, pays = run([_tile_row(st, lx, ly, kind, K, tx, ty, k)])[0].split()
+            assert abs(float(t) / us - 1) < 0.2, (case, k)
+            if us > 1.05 * k * one:
+                assert pays == "0", (case, k)
+            if us < 0.75 * k * one:
+                assert pays == "1", (case, k)
+
+
+def test_tilings_fit_their_blocks_and_beat_single_steps(tmp_path):
+    run = _driver(tmp_path, TILE_DRIVER)
+    import random
+
+    r = random.Random(4)
+    cases = [(st, lx, ly, kind) for st in STORAGE for kind in (0, 1, 2)
+             for lx, ly in [(1, 1), (1, 700), (700, 1), (5, 60000), (60000, 4), (8, 8), (512, 512), (384, 512), (300, 300),
+                            (551, 412), (1403, 170), (513, 512)] + [(r.randint(1, 900), r.randint(1, 900)) for _ in range(60)]]
+    none = 0
+    for (st, lx, ly, kind), line in zip(cases, run([_tile_row(*c) for c in cases])):
+        K, tx, ty, _, pays = line.split()
+        K, tx, ty = int(K), int(tx), int(ty)
+        if K == 0:
+            none += 1
+            continue
+        assert pays == "1" and lx * ly <= (1 << 18 if st == "f64" else 3 << 16)
+        p = kind == 2
+        limit = (512 if p else 768) if st == "f64" else (768 if p else 1024)
+        assert 1 <= tx <= lx and 1 <= ty <= ly and 2 <= K <= 8
+        assert (tx + 2 * (K - 1 + (2 if p else 0))) * (ty + 2 * (K - 1)) <= limit
+        assert not p or K + 4 <= lx
+    assert 0 < none < len(cases) // 2
+    assert run([_tile_row("f64", 551, 412, 2)])[0].startswith("0 ")   # 8.2 us a step, on tiles 13.3
+    assert run([_tile_row("f64", 1403, 170, 2)])[0].startswith("0 ")  # 9.1 and 12.2
