@@ -156,6 +156,32 @@ int batch_spread_rows(int rows, int threads, int k, bool f64, int64_t rows_total
     return (int)std::min<int64_t>(rows, std::max<int64_t>(2, spread));
 }
 
+bool batch_spread_pays(const std::vector<BatchGroup> &groups, int lanes, int cus, bool f64) {
+    if (groups.empty() || lanes < 1) return false;
+    std::vector<const BatchGroup *> order;
+    for (const BatchGroup &g : groups) order.push_back(&g);
+    std::sort(order.begin(), order.end(), [](const BatchGroup *a, const BatchGroup *b) { return a->nodes > b->nodes; });
+    const size_t nl = std::min(groups.size(), (size_t)lanes);
+    // row iterations of a step pair: of the longest lane, or of all waves
+    auto pair_time = [&](bool spread) {
+        std::vector<int64_t> load(nl, 0);
+        std::vector<double> chain(nl, 0.0);
+        double work = 0;
+        for (const BatchGroup *g : order) {
+            const int rows = std::max(1, spread ? g->spread : g->rows);
+            const double it = g->k == 3 ? (rows + 6) * 2 / 3.0 : rows + 3;
+            double blocks = 0;
+            for (uint32_t lx : g->lx) blocks += (lx + (uint32_t)rows - 1) / (uint32_t)rows;
+            work += blocks * g->waves * it * (g->k == 3 ? 1.6 : 1.0);
+            const size_t l = (size_t)(std::min_element(load.begin(), load.end()) - load.begin());
+            load[l] += g->nodes;
+            chain[l] += it;
+        }
+        return std::max(*std::max_element(chain.begin(), chain.end()), work / (std::max(cus, 1) * (f64 ? 16.0 : 32.0)));
+    };
+    return pair_time(true) < 0.95 * pair_time(false);
+}
+
 bool batch_three_steps_fill(int64_t rows_total, int cus) { return rows_total / (4 * (int64_t)std::max(cus, 1)) >= 8; }
 
 }  // namespace lbm

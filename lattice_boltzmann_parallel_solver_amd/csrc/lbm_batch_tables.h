@@ -94,10 +94,31 @@ int batch_group_rows(int threads, int k, int base_rows, bool rows_auto, int64_t 
 // the whole batch 16 blocks a CU (8 of 512 threads or more, half of both in
 // FP64; 6 of three steps), but 2.  120 steps of seeded channels, FP32, two / three
 // steps per launch, ms before -> after: 20 channels 7.4 -> 6.2 / 6.8 -> 6.0 (another
-// draw 9.9 -> 8.0 / 10.0 -> 8.2), 12 7.1 -> 4.3 / 6.6 -> 4.7, 8 4.9 -> 3.2; FP64 20
-// channels 15.0 -> 13.9, 10 8.3 -> 7.6 (and 10.4 at the FP32 counts).  At twice
-// as many blocks FP32 lost again (7.5 / 7.1).  Large batches keep their counts.
+// draw 9.9 -> 8.0 / 10.0 -> 8.2), 12 7.1 -> 4.3 / 6.6 -> 4.7; FP64 20 channels 15.0 ->
+// 13.9, 10 8.3 -> 7.6 (and 10.4 at the FP32 counts).  At twice as many blocks
+// FP32 lost again (7.5 / 7.1).  Large batches keep their counts, and so does
+// every batch where batch_spread_pays says no.
 int batch_spread_rows(int rows, int threads, int k, bool f64, int64_t rows_total, int cus);
+
+// One group of a batch's launches: its lattices' rows, waves of a block, steps per
+// launch, nodes, and the rows per block without and with batch_spread_rows.
+struct BatchGroup {
+    uint32_t waves = 0;
+    int k = 2;
+    int64_t nodes = 0;
+    std::vector<uint32_t> lx;
+    int rows = 0, spread = 0;
+};
+
+// Whether the smaller counts are the faster ones: they shorten the chain of row
+// iterations of the groups that follow one another on a side stream (largest
+// group onto the least loaded of `lanes`), and cost halo rows where the GPU's
+// waves (32 a CU, 16 in FP64, 20 with three steps) are all taken already.  The
+// time of a step pair is the longer of the two, in row iterations.  Measured time
+// with the smaller counts over that without, seeded channels, against this
+// rule's: FP64 8 channels 1.14 / 1.43, 6 1.09 / 1.08, another 6 0.85 / 0.71, 10 0.83
+// / 0.67; FP32 8 channels 1.11 / 1.31, 4 1.10 / 1.16, 10 0.67 / 0.45, 26 0.71 / 0.44.
+bool batch_spread_pays(const std::vector<BatchGroup> &groups, int lanes, int cus, bool f64);
 
 // With automatic rows, three steps per launch only where the batch's rows
 // make at least 8 per block at four blocks per CU.

@@ -1253,6 +1253,22 @@ int batch_run_sweep(lbm_batch *b, int64_t nsteps) {
         }
         wide_rows = pick_wide_rows(wide, cus, 128, 3);
     }
+    // rows per block of each group: fewer where that pays for the batch
+    std::vector<BatchGroup> gr(buckets.size());
+    for (size_t i = 0; i < buckets.size(); i++) {
+        const Bucket &bk = buckets[i];
+        gr[i].waves = bk.threads / 64;
+        gr[i].k = bk.k;
+        gr[i].rows = gr[i].spread =
+            batch_group_rows((int)bk.threads, bk.k, b->sweep_rows, b->rows_auto, rows_total, cus, wide_rows);
+        if (b->rows_auto && !(bk.k == 2 && bk.threads >= 512 && wide_rows > 0))
+            gr[i].spread = batch_spread_rows(gr[i].rows, (int)bk.threads, bk.k, b->storage == LBM_STORE_F64, rows_total, cus);
+        for (int j : bk.members) {
+            gr[i].lx.push_back(b->ctxs[j]->g.lx);
+            gr[i].nodes += b->ctxs[j]->g.N;
+        }
+    }
+    const bool spread = b->rows_auto && batch_spread_pays(gr, (int)kBatchLanes, cus, b->storage == LBM_STORE_F64);
     // tables: sweep jobs per bucket and pair parity with their block tables,
     // then the one-step jobs' records for the two steps of a pair
     std::vector<std::pair<int, uint32_t>> ilv;  // (job, rows) in the interleaved row order
@@ -1269,11 +1285,7 @@ int batch_run_sweep(lbm_batch *b, int64_t nsteps) {
             // three-step groups at 8, 16, 24, 32 and 48 rows: 132, 143, 147,
             // 149 and 148 GLUPS)
             LaunchCfg cfg = c->cfg;
-            cfg.sweep_rows =
-                batch_group_rows((int)bk.threads, bk.k, b->sweep_rows, b->rows_auto, rows_total, cus, wide_rows);
-            if (b->rows_auto && !(bk.k == 2 && bk.threads >= 512 && wide_rows > 0))
-                cfg.sweep_rows = batch_spread_rows(cfg.sweep_rows, (int)bk.threads, bk.k, b->storage == LBM_STORE_F64,
-                                                   rows_total, cus);
+            cfg.sweep_rows = spread ? gr[bi].spread : gr[bi].rows;
             uint32_t rows = (uint32_t)sweep_rows_for(c->g, cfg, 0);
             // the three-step kernel needs two rows in every block; the same
             // tables also serve its two-step launches
