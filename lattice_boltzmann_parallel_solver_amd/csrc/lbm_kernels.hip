@@ -2765,8 +2765,7 @@ __global__ __launch_bounds__(kBlock) void k_stream_aos(const T *__restrict__ in,
 // 331, 321 us: the halo rows come from L2, and short ranges keep the rows that
 // run at once close in memory), fewer where the lattice has not 768 row ranges
 // (three resident blocks a CU) of them: there the launch is latency.
-// 4200x1800: 800 -> 307 us a step (4.7 TB/s of the 192 bytes a node), 20x30:
-// 58 -> 18 us a call.
+// 4200x1800: 800 -> 307 us a step (4.7 TB/s of the 192 bytes a node).
 // ---------------------------------------------------------------------------
 struct StepAosParams {
     const double *f, *rho, *u;
@@ -2958,6 +2957,105 @@ __global__ __launch_bounds__(kBlock, 3) void k_step_aos(StepAosParams p) {
 #pragma unroll
     for (uint32_t k = 0; k < 12; k++) buf_store(none, lane * 8, 0.0);
     for (uint32_t it = 2; it < R + 2; it++) body(it, Flag<true>{});
+}
+
+// The same step for rows of up to 62 columns, of which a strip makes one wave at
+// most, with a lane of 64 for each column (7 columns: 9 lanes with the halo, and
+// fewer bytes in flight the fewer there are).  A block takes consecutive nodes
+// instead, whatever rows they lie in: each thread collides one, and those with 2 ly
+// - 1 nodes on either side (as far as a neighbour's index lies away, the wrap along
+// y included) stream and store theirs.  Bound by memory: 4 million nodes take 147
+// us with one column, 155 with 3, 157 with 16, 181 with 62 (5.2 to 4.2 TB/s of the
+// 192 bytes a node); in strips 6940, 3621, 717 and 226, and 2867, 1186, 474 and 502
+// through a context's planes.  600 nodes: as fast as in strips.  Results and
+// arithmetic are the other kernel's.
+constexpr uint32_t kFlatBlock = 512;
+constexpr uint32_t kFlatColumns = 62;
+
+__global__ __launch_bounds__(kFlatBlock) void k_step_aos_flat(StepAosParams p) {
+#pragma clang fp contract(off)
+    // collided populations 1 to 8, then the records of the stored nodes
+    __shared__ double ex[9 * kFlatBlock];
+    const uint32_t t = threadIdx.x, lx = p.lx, ly = p.ly, N = lx * ly, H = 2 * ly - 1;
+    const uint32_t o0 = xcd_block(blockIdx.x, gridDim.x) * p.W;  // first node stored
+    int64_t at = (int64_t)o0 + t - H;  // periodic
+    if (at < 0) at += N;
+    else if (at >= N) at -= N;
+    if (at < 0 || at >= N) at = (int64_t)(((uint64_t)o0 + t + (uint64_t)N * H - H) % N);  // (fewer nodes than a block has)
+    const uint32_t n = (uint32_t)at;
+    const uint32_t x = n / ly, y = n - x * ly;
+    const bool pressure = (p.bc.flags & kProgPressure) != 0;
+    auto load = [&](size_t m, double f[9], double &rho, double &ux, double &uy) {
+#pragma unroll
+        for (int i = 0; i < 9; i++) f[i] = p.f[m * 9 + i];
+        rho = p.rho[m];
+        ux = p.u[2 * m];
+        uy = p.u[2 * m + 1];
+    };
+    double s[9];
+    {
+        double f[9], e[9], rho, ux, uy;
+        load(n, f, rho, ux, uy);
+        feq_f64(rho, ux, uy, e);
+#pragma unroll
+        for (int i = 0; i < 9; i++) s[i] = f[i] + (e[i] - f[i]) * p.omega;
+    }
+    if (pressure && (x == 0 || x == lx - 1)) {
+        auto fix = [&](uint32_t from, double rho_fix, uint32_t dirs) {
+            double f[9], e[9], ef[9], rho, ux, uy;
+            load((size_t)from * ly + y, f, rho, ux, uy);
+            feq_f64(rho, ux, uy, e);
+            feq_f64(rho_fix, ux, uy, ef);
+#pragma unroll
+            for (int i = 0; i < 9; i++)
+                if ((dirs >> i) & 1u) s[i] = ef[i] + ((f[i] + (e[i] - f[i]) * p.omega) - e[i]);
+        };
+        if (x == 0) fix(lx - 2, p.bc.rho_in, p.bc.d1);
+        if (x == lx - 1) fix(1 % lx, p.bc.rho_out, p.bc.d2);
+    }
+#pragma unroll
+    for (int d = 1; d < 9; d++) ex[(d - 1) * kFlatBlock + t] = s[d];
+    __syncthreads();
+    const uint32_t cnt = min(p.W, N - o0);
+    const uint32_t j = t - H;  // (wraps before the first stored node)
+    const bool stored = t >= H && j < cnt;
+    double v[9];
+    v[0] = s[0];
+    if (stored) {
+        const int yp = y + 1 == ly ? 1 - (int)ly : 1, ym = y == 0 ? (int)ly - 1 : -1;  // index of y + 1, y - 1, less y's
+#pragma unroll
+        for (int d = 1; d < 9; d++) {
+            const int off = -kCX[d] * (int)ly + (kCY[d] == 1 ? ym : (kCY[d] == -1 ? yp : 0));
+            v[d] = ex[(d - 1) * kFlatBlock + (uint32_t)((int)t + off)];
+        }
+        const uint32_t code = p.bc.codes ? p.bc.codes[n] : 0;
+        if (code) {
+            const uint32_t w = p.bc.classes[code].src;
+#pragma unroll
+            for (int d = 0; d < 9; d++) {
+                const uint32_t kind = (w >> (2 * d)) & 3u;
+                const double k = p.bc.classes[code].k[d];
+                const double own = d == 0 ? s[0] : ex[(kOpp[d] - (d > 0)) * kFlatBlock + t];
+                if (kind == kSrcReflect) v[d] = own - k;
+                else if (kind == kSrcConst) v[d] = k;
+                else if (kind == kSrcOutlet) v[d] = p.f[((size_t)(lx - 2) * ly + y) * 9 + d];
+            }
+        }
+        double rho, jx, jy, ux, uy;
+        moments_f64(v, rho, jx, jy);
+        velocity_f64(rho, jx, jy, ux, uy);
+        p.ro[o0 + j] = rho;
+        p.uo[2 * (size_t)(o0 + j)] = ux;
+        p.uo[2 * (size_t)(o0 + j) + 1] = uy;
+    }
+    __syncthreads();
+    if (stored) {
+#pragma unroll
+        for (int i = 0; i < 9; i++) ex[j * 9 + i] = v[i];
+    }
+    __syncthreads();
+    double *out = p.fo + (size_t)o0 * 9;
+    for (uint32_t i = t; i < cnt * 9; i += kFlatBlock) out[i] = ex[i];
 }
 
 // rho_out, u_out: where the moments are also copied to, or null.
@@ -4055,7 +4153,7 @@ hipError_t launch_load_equilibrium(const double *rho, const double *u, double *f
 hipError_t launch_step_aos(uint32_t lx, uint32_t ly, const BcView &bc, const double *f, const double *rho,
                            const double *u, double omega, double *fo, double *ro, double *uo, hipStream_t s) {
     constexpr uint32_t kMaxW = kBlock - 2;
-    StepAosParams p;
+    StepAosParams p{};
     p.f = f;
     p.rho = rho;
     p.u = u;
@@ -4066,6 +4164,11 @@ hipError_t launch_step_aos(uint32_t lx, uint32_t ly, const BcView &bc, const dou
     p.ly = ly;
     p.bc = bc;
     p.omega = omega;
+    if (ly <= kFlatColumns) {
+        p.W = kFlatBlock - 2 * (2 * ly - 1);
+        hipLaunchKernelGGL(k_step_aos_flat, dim3((lx * ly + p.W - 1) / p.W), dim3(kFlatBlock), 0, s, p);
+        return hipGetLastError();
+    }
     p.strips = (ly + kMaxW - 1) / kMaxW;
     p.W = (ly + p.strips - 1) / p.strips;
     p.strips = (ly + p.W - 1) / p.W;  // every strip holds a column
