@@ -11,6 +11,7 @@ in one kernel; the boundary must be one of this package's boundary objects
 
 from __future__ import annotations
 
+from collections import OrderedDict
 from typing import Callable, Tuple
 
 import numpy as np
@@ -97,6 +98,30 @@ def equilibrium_distr_func(density_func, velocity_field):
     return back(out, kind)
 
 
+# device contexts of the torch-free path of lattice_boltzmann_step, by shape and boundary program
+_STEP_CONTEXTS: "OrderedDict[tuple, object]" = OrderedDict()
+_MAX_CONTEXTS = 4
+
+
+def _step_without_torch(f, density, velocity, omega, prog):
+    """The step on numpy arrays through a context of the C library alone, for
+    programs without torch or with one that sees no device."""
+    from .solver import Lattice
+
+    lx, ly = f.shape[:2]
+    key = (lx, ly, id(prog))
+    ctx = _STEP_CONTEXTS.get(key)
+    if ctx is None or ctx._program is not prog:
+        ctx = Lattice(lx, ly, boundary=prog, storage="f64")
+        _STEP_CONTEXTS[key] = ctx
+        while len(_STEP_CONTEXTS) > _MAX_CONTEXTS:
+            _STEP_CONTEXTS.popitem(last=False)[1].close()
+    _STEP_CONTEXTS.move_to_end(key)
+    ctx.set_state(f, density, velocity)
+    ctx.run(omega, 1)
+    return ctx.state()
+
+
 def lattice_boltzmann_step(f, density, velocity, omega: float,
                            boundary: Callable = None,
                            parallel_communication: Callable = None) -> Tuple:
@@ -122,7 +147,14 @@ def lattice_boltzmann_step(f, density, velocity, omega: float,
     assert tuple(velocity.shape) == (lx, ly, 2), f"velocity must have shape {(lx, ly, 2)}"
     prog = None if boundary is None else boundary.program(lx, ly)
     handle = None if prog is None else prog.handle
-    torch = torch_cuda()
+    try:
+        torch = torch_cuda()
+    except (ImportError, RuntimeError):
+        from .solver import _is_torch
+
+        if _is_torch(f):
+            raise
+        return _step_without_torch(f, density, velocity, float(omega), prog)
     if isinstance(f, torch.Tensor):
         ins = [t.detach() for t in (f, density, velocity)]
         if any(t.device.type != "cuda" for t in ins):
