@@ -430,7 +430,7 @@ int lbm_set_bc(lbm_ctx *c, const lbm_bc_prog *prog) {
     c->plan.ready = false;
     if (prog) {
         LBM_HIP_CHECK(upload_bc(*prog, c->bc), "lbm_set_bc: upload");
-        if (c->bc.view.nclasses <= 256 && sweepv_fits(c->storage, c->g)) {
+        if (sweepv_fits(c->storage, c->g, c->bc.view.nclasses)) {
             LBM_HIP_CHECK(hipMalloc(reinterpret_cast<void **>(&c->codes8), (size_t)c->g.lx * c->g.pitch), "lbm_set_bc: upload");
             LBM_HIP_CHECK(launch_codes8(c->g, c->bc.view.codes, c->codes8, c->stream), "lbm_set_bc: byte codes");
             c->bc.view.codes8 = c->codes8;

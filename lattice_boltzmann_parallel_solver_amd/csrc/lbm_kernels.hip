@@ -3646,8 +3646,8 @@ uint32_t sweepv_waves(int storage, const Geom &g) {
 }
 }  // namespace
 
-bool sweepv_fits(int storage, const Geom &g) {
-    if (storage == LBM_STORE_F16 || sweep_big(storage, g)) return false;
+bool sweepv_fits(int storage, const Geom &g, uint32_t nclasses) {
+    if (storage == LBM_STORE_F16 || sweep_big(storage, g) || nclasses > kSweepMaxClasses) return false;
     const uint32_t waves = sweepv_waves(storage, g);
     return waves >= 7 && waves <= 8 && sweepv_rows(g) >= 12;
 }
@@ -3655,8 +3655,7 @@ bool sweepv_fits(int storage, const Geom &g) {
 SweepVShape sweepv_shape(int storage, const Geom &g, const BcView &bc) {
     SweepVShape sh;
     const uint32_t ncls = bc.chunk ? bc.nclasses : 0;
-    if (!sweepv_fits(storage, g) || (bc.flags & kProgPressure)) return sh;
-    if (ncls > kSweepMaxClasses || (ncls && !bc.codes8)) return sh;
+    if (!sweepv_fits(storage, g, ncls) || (bc.flags & kProgPressure) || (ncls && !bc.codes8)) return sh;
     const bool f64 = storage == LBM_STORE_F64;
     const uint32_t V = f64 ? 2 : 4, waves = sweepv_waves(storage, g);
     sh.rows = sweepv_rows(g);

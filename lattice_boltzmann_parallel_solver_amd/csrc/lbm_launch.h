@@ -60,8 +60,9 @@ hipError_t launch_codes8(const Geom &g, const uint16_t *codes, uint8_t *codes8, 
 // fix, at most 128 classes, state buffers below 4 GiB): the shape, K = 0 where it
 // does not apply or another kernel is faster.  Probe slots as launch_sweepk.
 SweepVShape sweepv_shape(int storage, const Geom &g, const BcView &bc);
-// Whether the lattice's size is one it takes (its boundary tables then need codes8).
-bool sweepv_fits(int storage, const Geom &g);
+// Whether the lattice's size and number of classes are ones it takes (its boundary
+// tables then need codes8).
+bool sweepv_fits(int storage, const Geom &g, uint32_t nclasses);
 hipError_t launch_sweepv(int storage, const SweepVShape &sh, const Geom &g, const StateView &st, int src, const BcView &bc,
                          double omega, const ProbeView &pr, int64_t probe_slot, hipStream_t s);
 // K steps in one launch on tiles held in registers and LDS (small lattices).

@@ -24,7 +24,7 @@ struct BcView {
     uint32_t d1 = 0, d2 = 0;
     uint32_t flags = 0;                    // kProg*
     // codes as bytes, rows `pitch` apart as the state's (with a context's own
-    // tables of at most 256 classes; the pad holds 0)
+    // tables where the sweep of adjacent columns takes them; the pad holds 0)
     const uint8_t *codes8 = nullptr;
 };
 
