@@ -2763,8 +2763,8 @@ __global__ __launch_bounds__(kBlock) void k_stream_aos(const T *__restrict__ in,
 // reflections.  Arithmetic and order are k_collide_first's and k_finalize's.
 // Four rows a block (4200x1800 at 1, 2, 4, 8, 16, 33 rows: 387, 310, 307, 315,
 // 331, 321 us: the halo rows come from L2, and short ranges keep the rows that
-// run at once close in memory), fewer where the lattice has not 768 row ranges
-// (three resident blocks a CU) of them: there the launch is latency.
+// run at once close in memory), fewer where the lattice has not three row ranges a
+// CU (the resident blocks) of them: there the launch is latency.
 // 4200x1800: 800 -> 307 us a step (4.7 TB/s of the 192 bytes a node).
 // ---------------------------------------------------------------------------
 struct StepAosParams {
@@ -3637,7 +3637,7 @@ int sweepk_rows(const Geom &g, int rows, int K) {
 namespace {
 // One block a CU, in the fewest rounds.
 uint32_t sweepv_rows(const Geom &g) {
-    const uint32_t slots = 256, rounds = (g.lx + slots * kSweepMaxRows - 1) / (slots * kSweepMaxRows);
+    const uint32_t slots = (uint32_t)compute_units(), rounds = (g.lx + slots * kSweepMaxRows - 1) / (slots * kSweepMaxRows);
     return (g.lx + rounds * slots - 1) / (rounds * slots);
 }
 uint32_t sweepv_waves(int storage, const Geom &g) {
@@ -3788,7 +3788,8 @@ hipError_t launch_seam(int storage, int K, const Geom &g, const StateView &st, i
     const size_t elem = storage == LBM_STORE_F64 ? 8 : (storage == LBM_STORE_F32 ? 4 : 2);
     const uint32_t ry = (uint32_t)tile_threads(elem, true) / (2 * K + 2 * (K + 1));
     // narrow tiles: one wave a SIMD and the whole GPU, since nothing runs beside
-    sh.ty = std::min(std::min(g.ly, ry - 2 * (K - 1)), std::max(8u, (g.ly + 255) / 256));
+    const uint32_t cus = (uint32_t)compute_units();
+    sh.ty = std::min(std::min(g.ly, ry - 2 * (K - 1)), std::max(8u, (g.ly + cus - 1) / cus));
     return tile_rows(storage, sh, g, st, src, bc, omega, pr, slot, g.lx - K, 2 * K, s);
 }
 
@@ -4171,7 +4172,7 @@ hipError_t launch_step_aos(uint32_t lx, uint32_t ly, const BcView &bc, const dou
     p.strips = (ly + kMaxW - 1) / kMaxW;
     p.W = (ly + p.strips - 1) / p.strips;
     p.strips = (ly + p.W - 1) / p.W;  // every strip holds a column
-    const uint64_t slots = 3 * 256;
+    const uint64_t slots = 3 * (uint64_t)compute_units();
     p.rows = (uint32_t)std::min<uint64_t>(4, std::max<uint64_t>(1, ((uint64_t)lx * p.strips + slots - 1) / slots));
     const uint64_t grid = (uint64_t)((lx + p.rows - 1) / p.rows) * p.strips;
     const unsigned threads = (p.W + 2 + 63) / 64 * 64;
