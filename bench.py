@@ -5,15 +5,16 @@ Workload (the precision configuration of the reference's channel scaled up):
 offset, inlet equilibrium u = (0.1, 0), rho = 1, outlet extrapolation, rigid
 top and bottom walls, nu = 0.1*400/100 (Re = 100) so omega = 1/1.7.
 
-value      : MLUPS of the FP32-deviation step (inputs resident in HBM), two steps
-             per launch (the row-sweep kernel keeps the intermediate step on chip),
-             at the launch shape the library's autotuner picks for this lattice
-             (rows per block of the sweep; config.launch_shape), tuned outside
-             the timed region; --no-autotune times the default shape.
+value      : MLUPS of the FP32-deviation step (inputs resident in HBM), several steps
+             per launch (the row sweeps keep the intermediate steps on chip), at the
+             launch shape the library's autotuner picks for this lattice (setting
+             and rows per block; config.launch_shape), tuned outside the timed
+             region; --no-autotune times the default shape.  The kernels and steps
+             of the launches come from the library (config.launches).
 roofline   : HBM bound; achieved = algorithmic bytes per launch (every population
-             read and written once: 18 accesses x 4 B per node) / average launch
-             time over the timed region (HIP events on the stream the kernels run
-             on); traffic = HBM bytes per launch measured with rocprofv3
+             read and written once: 18 accesses x 4 B per node) x launches / time of
+             the timed region (HIP events on the stream the kernels run on; the
+             shorter launches of a remainder count as launches); traffic = HBM bytes per launch measured with rocprofv3
              FETCH_SIZE/WRITE_SIZE, copy-calibrated
              (profiles/fused_step_8192x2048_hbm_traffic.json).
              single_step_equivalent_gbs: the bandwidth a one-step-per-launch kernel
@@ -34,7 +35,7 @@ three_steps_per_launch: two against three steps per launch (k_sweepk) on an
              8192x1024 FP32 channel (three steps take rows of up to 1024).
 other_workloads_fp64: GPU rates of the shear wave (300x300, its whole 3000
              steps), the 4200x1800 channel and the 2048x2048 Couette and
-             Poiseuille boxes in FP64.
+             Poiseuille boxes in FP64, with the kernel each takes.
 fp64, f16  : the same workload with FP64 populations / FP16 deviation storage,
              two steps per launch (FP64 rows of 2048 split into three column
              tiles); fp64_single_step: FP64 with one step per launch.
@@ -82,6 +83,17 @@ def measured_traffic(storage, steps_per_launch=1):
             return float(json.load(fh)[key]["traffic_bytes"])
     except (OSError, KeyError, ValueError):
         return None
+
+
+def launches(lat, steps):
+    """[kernel, steps per launch, launches] of the timed run(steps), the longest
+    stretch first, as the library says (of a lattice that is running)."""
+    out, left = {}, steps
+    while left > 0:
+        kernel, k = lat.next_launch(left)
+        out[kernel, k] = out.get((kernel, k), 0) + 1
+        left -= k
+    return sorted(([kernel, k, n] for (kernel, k), n in out.items()), key=lambda e: -e[1] * e[2])
 
 
 def omega():
@@ -223,8 +235,8 @@ def three_step_leg(torch, steps=240, ly=1024):
 
 def config_legs(torch):
     """Rates of the other workloads on the GPU, FP64 (the oracle's arithmetic
-    bit for bit), each lattice resident, with the launch mode it supports
-    fastest (two steps per launch except the pressure-driven box):
+    bit for bit), each lattice resident, with a setting of two steps per launch or
+    (the pressure-driven box, which refuses one) the library's own choice:
     the 300x300 shear wave (omega 1, epsilon 0.05) over its whole 3000-step
     run, the 4200x1800 von Karman channel (plate 400 at x = 1050, +1 y offset,
     walls, inlet 0.1, Re 100), the 2048x2048 Couette box (lid 0.05, omega 1)
@@ -257,22 +269,25 @@ def config_legs(torch):
     lat.set_equilibrium(rho, u)
     lat.set_temporal(2)
     sec = timed(lat, 1.0, 3000)
+    kernel, spl, _ = launches(lat, 3000)[0]
     out["shear_wave_300x300"] = {"steps": 3000, "seconds": sec, "mlups": 90000 * 3000 / sec / 1e6,
-                                 "steps_per_launch": 2, "storage": "f64"}
+                                 "steps_per_launch": spl, "kernel": kernel, "storage": "f64"}
     lat.close()
     cases = (("channel_4200x1800", 4200, 1800,
               BU.von_karman_boundary_conditions(4200, 1800, 1.0, U_IN, 400, walls=True, y_offset=1),
-              1.0 / (3.0 * U_IN * 400 / RE + 0.5), U_IN, 2),
-             ("couette_2048x2048", 2048, 2048, BU.couette_flow_boundary_conditions(2048, 2048, 0.05, 1.0), 1.0, 0.0, 2),
+              1.0 / (3.0 * U_IN * 400 / RE + 0.5), U_IN),
+             ("couette_2048x2048", 2048, 2048, BU.couette_flow_boundary_conditions(2048, 2048, 0.05, 1.0), 1.0, 0.0),
              ("poiseuille_2048x2048", 2048, 2048,
-              BU.poiseuille_flow_boundary_conditions(2048, 2048, (1 + 1.5e-3) / 3, (1 - 1.5e-3) / 3), 1.5, 0.0, 1))
-    for name, lx, ly, bc, om, u_x, spl in cases:
+              BU.poiseuille_flow_boundary_conditions(2048, 2048, (1 + 1.5e-3) / 3, (1 - 1.5e-3) / 3), 1.5, 0.0))
+    for name, lx, ly, bc, om, u_x in cases:
         lat = Lattice(lx, ly, boundary=bc, storage="f64", stream=stream)
         equilibrium_at_rest(lat, u_x)
-        lat.set_temporal(spl)
+        if not name.startswith("poiseuille"):
+            lat.set_temporal(2)
         sec = timed(lat, om, 200)
+        kernel, spl, _ = launches(lat, 200)[0]
         out[name] = {"steps": 200, "seconds": sec, "mlups": lx * ly * 200 / sec / 1e6, "steps_per_launch": spl,
-                     "storage": "f64"}
+                     "kernel": kernel, "storage": "f64"}
         lat.close()
     torch.cuda.empty_cache()
     return out
@@ -518,7 +533,7 @@ def main():
     tuned = None
     if args.rows > 0 and lat.steps_per_launch == 2:
         lat.set_temporal(2, args.rows)
-        tuned = {"steps_per_launch": 2, "rows_per_block": args.rows}
+        tuned = {"steps_per_launch_setting": 2, "rows_per_block": args.rows}
     elif not args.no_autotune and args.temporal == 2:
         # the library's autotuner (launch shape, steps per launch and rows per
         # block timed on a scratch lattice of the same shape), outside the timed region
@@ -528,14 +543,13 @@ def main():
         best = W.autotune_lattice(lat, omega(), steps=200)
         lat.steps_per_launch = best[3]
         tuned = {"nodes_per_thread": best[0], "xcd_order": best[1], "nt_stores": best[2],
-                 "steps_per_launch": best[3], "rows_per_block": best[4]}
+                 "steps_per_launch_setting": best[3], "rows_per_block": best[4]}
         torch.cuda.empty_cache()
-    spl = lat.steps_per_launch
-    steps = -(-args.steps // spl) * spl  # whole launches
-    # full FP32 rows take three steps per launch from a setting of two on,
-    # unless rows per block are given (the same results)
-    taken = 3 if spl >= 2 and args.storage == "f32" and not (tuned and tuned["rows_per_block"]) else spl
+    spl, steps = lat.steps_per_launch, args.steps
     ms = time_steps(lat, steps, args.warmup, torch)
+    # (without a warmup the run began with the collision of the loaded state)
+    plan = launches(lat, steps if args.warmup > 0 else steps - 1) or [["step", 1, 0]]
+    kernel, taken, _ = plan[0]
     m, jx, _ = lat.moments_sum()
     assert m == m and abs(m / N - 1.0) < 0.1, "unstable run"
     lat.close()
@@ -543,7 +557,7 @@ def main():
     torch.cuda.empty_cache()
     sec = ms / 1e3
     mlups = N * steps / sec / 1e6
-    launch_s = sec / (steps / taken)
+    launch_s = sec / max(1, sum(n for _, _, n in plan) + (args.warmup == 0))
     # one launch reads and writes every population once, whatever its step count
     bytes_launch = BYTES_PER_NODE[args.storage] * N
     achieved = bytes_launch / launch_s / 1e9
@@ -551,15 +565,16 @@ def main():
     def leg(storage, steps, temporal):
         if steps <= 0:
             return None
-        steps += steps % 2
         lat = build_lattice(storage, torch, temporal)
-        spl_ = lat.steps_per_launch
         ms_ = time_steps(lat, steps, max(20, args.warmup), torch)
+        plan_ = launches(lat, steps)
+        spl_ = plan_[0][1]
         lat.close()
         torch.cuda.empty_cache()
-        ach = BYTES_PER_NODE[storage] * N / (ms_ / 1e3 / (steps / spl_)) / 1e9
+        ach = BYTES_PER_NODE[storage] * N / (ms_ / 1e3 / sum(n for _, _, n in plan_)) / 1e9
         return {"mlups": N * steps / (ms_ / 1e3) / 1e6, "ms_per_step": ms_ / steps, "steps": steps,
-                "steps_per_launch": spl_, "roofline_achieved_gbs": ach, "roofline_frac": ach / HBM_PEAK_GBS,
+                "steps_per_launch": spl_, "kernel": plan_[0][0], "roofline_achieved_gbs": ach,
+                "roofline_frac": ach / HBM_PEAK_GBS,
                 "bytes_per_node_step": BYTES_PER_NODE[storage] // spl_, "traffic": measured_traffic(storage, spl_)}
 
     single = leg(args.storage, args.single_steps, 1) if spl >= 2 else None
@@ -598,12 +613,12 @@ def main():
         "config": {"workload": f"von Karman channel {LX}x{LY}, plate {PLATE} at x={LX // 4} (+1 y offset), "
                                f"rigid walls, inlet u={U_IN}, Re={RE:g}, {args.storage} population storage",
                    "lx": LX, "ly": LY, "storage": args.storage, "omega": omega(), "steps_per_launch": taken,
-                   "launch_shape": tuned or "default",
+                   "launches": plan, "launch_shape": tuned or "default",
                    "parallelism": "single GPU (whole lattice resident)"},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": measured_traffic(args.storage, taken),
-                     "kernel": {1: "k_fused (one step per launch)", 2: "k_sweep2 (two steps per launch)",
-                                3: "k_sweepv (three steps per launch)"}[taken],
+                     "kernel": {"step": "k_fused", "tile": "k_tile"}.get(kernel, "k_" + kernel) +
+                               f" ({taken} step{'s' if taken > 1 else ''} per launch)",
                      "bytes_per_node_launch": BYTES_PER_NODE[args.storage],
                      "bytes_per_node_step": BYTES_PER_NODE[args.storage] // taken,
                      "single_step_equivalent_gbs": mlups * 1e6 * BYTES_PER_NODE[args.storage] / 1e9,
