@@ -122,6 +122,22 @@ def _step_without_torch(f, density, velocity, omega, prog):
     return ctx.state()
 
 
+def _piece_bytes(total: int) -> int:
+    """Bytes of the pieces that `total` bytes of host arrays go through pinned
+    memory in, a multiple of 256.  Each piece costs 20 to 25 us, and the memcpy of
+    one runs beside the transfer of the others: one up to 2.8 MB (160x160: 253 us a
+    call in one, 263 in three, 279 in four), three up to 3.5 MB (180x180: 300, 287,
+    307), then four or more of up to 2 MiB (200x200: 366, 354, 341; 420x300: 1040,
+    833, 842, in eight 866)."""
+    if total <= 2_800_000:
+        piece = total
+    elif total <= 3_500_000:
+        piece = -(-total // 3)
+    else:
+        piece = min(2 << 20, -(-total // 4))
+    return max(256, -(-piece // 256) * 256)
+
+
 def lattice_boltzmann_step(f, density, velocity, omega: float,
                            boundary: Callable = None,
                            parallel_communication: Callable = None) -> Tuple:
@@ -167,12 +183,8 @@ def lattice_boltzmann_step(f, density, velocity, omega: float,
     ins = [np.ascontiguousarray(a, dtype=np.float64) for a in (f, density, velocity)]
     outs = tuple(np.empty(a.shape) for a in ins)
     work = torch.empty(24 * lx * ly, dtype=torch.float64, device="cuda")
-    # four pinned quarters (torch keeps and hands them out again): arrays of up
-    # to 2 MiB go in one piece, since each piece costs 25 us (88x68: 90 us a call
-    # in one, 182 in four), larger ones in four or more (420x180: 649 and 572)
-    total = 96 * lx * ly
-    piece = total if total <= 2 << 20 else min(2 << 20, -(-total // 4))
-    stage = torch.empty(4 * max(256, -(-piece // 256) * 256), dtype=torch.uint8, pin_memory=True)
+    # four pinned quarters (torch keeps and hands them out again)
+    stage = torch.empty(4 * _piece_bytes(96 * lx * ly), dtype=torch.uint8, pin_memory=True)
     check(_lib.load().lbm_step_host(handle, *(a.ctypes.data for a in ins), float(omega), lx, ly,
                                     *(a.ctypes.data for a in outs), work.data_ptr(), stage.data_ptr(), stage.numel(),
                                     stream()))
