@@ -118,6 +118,7 @@ struct RunPlan {
     bool tile_ready = false;
     bool free = false;    // tiles and sweeps of adjacent columns may be taken
     TileShape tile;       // K = 0: no tiles
+    double other_us = 0;  // a step without them
     int seam = 0;         // steps of a sweep that the pressure fix's rows are put right after; 0: not taken
     BcView nofix;         // the boundary without the fix, for those sweeps
     SweepVShape v;        // K = 0: not taken
@@ -142,7 +143,7 @@ struct lbm_ctx {
     double *sums = nullptr;
     LaunchCfg cfg;
     uint8_t *codes8 = nullptr;  // bc.view.codes8
-    int64_t single_steps = 0;  // launched by lbm_run
+    int64_t steps_run = 0;  // by lbm_run, over all states
     RunPlan plan;  // (cleared with each change of boundary or settings)
     bool stage_eq = false;  // pending: stage_f is the equilibrium of stage_rho and stage_u
 };
@@ -494,9 +495,21 @@ int lbm_set_state_equilibrium(lbm_ctx *c, const double *rho, const double *u, in
 // extra_us a launch on top.
 static bool sweep_pays(const lbm_ctx *c, const BcView &bc, double extra_us) {
     const LaunchCfg automatic{1, 1, 0};
-    return two_steps_pay(c->storage, c->g, bc.codes != nullptr, sweep_shape(c->storage, c->g.ly),
-                         sweep2_rows(c->storage, c->g, bc, automatic),
+    return two_steps_pay(c->storage, c->g, bc.codes != nullptr, (bc.flags & kProgOutlet) != 0,
+                         sweep_shape(c->storage, c->g.ly), sweep2_rows(c->storage, c->g, bc, automatic),
                          sweep2_resident_ranges(c->storage, c->g, bc, automatic), extra_us);
+}
+
+// Time of a step without tiles, us.
+static double other_step_us(const lbm_ctx *c, bool sweeps) {
+    const BcView &bc = c->bc.view;
+    const double one = step_us(c->storage, c->g, bc.codes != nullptr);
+    if (!sweeps) return one;
+    const int rows = sweep2_rows(c->storage, c->g, bc, c->cfg);
+    const int resident = sweep2_resident_ranges(c->storage, c->g, bc, c->cfg);
+    if (rows < 1 || resident < 1) return one;
+    return sweep2_us(c->storage, c->g, bc.codes != nullptr, (bc.flags & kProgOutlet) != 0,
+                     sweep_shape(c->storage, c->g.ly), rows, resident) / 2;
 }
 
 // Steps per launch of a run: the caller's, or for a context that was given no
@@ -554,14 +567,15 @@ static const RunPlan &run_plan(lbm_ctx *c) {
     if (free && p.K >= 2) p.v = sweepv_shape(c->storage, c->g, c->bc.view);
     p.sweepk = p.K >= 3 && sweepk_supported(c->storage, c->g, c->bc.view, p.K);
     p.sweep2 = p.K >= 2 && sweep_supported(c->storage, c->g, c->bc.view, c->cfg.sweep_tile, c->cfg.sweep_v);
+    if (free) p.other_us = other_step_us(c, p.sweep2);
     p.ready = true;
     return p;
 }
 
-// The search for a tiling takes about 10 us, which some steps on tiles win back:
-// a run that comes to fewer since the context was made, this one included, goes
-// without (a new 300x300 FP64 lattice's first two steps: 24 us, 54 with a search).
-constexpr int64_t kTileSearchSteps = 4;
+// The search for a tiling takes 10 to 40 us, which 16 steps on tiles win back: a
+// context that has not come to as many, with the run at hand, goes without (a new
+// 300x300 FP64 lattice's first two steps: 23 us, 54 with a search).
+constexpr int64_t kTileSearchSteps = 16;
 
 // The kernel of a run's next launch with `left` steps to go, and its steps.
 struct Launch {
@@ -571,13 +585,13 @@ static Launch next_launch(lbm_ctx *c, int64_t left) {
     if (c->phase == kPending) return {LBM_LAUNCH_FIRST, 1};
     if (left < 2) return {LBM_LAUNCH_STEP, 1};
     const RunPlan &p = run_plan(c);
-    if (p.free && !p.tile_ready && c->single_steps + left >= kTileSearchSteps) {
-        c->plan.tile = tile_shape(c->storage, c->g, c->bc.view);
+    if (p.free && !p.tile_ready && c->steps_run + left >= kTileSearchSteps) {
+        c->plan.tile = tile_shape(c->storage, c->g, c->bc.view, p.other_us);
         c->plan.tile_ready = true;
     }
     if (p.tile.K > 0) {
         const int k = (int)std::min<int64_t>(p.tile.K, left);
-        if (k == p.tile.K || tile_steps_pay(c->storage, c->g, c->bc.view, p.tile, k)) return {LBM_LAUNCH_TILE, k};
+        if (k == p.tile.K || tile_steps_pay(c->storage, c->g, c->bc.view, p.tile, k, p.other_us)) return {LBM_LAUNCH_TILE, k};
     }
     if (p.seam > 0) {
         if (left >= p.seam) return {p.seam == 2 ? LBM_LAUNCH_SWEEP2_SEAM : LBM_LAUNCH_SWEEPV_SEAM, p.seam};
@@ -725,7 +739,7 @@ int lbm_run(lbm_ctx *c, double omega, int64_t nsteps) {
                                            c->stream, nullptr),
                               "fused step kernel");
         }
-        if (l.kernel == LBM_LAUNCH_STEP) c->single_steps++;
+        c->steps_run += l.steps;
         if (l.kernel != LBM_LAUNCH_FIRST) c->cur ^= 1;  // (the first collision writes planes[cur])
         c->steps += l.steps;
         left -= l.steps;

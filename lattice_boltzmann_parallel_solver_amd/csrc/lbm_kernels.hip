@@ -3703,13 +3703,13 @@ hipError_t launch_sweepv(int storage, const SweepVShape &sh, const Geom &g, cons
     return hipErrorInvalidValue;
 }
 
-TileShape tile_shape(int storage, const Geom &g, const BcView &bc) {
+TileShape tile_shape(int storage, const Geom &g, const BcView &bc, double other_us) {
     if (bc.codes && bc.nclasses > kSweepMaxClasses) return TileShape{};
-    return pick_tile(storage, g, bc.codes != nullptr, (bc.flags & kProgPressure) != 0, compute_units());
+    return pick_tile(storage, g, bc.codes != nullptr, (bc.flags & kProgPressure) != 0, compute_units(), other_us);
 }
 
-bool tile_steps_pay(int storage, const Geom &g, const BcView &bc, const TileShape &sh, int k) {
-    return tile_pays(storage, g, bc.codes != nullptr, (bc.flags & kProgPressure) != 0, compute_units(), sh, k);
+bool tile_steps_pay(int storage, const Geom &g, const BcView &bc, const TileShape &sh, int k, double other_us) {
+    return tile_pays(storage, g, bc.codes != nullptr, (bc.flags & kProgPressure) != 0, compute_units(), sh, k, other_us);
 }
 
 namespace {

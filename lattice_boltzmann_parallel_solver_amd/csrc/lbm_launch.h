@@ -67,10 +67,11 @@ hipError_t launch_sweepv(int storage, const SweepVShape &sh, const Geom &g, cons
                          double omega, const ProbeView &pr, int64_t probe_slot, hipStream_t s);
 // K steps in one launch on tiles held in registers and LDS (small lattices).
 // The samples of step s (1-based) go to ring slot probe_slot + s - 1.
-// tile_shape: the fastest tiling of a lattice (K = 0: single steps are as fast);
-// a launch may take fewer steps than its K, where tile_steps_pay says so.
-TileShape tile_shape(int storage, const Geom &g, const BcView &bc);
-bool tile_steps_pay(int storage, const Geom &g, const BcView &bc, const TileShape &sh, int k);
+// tile_shape: the fastest tiling of a lattice (K = 0: what would run otherwise, with
+// other_us a step, is as fast); a launch may take fewer steps than its K, where
+// tile_steps_pay says so.
+TileShape tile_shape(int storage, const Geom &g, const BcView &bc, double other_us);
+bool tile_steps_pay(int storage, const Geom &g, const BcView &bc, const TileShape &sh, int k, double other_us);
 hipError_t launch_tile(int storage, const TileShape &sh, const Geom &g, const StateView &st, int src, const BcView &bc,
                        double omega, const ProbeView &pr, int64_t probe_slot, hipStream_t s);
 // K steps of the rows that the pressure fix reaches in them, lx - K to K - 1

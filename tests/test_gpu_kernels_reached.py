@@ -41,6 +41,8 @@ def _run(lx, ly, storage, kind, steps, settings, probe, capacity, kernel):
     assert lat.next_launch(steps) == ("first", 1)
     lat.run(1.3, 1)
     done, reached = 1, set()
+    if settings is None:
+        assert lat.next_launch(14) == ("step", 1)  # too few steps to look for a tiling
     for upto in (steps // 2, steps):  # two runs, so that remainders come up
         left = upto - done
         if left > 0:
@@ -97,13 +99,13 @@ def test_k_step_sweep_automatic_rows(lx, ly, storage, kind, k):
 
 @pytest.mark.parametrize("k,rows,kernel", [(2, 4, "sweep2"), (3, 4, "sweepk"), (4, 5, "sweepk"), (2, 0, "tile")])
 def test_probe_ring_shorter_than_the_run(k, rows, kernel):
-    _equal(30, 100, "f32", "channel", 23, (k, rows), kernel, capacity=7)
+    _equal(30, 100, "f32", "channel", 43, (k, rows), kernel, capacity=7)
 
 
 @pytest.mark.parametrize("lx,ly,storage,kind", [(20, 30, "f64", "couette"), (64, 32, "f16", "channel"),
                                                 (41, 67, "f32", "poiseuille"), (3, 2, "f64", "couette")])
 def test_tiles(lx, ly, storage, kind):
-    _equal(lx, ly, storage, kind, 12, None, "tile")
+    _equal(lx, ly, storage, kind, 60, None, "tile")
 
 
 def _kernel(lx, ly, storage, kind, temporal, steps):
@@ -160,11 +162,11 @@ def test_a_launch_shape_means_single_steps(shape):
     lat = Lattice(300, 100)
     lat.set_equilibrium(np.ones((300, 100)), np.zeros((300, 100, 2)))
     lat.run(1.0, 1)
-    assert lat.next_launch(9)[0] == "tile"
+    assert lat.next_launch(29)[0] == "tile"
     lat.set_launch(*shape)
     assert lat.next_launch(9) == ("step", 1)
     lat.set_temporal(2)
-    assert lat.next_launch(9)[0] == ("tile" if shape == (1, True, False) else "sweep2")
+    assert lat.next_launch(29)[0] == ("tile" if shape == (1, True, False) else "sweep2")
     lat.close()
 
 
@@ -176,11 +178,11 @@ def test_column_tiles_asked_for_are_kept(lx, ly, tile):
     lat.set_equilibrium(np.ones((lx, ly)), np.zeros((lx, ly, 2)))
     lat.run(1.0, 1)
     lat.set_temporal(2)
-    assert lat.next_launch(9)[0] in ("tile", "sweepv")
+    assert lat.next_launch(29)[0] in ("tile", "sweepv")
     lat.set_sweep_tile(*tile)
-    assert lat.next_launch(9) == ("sweep2", 2)
+    assert lat.next_launch(29) == ("sweep2", 2)
     lat.set_sweep_tile()
-    assert lat.next_launch(9)[0] in ("tile", "sweepv")
+    assert lat.next_launch(29)[0] in ("tile", "sweepv")
     lat.close()
 
 

@@ -31,7 +31,7 @@ int main() {
         sh.v = v;
         sh.ntiles = tiles;
         sh.threads = threads;
-        std::printf("%d\n", (int)lbm::two_steps_pay(storage, g, program != 0, sh, rows, resident, extra));
+        std::printf("%d\n", (int)lbm::two_steps_pay(storage, g, program > 0, program == 2, sh, rows, resident, extra));
     }
     return 0;
 }
@@ -54,11 +54,11 @@ def _driver(tmp_path, text):
     return run
 
 
-# storage, lx, ly, boundary program, columns per thread, column tiles, threads, rows a block, resident
+# storage, lx, ly, boundary program (2: with an outlet), columns per thread, column tiles, threads, rows a block, resident
 # ranges, us a step with one / with two steps per launch
 MEASURED = [
-    ("f32", 1519, 312, 1, 1, 1, 320, 1, 1536, 7.9, 8.8), ("f16", 1332, 284, 1, 1, 1, 320, 1, 1536, 6.9, 8.2),
-    ("f16", 2793, 277, 1, 1, 1, 320, 2, 1536, 10.2, 11.3), ("f64", 1100, 300, 1, 1, 1, 320, 2, 768, 10.8, 14.2),
+    ("f32", 1519, 312, 2, 1, 1, 320, 1, 1536, 7.9, 8.8), ("f16", 1332, 284, 2, 1, 1, 320, 1, 1536, 6.9, 8.2),
+    ("f16", 2793, 277, 2, 1, 1, 320, 2, 1536, 10.2, 11.3), ("f64", 1100, 300, 2, 1, 1, 320, 2, 768, 10.8, 14.2),
     ("f16", 3300, 65, 0, 1, 1, 128, 1, 4096, 5.6, 4.5),
     ("f16", 256, 900, 0, 1, 1, 960, 1, 512, 4.4, 3.4),
     ("f16", 1600, 1500, 0, 2, 1, 768, 7, 256, 15.6, 12.1),
@@ -67,13 +67,13 @@ MEASURED = [
     ("f16", 300, 2048, 0, 2, 1, 1024, 2, 256, 6.5, 7.0),
     ("f16", 300, 2500, 0, 2, 2, 640, 3, 128, 7.1, 7.8),
     ("f16", 30, 9000, 0, 2, 5, 960, 1, 51, 4.7, 5.8),
-    ("f16", 5000, 300, 1, 1, 1, 320, 4, 1536, 16.7, 13.3),
-    ("f16", 2300, 640, 1, 1, 1, 640, 3, 768, 13.8, 14.7),
-    ("f16", 5000, 770, 1, 1, 1, 832, 10, 512, 28.7, 22.9),
-    ("f16", 400, 900, 1, 1, 1, 960, 1, 512, 6.5, 6.9),
-    ("f16", 1600, 1500, 1, 2, 1, 768, 7, 256, 18.8, 19.9),
-    ("f16", 1100, 2048, 1, 2, 1, 1024, 5, 256, 17.8, 18.9),
-    ("f16", 2300, 3000, 1, 2, 2, 768, 18, 128, 40.5, 42.7),
+    ("f16", 5000, 300, 2, 1, 1, 320, 4, 1536, 16.7, 13.3),
+    ("f16", 2300, 640, 2, 1, 1, 640, 3, 768, 13.8, 14.7),
+    ("f16", 5000, 770, 2, 1, 1, 832, 10, 512, 28.7, 22.9),
+    ("f16", 400, 900, 2, 1, 1, 960, 1, 512, 6.5, 6.9),
+    ("f16", 1600, 1500, 2, 2, 1, 768, 7, 256, 18.8, 19.9),
+    ("f16", 1100, 2048, 2, 2, 1, 1024, 5, 256, 17.8, 18.9),
+    ("f16", 2300, 3000, 2, 2, 2, 768, 18, 128, 40.5, 42.7),
     ("f16", 300, 9000, 1, 2, 5, 960, 6, 51, 18.6, 20.0),
     ("f32", 800, 640, 0, 1, 1, 640, 2, 768, 6.6, 5.2),
     ("f32", 256, 900, 0, 1, 1, 960, 1, 512, 4.9, 3.8),
@@ -84,37 +84,38 @@ MEASURED = [
     ("f32", 180, 9000, 0, 2, 5, 960, 4, 51, 17.8, 12.4),
     ("f32", 30, 9000, 0, 2, 5, 960, 1, 51, 5.5, 6.1),
     ("f32", 3300, 200, 1, 1, 1, 256, 2, 2048, 12.2, 9.6),
-    ("f32", 1100, 640, 1, 1, 1, 640, 2, 768, 10.7, 11.9),
-    ("f32", 1600, 770, 1, 1, 1, 832, 4, 512, 16.3, 13.0),
-    ("f32", 300, 770, 1, 1, 1, 832, 1, 512, 6.2, 6.5),
-    ("f32", 2300, 1200, 1, 2, 1, 640, 9, 256, 30.7, 23.9),
-    ("f32", 520, 1500, 1, 2, 1, 768, 3, 256, 11.5, 12.8),
+    ("f32", 1100, 640, 2, 1, 1, 640, 2, 768, 10.7, 11.9),
+    ("f32", 1600, 770, 2, 1, 1, 832, 4, 512, 16.3, 13.0),
+    ("f32", 300, 770, 2, 1, 1, 832, 1, 512, 6.2, 6.5),
+    ("f32", 2300, 1200, 2, 2, 1, 640, 9, 256, 30.7, 23.9),
+    ("f32", 520, 1500, 2, 2, 1, 768, 3, 256, 11.5, 12.8),
     ("f32", 800, 2048, 1, 2, 1, 1024, 4, 256, 19.2, 15.0),
-    ("f32", 400, 2048, 1, 2, 1, 1024, 2, 256, 11.8, 12.8),
-    ("f32", 1100, 3000, 1, 2, 2, 768, 9, 128, 35.5, 26.2),
-    ("f32", 800, 2060, 1, 2, 2, 576, 7, 128, 19.7, 20.9),
+    ("f32", 400, 2048, 2, 2, 1, 1024, 2, 256, 11.8, 12.8),
+    ("f32", 1100, 3000, 2, 2, 2, 768, 9, 128, 35.5, 26.2),
+    ("f32", 800, 2060, 2, 2, 2, 576, 7, 128, 19.7, 20.9),
     ("f32", 256, 9000, 1, 2, 5, 960, 6, 51, 25.7, 20.4),
-    ("f32", 100, 9000, 1, 2, 5, 960, 2, 51, 12.5, 13.6),
+    ("f32", 100, 9000, 2, 2, 5, 960, 2, 51, 12.5, 13.6),
     ("f64", 3300, 200, 0, 1, 1, 256, 4, 1024, 15.5, 12.2),
     ("f64", 800, 900, 0, 1, 1, 960, 4, 256, 16.3, 12.5),
     ("f64", 300, 2048, 0, 1, 3, 704, 4, 85, 14.1, 10.9),
     ("f64", 300, 2500, 0, 1, 3, 896, 4, 85, 16.8, 12.9),
     ("f64", 30, 9000, 0, 1, 9, 1024, 2, 28, 7.8, 8.3),
-    ("f64", 3300, 520, 1, 1, 1, 576, 13, 256, 38.1, 30.2),
-    ("f64", 800, 520, 1, 1, 1, 576, 4, 256, 12.5, 13.1),
-    ("f64", 1100, 1024, 1, 1, 1, 1024, 5, 256, 25.3, 19.3),
+    ("f64", 3300, 520, 2, 1, 1, 576, 13, 256, 38.1, 30.2),
+    ("f64", 800, 520, 2, 1, 1, 576, 4, 256, 12.5, 13.1),
+    ("f64", 1100, 1024, 2, 1, 1, 1024, 5, 256, 25.3, 19.3),
     ("f64", 300, 900, 1, 1, 1, 960, 2, 256, 9.6, 10.2),
-    ("f64", 800, 1500, 1, 1, 2, 768, 7, 128, 27.0, 20.8),
-    ("f64", 180, 2048, 1, 1, 3, 704, 3, 85, 11.3, 11.9),
-    ("f64", 520, 2500, 1, 1, 3, 896, 7, 85, 29.1, 23.0),
-    ("f64", 180, 2500, 1, 1, 3, 896, 3, 85, 12.9, 13.6),
+    ("f64", 800, 1500, 2, 1, 2, 768, 7, 128, 27.0, 20.8),
+    ("f64", 180, 2048, 2, 1, 3, 704, 3, 85, 11.3, 11.9),
+    ("f64", 520, 2500, 2, 1, 3, 896, 7, 85, 29.1, 23.0),
+    ("f64", 180, 2500, 2, 1, 3, 896, 3, 85, 12.9, 13.6),
 ]
 # the same for the rows of a pressure fix beside the sweep (11 us a launch more)
 MEASURED_SEAM = [
     ("f64", 1030, 1030, 1, 1, 2, 576, 9, 128, 24.4, 27.6), ("f64", 4000, 300, 1, 1, 1, 320, 6, 768, 27.4, 31.4),
     ("f64", 300, 4000, 1, 1, 4, 1024, 5, 64, 26.8, 23.7), ("f64", 2048, 2048, 1, 1, 3, 704, 25, 85, 107.8, 73.1),
     ("f32", 2048, 2048, 1, 2, 1, 1024, 8, 256, 47.2, 37.6), ("f16", 2048, 2048, 1, 2, 1, 1024, 8, 256, 27.2, 28.0),
-    ("f16", 5000, 900, 1, 1, 1, 960, 10, 512, 31.1, 26.5), ("f32", 16000, 260, 1, 1, 1, 320, 11, 1536, 67.2, 48.7),
+    ("f16", 5000, 900, 1, 1, 1, 960, 10, 512, 31.1, 26.5),
+    ("f64", 1615, 1094, 1, 1, 2, 576, 13, 128, 41.4, 37.4), ("f32", 16000, 260, 1, 1, 1, 320, 11, 1536, 67.2, 48.7),
 ]
 
 
@@ -127,7 +128,7 @@ def test_two_steps_only_where_they_are_faster(tmp_path):
             one, two = case[-2:]
             if two > 1.03 * one:
                 assert takes == "0", case
-            if two < 0.75 * one:
+            if two < (0.75 if extra == 0 else 0.91) * one:
                 assert takes == "1", case
 
 
@@ -157,11 +158,12 @@ int main() {
         sh.K = K;
         sh.tx = tx;
         sh.ty = ty;
-        if (K == 0) sh = lbm::pick_tile(storage, g, program != 0, pressure != 0, cus);
+        const double other = lbm::step_us(storage, g, program != 0);
+        if (K == 0) sh = lbm::pick_tile(storage, g, program != 0, pressure != 0, cus, other);
         const int n = K == 0 ? sh.K : k;
         std::printf("%d %u %u %.3f %d\n", sh.K, sh.tx, sh.ty,
                     n > 0 ? lbm::tile_us(storage, g, program != 0, pressure != 0, cus, sh, n) : 0.0,
-                    n > 0 ? (int)lbm::tile_pays(storage, g, program != 0, pressure != 0, cus, sh, n) : 0);
+                    n > 0 ? (int)lbm::tile_pays(storage, g, program != 0, pressure != 0, cus, sh, n, other) : 0);
     }
     return 0;
 }
