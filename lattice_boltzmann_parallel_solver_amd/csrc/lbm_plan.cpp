@@ -40,7 +40,8 @@ double sweep2_us(int storage, const Geom &g, bool program, bool outlet, const Sw
         if (!program) row *= 0.65;
         else if (rows == 1 && 20 * ranges <= 11 * places) row *= 0.87;  // half the blocks a CU holds
     } else if (outlet) {
-        row = waves <= 12 ? 4.2 : (sh.ntiles == 1 ? 4.65 : 5.1);
+        row = waves <= 12 ? (sh.ntiles == 1 ? 3.7 : 4.05) : (sh.ntiles == 1 ? 4.2 : 4.6);
+        head = 3.9;
     } else if (program) {
         row = (waves <= 12 ? 3.75 : 4.4) * (sh.ntiles == 1 ? 1 : 1.07);
         head = 2.4;

@@ -18,8 +18,8 @@ double step_us(int storage, const Geom &g, bool program);
 
 // Time of a two-step launch of whole rows or column tiles, us: rounds of
 // `resident` row ranges of `rows` rows each.  A block walks its rows one after
-// another, so a range costs its rows and about three more (the halo rows and the
-// first loads), 3.7 to 5.1 us each whatever the storage, by the waves and columns
+// another, so a range costs its rows and three or four more (the halo rows and the
+// first loads), 3.7 to 4.9 us each whatever the storage, by the waves and columns
 // per thread of the block, less without an outlet and half to 0.7 of it without a
 // boundary program.  Of blocks of five and of ten waves a CU holds one less than the
 // runtime says (five waves: two, not three, in FP64 and five, not six, else; ten:
