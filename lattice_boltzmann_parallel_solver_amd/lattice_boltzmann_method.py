@@ -125,13 +125,14 @@ def _step_without_torch(f, density, velocity, omega, prog):
 def _piece_bytes(total: int) -> int:
     """Bytes of the pieces that `total` bytes of host arrays go through pinned
     memory in, a multiple of 256.  Each piece costs 20 to 25 us, and the memcpy of
-    one runs beside the transfer of the others: one up to 2.8 MB (160x160: 253 us a
-    call in one, 263 in three, 279 in four), three up to 3.5 MB (180x180: 300, 287,
-    307), then four or more of up to 2 MiB (200x200: 366, 354, 341; 420x300: 1040,
-    833, 842, in eight 866)."""
-    if total <= 2_800_000:
+    one runs beside the transfer of the others: one up to 2 MiB, three up to 3 MiB
+    (calls fed with the last one's result, 170x170: 314 us in one, 274 in three, 293
+    in four; pieces above 1 MiB start to cost more, 136x249: 336 in three, 312 in
+    four), then four or more of up to 2 MiB (420x300: 1040 in one, 833 in three, 842
+    in four, 866 in eight)."""
+    if total <= 2 << 20:
         piece = total
-    elif total <= 3_500_000:
+    elif total <= 3 << 20:
         piece = -(-total // 3)
     else:
         piece = min(2 << 20, -(-total // 4))
