@@ -173,12 +173,15 @@ int lbm_set_launch(lbm_ctx *ctx, int cells_per_thread, int xcd_remap, int nt_sto
  * steps_per_launch = 3 or 4: that many steps per launch (FP32/FP16, ny <=
  * 1024, the LDS of K - 1 intermediate stages within 160 KiB: ny <= 1024 for
  * 3, about 700 for 4); a run's remainder goes two steps and one step at a
- * time.  With 2 or more and rows_per_block = 0, small lattices (2^18 nodes in
- * FP64, 3 * 2^16 else) advance up to eight steps per launch on tiles held on
- * chip.  A context that this and lbm_set_launch were never called on takes the
- * number of steps that measured fastest for it.  Results are identical in
- * every setting.  No counterpart in the reference (a launch setting of this
- * library). */
+ * time.  With 2 or more, rows_per_block = 0 and no column tiles asked for, the
+ * library goes further where it measured faster: lattices of up to 2^18 nodes in
+ * FP64 and 3 * 2^16 else advance up to eight steps per launch on tiles held on
+ * chip (in contexts that have come to 16 steps), and full rows (FP32 1537 to 2048
+ * columns, FP64 769 to 1024, twelve or more rows a compute unit) three.  A context
+ * that this and lbm_set_launch were never called on takes the number of steps that
+ * measured fastest for it.  Results are identical in every setting;
+ * lbm_next_launch tells which kernel runs.  No counterpart in the reference (a
+ * launch setting of this library). */
 int lbm_set_temporal(lbm_ctx *ctx, int steps_per_launch, int rows_per_block);
 /* The kernel that lbm_run(ctx, omega, nsteps) would launch first in the
  * context's present state and settings, and the steps that this launch
@@ -203,10 +206,10 @@ int lbm_next_launch(lbm_ctx *ctx, int64_t nsteps, int *kernel, int *steps);
  * reference (a launch setting). */
 int lbm_set_sweep_tile(lbm_ctx *ctx, int threads, int cols_per_thread);
 /* Row order of long two-step runs.  interleave = 1 (default): an lbm_run of
- * at least 64 steps with two steps per launch first copies the state into an
- * order that stores offset t of every row range of the sweep next to each
- * other (so the rows that all blocks read and write at once are neighbours in
- * memory), sweeps there, and copies it back before returning -- for FP32 rows
+ * at least 64 steps with two steps per launch keeps the state in an order that
+ * stores offset t of every row range of the sweep next to each other (so the
+ * rows that all blocks read and write at once are neighbours in memory): its
+ * first launch writes that order, its last the plain one -- for FP32 rows
  * of two columns per thread (ny > 1024) and FP64 column tiles (ny > 1024)
  * with 16 or more rows per block and at most two rounds of the row ranges
  * the GPU holds at once, where it measured faster; 0: the plain row

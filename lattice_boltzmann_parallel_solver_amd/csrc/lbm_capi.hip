@@ -158,7 +158,9 @@ bool three_steps_pay(int storage, unsigned waves) {
 }
 
 // Two-step runs of at least this many launches take the range-interleaved row
-// order (moving the state there and back costs about two launches).
+// order.  Batches move the state there and back, which costs about two launches;
+// a single lattice's sweeps enter and leave it themselves, and its line has not
+// been measured anew since.
 constexpr int64_t kInterleaveMinPairs = 32;
 constexpr int kInterleaveMinRows = 16;
 

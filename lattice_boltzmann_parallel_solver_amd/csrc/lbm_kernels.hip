@@ -874,13 +874,13 @@ struct Flag {
     static constexpr bool value = B;
 };
 
+// Instances that can run in the range-interleaved row order.
+constexpr bool sweep_interleaves(size_t elem, int v, bool tiled) { return elem >= 4 && (v == 2 || tiled); }
+
 // The threads that sweep one row range: the whole block, or in a packed block
 // one run of its waves (tid counts from the run's first thread; T threads;
 // its LDS area from smem), and the row iterations every wave of the block
 // runs (packed blocks: the longest range's rows + 2).
-// Instances that can run in the range-interleaved row order.
-constexpr bool sweep_interleaves(size_t elem, int v, bool tiled) { return elem >= 4 && (v == 2 || tiled); }
-
 struct SweepLanes {
     uint32_t tid, T;
     unsigned char *smem;
@@ -1255,7 +1255,9 @@ __device__ __forceinline__ void sweep_block(const SweepParams<S> &p, uint32_t xa
 
 // Whole rows of one column per thread in FP32 and FP16: two 1024-thread blocks a CU, which
 // takes at most 64 vector and 80 scalar registers (with 88 scalar registers,
-// one block: 1531x1023 FP16 23.6 us a launch instead of 30.9).
+// one block: 1531x1023 FP16 23.6 us a launch instead of 30.9).  The FP64 column
+// tiles take 126 of 128 vector registers, and with a probe six more are spilled:
+// 4200x1800 118 us a step without and 124 with one.
 template <class S, int V, bool kProbe, bool kTiled, bool kBig>
 __global__ __launch_bounds__(kSweepThreads, sizeof(S) < 8 && V == 1 && !kBig && !kTiled ? 8 : 4) void k_sweep2(SweepParams<S> p) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -1834,6 +1836,10 @@ __device__ __forceinline__ void buf_store(BufRsrc r, uint32_t off, double v) {
 //
 // Each wave takes one of two loops: the waves with boundary nodes in the
 // block's rows one that looks classes up, the others one without that code.
+//
+// Two stages' rows and the prefetched one fill the registers: 229 vector
+// registers in FP32 and 251 in FP64 at two waves a SIMD, none spilled, but 54 and
+// 45 scalar ones (48 and 64 bytes of scratch a lane).
 // ---------------------------------------------------------------------------
 template <class S>
 struct SweepVParams {
@@ -2513,16 +2519,13 @@ __global__ void k_add_step(int64_t *step, int64_t k) { *step += k; }
 // at 1021x773, density 118 -> 118 and 6.5 -> 7.5).
 constexpr int kRecLds = 64 * 9;  // values of one wave's records
 
-// The records of `cnt` (<= 64 - first) consecutive nodes, lane first + l's v
-// for node l, to out[0 .. 9 cnt).  `lds`: kRecLds values of this wave.  Every
-// lane calls it.
+// The records of `cnt` (<= 64) consecutive nodes, lane l's v for node l, to
+// out[0 .. 9 cnt).  `lds`: kRecLds values of this wave.  Every lane calls it.
 template <class T>
-__device__ __forceinline__ void store_records(T *out, uint32_t cnt, const T v[9], T *lds, uint32_t first = 0) {
+__device__ __forceinline__ void store_records(T *out, uint32_t cnt, const T v[9], T *lds) {
     const uint32_t lane = threadIdx.x & 63;
-    if (lane >= first) {
 #pragma unroll
-        for (int i = 0; i < 9; i++) lds[(lane - first) * 9 + i] = v[i];
-    }
+    for (int i = 0; i < 9; i++) lds[lane * 9 + i] = v[i];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
     const uint32_t n = cnt * 9;
@@ -3622,18 +3625,6 @@ int sweepk_rows(const Geom &g, int rows, int K) {
     return std::min(r, lx);
 }
 
-// Where it beats the kernels with separate columns: rows that fill seven or
-// eight waves of adjacent columns (FP32 1537 to 2048 columns, FP64 769 to 1024)
-// and twelve or more rows a block.  Time of a step, channels with walls, this
-// kernel with three steps / two steps per launch: FP32 8192x2048 93 us / 118,
-// 4200x1800 55.8 / 63.1, 2048x2048 (8 rows a block) 34.1 / 34.2, 8192x1300 84 /
-// 82, 1024x2048 24.7 / 18.7; FP64 8192x1024 99 / 124, 4096x1024 58.6 / 65.5,
-// 4096x768 54.0 / 50.7, 2000x1000 35.8 / 34.2.  An iteration's three barriers
-// and its chain of stages take 7 us whatever the row's width, which the memory
-// traffic of a full row covers (8192x2048 periodic: 81 us, 5.9 TB/s with the
-// halo rows) and a narrower one's does not; column tiles with halos lost too
-// (FP64 4200x1800 142 / 118).  With two steps it lost everywhere (FP32
-// 8192x2048 130).
 namespace {
 // One block a CU, in the fewest rounds.
 uint32_t sweepv_rows(const Geom &g) {
@@ -3646,6 +3637,18 @@ uint32_t sweepv_waves(int storage, const Geom &g) {
 }
 }  // namespace
 
+// Where it beats the kernels with separate columns: rows that fill seven or
+// eight waves of adjacent columns (FP32 1537 to 2048 columns, FP64 769 to 1024)
+// and twelve or more rows a block.  Time of a step, channels with walls, this
+// kernel with three steps / two steps per launch: FP32 8192x2048 93 us / 118,
+// 4200x1800 55.8 / 63.1, 2048x2048 (8 rows a block) 34.1 / 34.2, 8192x1300 84 /
+// 82, 1024x2048 24.7 / 18.7; FP64 8192x1024 99 / 124, 4096x1024 58.6 / 65.5,
+// 4096x768 54.0 / 50.7, 2000x1000 35.8 / 34.2.  An iteration's two barriers
+// and its chain of stages take 7 us whatever the row's width, which the memory
+// traffic of a full row covers (8192x2048 periodic: 81 us, 5.9 TB/s with the
+// halo rows) and a narrower one's does not; column tiles with halos lost too
+// (FP64 4200x1800 142 / 118).  With two steps it lost everywhere (FP32
+// 8192x2048 130).
 bool sweepv_fits(int storage, const Geom &g, uint32_t nclasses) {
     if (storage == LBM_STORE_F16 || sweep_big(storage, g) || nclasses > kSweepMaxClasses) return false;
     const uint32_t waves = sweepv_waves(storage, g);

@@ -68,7 +68,7 @@ struct LaunchCfg {
     int sweep_rows = 0;        // output rows per block of the sweep kernel (0: automatic)
     int sweep_tile = 0;        // threads per column tile of the sweep kernel (0: whole rows up to one block)
     int sweep_v = 0;           // columns per thread of column tiles (0: two for FP32/FP16, one for FP64)
-    int row_interleave = 1;    // long two-step runs move the state to the range-interleaved row order
+    int row_interleave = 1;    // long two-step runs keep the state in the range-interleaved row order
     bool shape_given = false;  // lbm_set_launch was called, with any shape: steps_per_launch 0 means 1
     // (per launch) the source / destination is in that order for sweep_rows-row ranges
     int sweep_il_src = 0, sweep_il_dst = 0;

@@ -163,12 +163,15 @@ class Lattice:
         more steps keep the intermediate states on chip (identical results,
         1/K of the population traffic per step).  Rows wider than one kernel
         block run as column tiles with two steps; three and four need FP32 or
-        FP16 rows of at most 1024 columns.  With 2 or more and automatic rows,
-        small lattices (2^18 nodes FP64, 3 * 2^16 else) take up to eight per
-        launch on tiles.  A lattice on which neither this nor `set_launch` was
-        called takes the number that measured fastest for it.  Raises LbmError
-        where the kernel does not apply (pressure fix, fewer than three rows,
-        more than 128 boundary classes, LDS)."""
+        FP16 rows of at most 1024 columns.  With 2 or more, automatic rows and
+        no column tiles asked for, lattices of up to 2^18 nodes (FP64, 3 * 2^16
+        else) take up to eight per launch on tiles, and full rows (FP32 1537 to
+        2048 columns, FP64 769 to 1024, of twelve or more rows a compute unit)
+        three, where that measured faster.  A lattice on which neither this nor
+        `set_launch` was called takes the number that measured fastest for it;
+        `next_launch` tells which kernel runs.  Raises LbmError where the kernel
+        does not apply (pressure fix, fewer than three rows, more than 128
+        boundary classes, LDS)."""
         check(_lib.load().lbm_set_temporal(self._h, int(steps_per_launch), int(rows_per_block)))
 
     def next_launch(self, steps: int) -> Tuple[str, int]:
@@ -188,11 +191,11 @@ class Lattice:
 
     def set_row_layout(self, interleave: bool = True) -> None:
         """Long two-step runs (64 steps or more) sweep the state in a row order
-        that stores the rows the blocks touch at once next to each other,
-        moving it there and back around the run (default on; used for FP32
-        rows of more than 1024 columns and FP64 column tiles with 16 or more
-        rows per block, where it measured faster).  Identical results; the
-        state is in the plain order between runs."""
+        that stores the rows the blocks touch at once next to each other: the
+        first launch writes that order, the last the plain one (default on;
+        used for FP32 rows of more than 1024 columns and FP64 column tiles
+        with 16 or more rows per block, where it measured faster).  Identical
+        results; the state is in the plain order between runs."""
         check(_lib.load().lbm_set_row_layout(self._h, 1 if interleave else 0))
 
     # -- state ------------------------------------------------------------------
