@@ -185,8 +185,9 @@ int lbm_set_launch(lbm_ctx *ctx, int cells_per_thread, int xcd_remap, int nt_sto
 int lbm_set_temporal(lbm_ctx *ctx, int steps_per_launch, int rows_per_block);
 /* The kernel that lbm_run(ctx, omega, nsteps) would launch first in the
  * context's present state and settings, and the steps that this launch
- * advances (a run is the launches for nsteps, nsteps - steps, ...).  Launches
- * nothing.  No counterpart in the reference. */
+ * advances (a run is the launches for nsteps, nsteps - steps, ..., but that it
+ * keeps to tiles, or off them, as its first launch does).  Launches nothing.
+ * No counterpart in the reference. */
 #define LBM_LAUNCH_FIRST 0       /* the collision of a loaded state */
 #define LBM_LAUNCH_STEP 1        /* one step */
 #define LBM_LAUNCH_TILE 2        /* several steps on tiles held on chip */

@@ -583,7 +583,10 @@ constexpr int64_t kTileSearchSteps = 16;
 struct Launch {
     int kernel, steps;
 };
-static Launch next_launch(lbm_ctx *c, int64_t left) {
+// run_tiles: whether the run goes through tiles, set (from kUndecided) by the first
+// launch that may.
+constexpr int kUndecided = -1;
+static Launch next_launch(lbm_ctx *c, int64_t left, int &run_tiles) {
     if (c->phase == kPending) return {LBM_LAUNCH_FIRST, 1};
     if (left < 2) return {LBM_LAUNCH_STEP, 1};
     const RunPlan &p = run_plan(c);
@@ -591,7 +594,9 @@ static Launch next_launch(lbm_ctx *c, int64_t left) {
         c->plan.tile = tile_shape(c->storage, c->g, c->bc.view, p.other_us);
         c->plan.tile_ready = true;
     }
-    if (p.tile.K > 0) {
+    if (p.tile.K > 0 && run_tiles == kUndecided)
+        run_tiles = tile_steps_run(c->storage, c->g, c->bc.view, p.tile, left, p.other_us);
+    if (p.tile.K > 0 && run_tiles) {
         const int k = (int)std::min<int64_t>(p.tile.K, left);
         if (k == p.tile.K || tile_steps_pay(c->storage, c->g, c->bc.view, p.tile, k, p.other_us)) return {LBM_LAUNCH_TILE, k};
     }
@@ -649,7 +654,8 @@ int lbm_next_launch(lbm_ctx *c, int64_t nsteps, int *kernel, int *steps) {
         set_error("lbm_next_launch: no state loaded (call lbm_set_state first)");
         return LBM_ERR_STATE;
     }
-    const Launch l = next_launch(c, nsteps);
+    int run_tiles = kUndecided;
+    const Launch l = next_launch(c, nsteps, run_tiles);
     *kernel = l.kernel;
     *steps = l.steps;
     return LBM_OK;
@@ -676,8 +682,9 @@ int lbm_run(lbm_ctx *c, double omega, int64_t nsteps) {
     const BcView &bc = c->bc.view;
     LaunchCfg cfg2 = c->cfg;  // of the two-step sweeps
     bool cfg2_set = false, interleave = false;
+    int run_tiles = kUndecided;
     while (left > 0) {
-        const Launch l = next_launch(c, left);
+        const Launch l = next_launch(c, left, run_tiles);
         // a launch of s steps materialises f_{steps} .. f_{steps+s-1} on chip:
         // it records them if probed
         const int64_t slot = probing ? c->steps - c->probe_base - 1 : -1;

@@ -3715,6 +3715,11 @@ bool tile_steps_pay(int storage, const Geom &g, const BcView &bc, const TileShap
     return tile_pays(storage, g, bc.codes != nullptr, (bc.flags & kProgPressure) != 0, compute_units(), sh, k, other_us);
 }
 
+bool tile_steps_run(int storage, const Geom &g, const BcView &bc, const TileShape &sh, int64_t steps, double other_us) {
+    return tile_run_pays(storage, g, bc.codes != nullptr, (bc.flags & kProgPressure) != 0, compute_units(), sh, steps,
+                         other_us);
+}
+
 namespace {
 template <class S>
 hipError_t tile_typed(const TileShape &sh, const Geom &g, const StateView &st, int src, const BcView &bc, double omega,

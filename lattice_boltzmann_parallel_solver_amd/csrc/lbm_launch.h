@@ -72,6 +72,8 @@ hipError_t launch_sweepv(int storage, const SweepVShape &sh, const Geom &g, cons
 // tile_steps_pay says so.
 TileShape tile_shape(int storage, const Geom &g, const BcView &bc, double other_us);
 bool tile_steps_pay(int storage, const Geom &g, const BcView &bc, const TileShape &sh, int k, double other_us);
+// Whether a run of so many steps takes tiles at all.
+bool tile_steps_run(int storage, const Geom &g, const BcView &bc, const TileShape &sh, int64_t steps, double other_us);
 hipError_t launch_tile(int storage, const TileShape &sh, const Geom &g, const StateView &st, int src, const BcView &bc,
                        double omega, const ProbeView &pr, int64_t probe_slot, hipStream_t s);
 // K steps of the rows that the pressure fix reaches in them, lx - K to K - 1

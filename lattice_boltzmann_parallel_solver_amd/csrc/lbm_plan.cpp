@@ -147,4 +147,18 @@ bool tile_pays(int storage, const Geom &g, bool program, bool pressure, int cus,
     return tile_us(storage, g, program, pressure, cus, sh, k) < tile_margin(pressure) * k * other_us;
 }
 
+bool tile_run_pays(int storage, const Geom &g, bool program, bool pressure, int cus, const TileShape &sh, int64_t steps,
+                   double other_us) {
+    if (steps < sh.K) return tile_pays(storage, g, program, pressure, cus, sh, (int)steps, other_us);
+    const int64_t n = steps / sh.K;
+    const int r = (int)(steps % sh.K);
+    if (r == 0 || n > 16) return true;
+    double t = (double)n * tile_us(storage, g, program, pressure, cus, sh, sh.K);
+    if (r > 1 && tile_pays(storage, g, program, pressure, cus, sh, r, other_us))
+        t += tile_us(storage, g, program, pressure, cus, sh, r);
+    else
+        t += r * other_us + 9e-6 * g.N * elem_of(storage) * (program ? 0.25 : 0.65);
+    return t < 0.96 * (double)steps * other_us;
+}
+
 }  // namespace lbm

@@ -64,4 +64,12 @@ TileShape pick_tile(int storage, const Geom &g, bool program, bool pressure, int
 bool tile_pays(int storage, const Geom &g, bool program, bool pressure, int cus, const TileShape &sh, int k,
                double other_us);
 
+// Whether a run of `steps` steps goes through tiles: its last steps, too few for a
+// launch of their own, run on the other kernel, which finds the state in other L2
+// caches than it would write it to (0.25 us a MB of state, 0.65 without a boundary
+// program).  FP64 62x2261, periodic, two steps a launch, us a step in runs of 2, 3, 5
+// and 7: 4.2, 7.0, 5.8 and 5.3, single steps 5.4.
+bool tile_run_pays(int storage, const Geom &g, bool program, bool pressure, int cus, const TileShape &sh, int64_t steps,
+                   double other_us);
+
 }  // namespace lbm

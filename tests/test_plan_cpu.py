@@ -146,7 +146,7 @@ TILE_DRIVER = r"""
 int main() {
     int storage, program, pressure, cus, K, k;
     unsigned lx, ly, pitch, tx, ty;
-    // K = 0: pick a tiling; else the time of k steps of the given one
+    // K = 0: pick a tiling; else the time of k steps of the given one, or (k < 0) whether a run of -k steps takes it
     while (std::scanf("%d %u %u %u %d %d %d %d %u %u %d", &storage, &lx, &ly, &pitch, &program, &pressure, &cus, &K, &tx, &ty,
                       &k) == 11) {
         lbm::Geom g;
@@ -160,6 +160,10 @@ int main() {
         sh.ty = ty;
         const double other = lbm::step_us(storage, g, program != 0);
         if (K == 0) sh = lbm::pick_tile(storage, g, program != 0, pressure != 0, cus, other);
+        if (k < 0) {
+            std::printf("%d\n", (int)lbm::tile_run_pays(storage, g, program != 0, pressure != 0, cus, sh, -k, other));
+            continue;
+        }
         const int n = K == 0 ? sh.K : k;
         std::printf("%d %u %u %.3f %d\n", sh.K, sh.tx, sh.ty,
                     n > 0 ? lbm::tile_us(storage, g, program != 0, pressure != 0, cus, sh, n) : 0.0,
@@ -196,6 +200,18 @@ def test_tile_times_and_where_they_pay(tmp_path):
                 assert pays == "0", (case, k)
             if us < 0.75 * k * one:
                 assert pays == "1", (case, k)
+
+
+def test_short_runs_that_tiles_do_not_divide(tmp_path):
+    """us a step in runs of so many steps over single steps: FP64 62x2261 periodic 2 0.77, 3 1.28, 5 1.06, 40 0.77;
+    95x1728 2 0.84, 3 1.03, 5 0.95; 60x2300 3 0.66, 4 0.89; FP32 59x2388 with the pressure fix 3 1.02"""
+    run = _driver(tmp_path, TILE_DRIVER)
+    for st, lx, ly, kind, tile, takes in (("f64", 62, 2261, 0, (2, 62, 9), {2: 1, 3: 0, 5: 0, 6: 1, 33: 1, 40: 1}),
+                                          ("f64", 95, 1728, 1, (2, 24, 27), {2: 1, 3: 0, 5: 1, 41: 1}),
+                                          ("f64", 60, 2300, 1, (3, 30, 18), {3: 1, 4: 1, 5: 1, 7: 1}),
+                                          ("f32", 59, 2388, 2, (2, 30, 19), {3: 0, 4: 1})):
+        got = run([_tile_row(st, lx, ly, kind, *tile, -n) for n in takes])
+        assert [int(v) for v in got] == list(takes.values()), (lx, ly)
 
 
 def test_tilings_fit_their_blocks_and_beat_single_steps(tmp_path):
